@@ -213,6 +213,7 @@ SIGNATURES = {
     "apy_synth_so_ints": (c_int, [ctypes.c_uint64, ctypes.c_uint64, c_dbl, c_int, c_dbl, c_int,
                                   ctypes.POINTER(SoInts), c_vp]),
     "apy_so_fock_from_mo": (c_int, [c_i64, c_vp, c_vp, c_vp]),
+    "apy_so_fock_from_mo_batch": (c_int, [c_i64, c_i64, c_vp, c_vp, c_vp]),
     "apy_cisd_so_pair_operator": (c_int, [c_i64, c_i64, c_vp, c_vp, c_vp, c_vp]),
     "apy_cisd_so_ring_fock": (c_int, [c_i64, c_i64, c_vp, c_vp, c_vp, c_vp]),
     "apy_cisd_so_workspace": (c_size, [c_i64, c_i64, c_int]),

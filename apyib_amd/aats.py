@@ -154,7 +154,7 @@ class AAT(object):
         Ck = np.stack([np.asarray(c, dtype=np.complex128) for _, _, _, _, (_, c) in pairs])
         S_mo = tr.mo_overlap(tr.to_dev(Cb, dev), tr.to_dev(S_ao, dev), tr.to_dev(Ck, dev))
         if self.so:
-            S_mo = torch.stack([tr.so_fock(S_mo[q]) for q in range(nov)])
+            S_mo = tr.so_fock(S_mo)
             n, no, nf = 2 * nbf, 2 * self.ndocc, 0
         else:
             n, no, nf = nbf, self.ndocc, self.nfzc

@@ -193,11 +193,11 @@ int build_all(const Src& src, const apy_so_ints* I, int accumulate, double scale
   return APY_OK;
 }
 
-__global__ void so_fock_kernel(int64_t m, const double2* fmo, double2* fso) {
-  const int64_t n = 2 * m;
-  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < n * n; t += (int64_t)gridDim.x * blockDim.x) {
-    int64_t p = t / n, q = t % n;
-    fso[t] = ((p ^ q) & 1) ? make_double2(0.0, 0.0) : fmo[(p >> 1) * m + (q >> 1)];
+__global__ void so_fock_kernel(int64_t m, int64_t nb, const double2* fmo, double2* fso) {
+  const int64_t n = 2 * m, total = nb * n * n;
+  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total; t += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t r = t / n, p = r % n, q = t % n;
+    fso[t] = ((p ^ q) & 1) ? make_double2(0.0, 0.0) : fmo[((r / n) * m + (p >> 1)) * m + (q >> 1)];
   }
 }
 
@@ -857,8 +857,13 @@ int apy_synth_so_ints(uint64_t seed, uint64_t tag, double sd, int accumulate, do
 }
 
 int apy_so_fock_from_mo(int64_t m, const void* f_mo, void* f_so, void* stream) {
-  if (m <= 0 || !f_mo || !f_so) return APY_E_ARG;
-  so_fock_kernel<<<apy_grid1d(4 * m * m), 256, 0, (hipStream_t)stream>>>(m, (const double2*)f_mo, (double2*)f_so);
+  return apy_so_fock_from_mo_batch(m, 1, f_mo, f_so, stream);
+}
+
+int apy_so_fock_from_mo_batch(int64_t m, int64_t nb, const void* f_mo, void* f_so, void* stream) {
+  if (m <= 0 || nb <= 0 || !f_mo || !f_so) return APY_E_ARG;
+  so_fock_kernel<<<apy_grid1d(4 * m * m * nb), 256, 0, (hipStream_t)stream>>>(m, nb, (const double2*)f_mo,
+                                                                               (double2*)f_so);
   APY_LAUNCH_CHECK();
   return APY_OK;
 }

@@ -194,16 +194,23 @@ def mixed_overlaps(pairs, device):
     function at its own centre (utils.py:371-376 for every pair): pairs with
     the same function shapes share one apy_oei_gto launch.  Returns a list of
     float64 device tensors [na, nb] in the order of `pairs`."""
+    # a finite-difference set pairs a few dozen function lists in hundreds of ways: each list (alive in `pairs`
+    # throughout) is read once
+    seen = {}
+    for pair in pairs:
+        for fns in pair:
+            if id(fns) not in seen:
+                seen[id(fns)] = (_signature(fns), np.array([f.center for f in fns], dtype=np.float64))
     groups = {}
     for q, (bra, ket) in enumerate(pairs):
-        groups.setdefault((_signature(bra), _signature(ket)), []).append(q)
+        groups.setdefault((seen[id(bra)][0], seen[id(ket)][0]), []).append(q)
     out = [None] * len(pairs)
     for qs in groups.values():
         bra0, ket0 = pairs[qs[0]]
         fa, _ = function_table(bra0, device)
         fb, _ = function_table(ket0, device)
-        ca = np.stack([[np.asarray(f.center, dtype=np.float64) for f in pairs[q][0]] for q in qs])
-        cb = np.stack([[np.asarray(f.center, dtype=np.float64) for f in pairs[q][1]] for q in qs])
+        ca = np.stack([seen[id(pairs[q][0])][1] for q in qs])
+        cb = np.stack([seen[id(pairs[q][1])][1] for q in qs])
         S = one_electron(fa, ca, fb, cb, _lib.APY_OEI_OVERLAP, device)
         for k, q in enumerate(qs):
             out[q] = S[k, 0]

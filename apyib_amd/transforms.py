@@ -113,12 +113,14 @@ def eri_so(eri_mo_t):
 
 
 def so_fock(f_mo):
-    """utils.py:283-313."""
+    """utils.py:283-313 for one matrix [m, m] or a batch [nb, m, m]."""
     lib = _lib.load()
-    m = f_mo.shape[0]
-    out = torch.empty((2 * m, 2 * m), dtype=CDT, device=f_mo.device)
-    _lib.check(lib.apy_so_fock_from_mo(m, _vp(f_mo.contiguous()), _vp(out), stream_of(f_mo.device)),
-               "apy_so_fock_from_mo")
+    m = f_mo.shape[-1]
+    f_mo = f_mo.contiguous()
+    out = torch.empty((*f_mo.shape[:-2], 2 * m, 2 * m), dtype=CDT, device=f_mo.device)
+    nb = f_mo.shape[0] if f_mo.dim() == 3 else 1
+    _lib.check(lib.apy_so_fock_from_mo_batch(m, nb, _vp(f_mo), _vp(out), stream_of(f_mo.device)),
+               "apy_so_fock_from_mo_batch")
     return out
 
 

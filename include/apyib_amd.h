@@ -148,6 +148,8 @@ int apy_synth_so_ints(uint64_t seed, uint64_t tag, double std, int accumulate, d
 /* Spin-orbital Fock matrix F_SO[p,q] = F_MO[p/2,q/2] delta(spin p, spin q)
  * (compute_F_SO, utils.py:283-313): f_mo is [m][m], f_so [2m][2m]. */
 int apy_so_fock_from_mo(int64_t m, const void* f_mo, void* f_so, void* stream);
+/* The same for nb matrices stored one after another. */
+int apy_so_fock_from_mo_batch(int64_t m, int64_t nb, const void* f_mo, void* f_so, void* stream);
 
 /* ------------------------------------------------------------------------
  * Spin-adapted closed-shell CISD / CID (ci_wfn.py:420-574 and :51-167) on
