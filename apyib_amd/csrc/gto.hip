@@ -2,13 +2,14 @@
 // the AO integrals psi4's MintsHelper gives the reference (hamiltonian.py:33 ao_eri, analytic_aats.py:94
 // mo_tei_deriv1 before its MO transform).  A function is one or two terms sharing a centre and the
 // exponents, sum_term sum_p c_term,p x^l y^m z^n exp(-a_p r^2): an s/p basis function is one term, its
-// derivative with respect to its centre two (l+1 and l-1).  One thread per output element; every
+// derivative with respect to its centre two (l+1 and l-1).  One workgroup per quartet of shells; every
 // primitive quartet is expanded in Hermite Gaussians (E coefficients), the Coulomb integrals R_tuv come
 // from the Boys function by the Hermite recursion, and the quartet sum is
 //   (ab|cd) = 2 pi^(5/2) / (p q sqrt(p+q)) sum_tuv E^ab_tuv sum_t'u'v' (-1)^(t'+u'+v') E^cd_t'u'v'
 //             R_(t+t')(u+u')(v+v')(alpha, P - Q).
 #include "common.h"
 
+#include <algorithm>
 #include <mutex>
 
 namespace {
@@ -159,62 +160,6 @@ __device__ int herm_R(int L, const int* Lt, double alpha, const double* PQ, cons
   return cur;
 }
 
-// One primitive quartet of (a b | c d): terms (ta, tb, tc, td), primitives (pa, pb, pc, pd), centres ca..cd,
-// qab = A - B, qcd = C - D.  The caller has checked the table entries and that the quartet's total angular
-// momentum is at most LQ.
-__device__ double eri_prim(const apy_gto& A, const apy_gto& B, const apy_gto& C, const apy_gto& D, int ta, int tb,
-                           int tc, int td, int pa, int pb, int pc, int pd, const double* ca, const double* cb,
-                           const double* cc, const double* cd, const double* qab, const double* qcd) {
-  const int* la = A.lmn[ta];
-  const int* lb = B.lmn[tb];
-  const int* lc = C.lmn[tc];
-  const int* ld = D.lmn[td];
-  int L1[3], L2[3], Lt[3];
-  for (int x = 0; x < 3; ++x) { L1[x] = la[x] + lb[x]; L2[x] = lc[x] + ld[x]; Lt[x] = L1[x] + L2[x]; }
-  const int L = Lt[0] + Lt[1] + Lt[2];
-  const int sz = Lt[2] + 1, sy = (Lt[1] + 1) * sz;  // R index (t, u, v) -> t sy + u sz + v
-  const double a = A.exps[pa], b = B.exps[pb], p = a + b;
-  const double c = C.exps[pc], d = D.exps[pd], q = c + d;
-  double Eab[3][NE], Ecd[3][NE], PQ[3];
-  for (int x = 0; x < 3; ++x) {
-    herm_E(la[x], lb[x], qab[x], a, b, Eab[x]);
-    herm_E(lc[x], ld[x], qcd[x], c, d, Ecd[x]);
-    PQ[x] = (a * ca[x] + b * cb[x]) / p - (c * cc[x] + d * cd[x]) / q;
-  }
-  const double alpha = p * q / (p + q);
-  double F[LQ + 1];
-  boys_fn(L, alpha * (PQ[0] * PQ[0] + PQ[1] * PQ[1] + PQ[2] * PQ[2]), F);
-  double Rb[2][NRB];
-  const double* R = Rb[herm_R(L, Lt, alpha, PQ, F, Rb)];
-  double val = 0.0;
-  for (int t = 0; t <= L1[0]; ++t)
-    for (int u = 0; u <= L1[1]; ++u)
-      for (int v = 0; v <= L1[2]; ++v) {
-        const double e1 = Eab[0][t] * Eab[1][u] * Eab[2][v];
-        double s2 = 0.0;
-        for (int tt = 0; tt <= L2[0]; ++tt)
-          for (int uu = 0; uu <= L2[1]; ++uu)
-            for (int vv = 0; vv <= L2[2]; ++vv) {
-              const double e2 = Ecd[0][tt] * Ecd[1][uu] * Ecd[2][vv];
-              const double sg = ((tt + uu + vv) & 1) ? -1.0 : 1.0;
-              s2 += sg * e2 * R[(t + tt) * sy + (u + uu) * sz + (v + vv)];
-            }
-        val += e1 * s2;
-      }
-  const double pref0 = 2.0 * M_PI * M_PI * sqrt(M_PI);
-  return A.coefs[ta][pa] * B.coefs[tb][pb] * C.coefs[tc][pc] * D.coefs[td][pd] * pref0 / (p * q * sqrt(p + q)) * val;
-}
-
-// Whether every term combination of the quartet stays within the total angular momentum LQ.
-__device__ bool quartet_ok(const apy_gto& A, const apy_gto& B, const apy_gto& C, const apy_gto& D) {
-  for (int ta = 0; ta < A.nterm; ++ta)
-    for (int tb = 0; tb < B.nterm; ++tb)
-      for (int tc = 0; tc < C.nterm; ++tc)
-        for (int td = 0; td < D.nterm; ++td)
-          if (lsum(A.lmn[ta]) + lsum(B.lmn[tb]) + lsum(C.lmn[tc]) + lsum(D.lmn[td]) > LQ) return false;
-  return true;
-}
-
 // x = hi (hi + 1) / 2 + lo with 0 <= lo <= hi: the row-packed lower triangle.
 __device__ inline void tri_split(int64_t x, int64_t& hi, int64_t& lo) {
   int64_t h = (int64_t)((sqrt(8.0 * (double)x + 1.0) - 1.0) * 0.5);
@@ -229,87 +174,422 @@ __device__ inline void tri_split(int64_t x, int64_t& hi, int64_t& lo) {
 // ket tables are one table ((ab|cd) = (ab|dc): 2 images, k >= l), ERI_NONE otherwise.
 enum EriSym { ERI_NONE = 0, ERI_KET = 1, ERI_ALL = 2 };
 
-// One wavefront per computed element (wave-uniform control flow): the lanes split the element's
-// (term, primitive) quartets and a fixed-order butterfly sums them; lane 0 writes the value to every
-// image of the element under the launch's symmetry.  A table entry outside the limits (angular
-// momentum, primitive count, term count, atom index) gives NaN before any indexing.
-__global__ __launch_bounds__(256) void eri_kernel(int64_t ngeom, int64_t natom, const double* __restrict__ centers,
-                                                  const apy_gto* __restrict__ fa, int64_t na,
-                                                  const apy_gto* __restrict__ fb, int64_t nb,
-                                                  const apy_gto* __restrict__ fc, int64_t nc,
-                                                  const apy_gto* __restrict__ fd, int64_t nd, int sym,
-                                                  double2* __restrict__ out) {
-  const int lane = threadIdx.x & 63;
-  const int64_t full = na * nb * nc * nd;
-  const int64_t pc = nc * (nc + 1) / 2;
-  const int64_t per = sym == ERI_ALL ? pc * (pc + 1) / 2 : sym == ERI_KET ? na * nb * pc : full;
-  const int64_t total = ngeom * per;
-  const int64_t nwave = (int64_t)gridDim.x * (blockDim.x >> 6);
-  for (int64_t e = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6; e < total; e += nwave) {
-    const int64_t g = e / per, r = e % per;
-    int64_t i, j, k, l;
+// Functions that sit next to each other in a table on one centre with the same exponents (an sp or a d
+// shell) form a group of up to EG.  A group quartet shares every primitive quartet's Boys functions and
+// Hermite Coulomb integrals, which is why the work is split by group quartets and not by elements: at
+// H2O2/6-31G* (34 functions, 2.1e6 primitive quartets of functions) there are 1.0e5 of groups.
+//
+// One workgroup computes the (up to EG^4) elements of a group quartet.  Primitive pairs are taken in
+// batches that fit LDS; per batch
+//   1. Hermite E coefficients of the bra and ket primitive pairs (a thread per pair, axis and bra power),
+//      G_n = pref (-2 alpha)^n F_n and the powers of P - Q (a thread per primitive quartet and order),
+//   2. R_tuv = sum_ijk a_ti a_uj a_vk X^(t-2i) Y^(u-2j) Z^(v-2k) G_(t+u+v-i-j-k), a_ti = t!/(i!(t-2i)!2^i)
+//      (the Hermite recursion in closed form: every entry on its own, no order of evaluation between them),
+//   3. H[bra pair][ket element][tuv] += sum over the ket pairs of E^cd R, signs (-1)^t in E^cd,
+// and per bra batch acc[element] += E^ab H.  Contracting the ket pairs first makes the step
+// that touches every element run once a bra pair instead of once a primitive quartet.
+// Bound by the latency of these short phases, not by bytes or flops: 118 registers and 40 KB of LDS keep
+// four workgroups on a CU.  H2O2/6-31G*: 5040 us with a wave an element and every expansion redone for
+// each quartet of functions, 210 us so.
+constexpr int EG = 6;                 // functions of a group
+constexpr int EPP = APY_GTO_MAXPRIM * APY_GTO_MAXPRIM;
+constexpr int EW = 1024;              // doubles: G, powers and R of a batch
+constexpr int EH = 36 * 36;           // doubles: H (a d,d pair's 35 tuv with its 36 ket elements: 1260)
+constexpr int EE = 448;               // doubles: E coefficients of a batch, bra or ket (f,f: 336 a pair)
+constexpr int ENR = (LQ + 1) * (LQ + 2) * (LQ + 3) / 6;   // tuv with t + u + v <= LQ
+constexpr int ETAB = 4096;            // group starts that LDS holds, all tables together
+
+// index of (t, u, v) in order of t + u + v: the entries up to a total L come first
+__host__ __device__ inline int tuv_index(int t, int u, int v) {
+  const int r = u + v, s = t + r;
+  return s * (s + 1) * (s + 2) / 6 + r * (r + 1) / 2 + v;
+}
+__host__ __device__ inline int tuv_count(int L) { return (L + 1) * (L + 2) * (L + 3) / 6; }
+
+// w / d and w % d for 0 <= w < 2^16 and one d of a workgroup: a multiplication instead of the ~40
+// instructions of an integer division (several a work item, as long as the item's own sums)
+struct SmallDiv {
+  unsigned inv;
+  int d;
+  __device__ explicit SmallDiv(int n) : inv(n > 1 ? 0xffffffffu / (unsigned)n + 1u : 0u), d(n) {}
+  __device__ int div(int w) const { return d > 1 ? (int)__umulhi((unsigned)w, inv) : w; }
+  __device__ int mod(int w) const { return w - div(w) * d; }
+};
+
+// an LDS value that every thread reads alike, in a scalar register
+__device__ inline int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+
+struct EriTab {
+  const apy_gto* f[4];
+  int64_t n[4];
+};
+
+struct EriShared {
+  double W[EW], H[EH], acc[EG * EG * EG * EG], Eb[EE], Ek[EE];
+  double exps[4][APY_GTO_MAXPRIM], cen[4][3], coef[4][EG][2][APY_GTO_MAXPRIM];
+  double herm[LQ + 1][LQ / 2 + 1];    // a_ti
+  int8_t lmn[4][EG][2][3];
+  uint8_t nterm[4][EG];
+  uint8_t tuv[ENR][3];
+  uint8_t prim[2][EPP][2];            // primitives of pair b (bra) or q (ket)
+  int size[4], nprim[4], L[4], first[4], bad, ngrp[4];
+};
+
+// Starts of the groups of a table into `start` (start[ngrp] = n); by one thread.
+__device__ int find_groups(int64_t n, const uint8_t* joins, uint16_t* start) {
+  int g = 0, len = 0;
+  for (int i = 0; i < (int)n; ++i) {
+    if (i == 0 || !joins[i] || len == EG) { start[g++] = (uint16_t)i; len = 0; }
+    ++len;
+  }
+  start[g] = (uint16_t)n;
+  return g;
+}
+
+// E^{ij}_t of one primitive pair and axis for this i and all j <= Lb, into out[(i (Lb+1) + j) nt + t],
+// nt = La + Lb + 1, times sgn^t; the recursion of herm_E along one row, in registers.
+__device__ void herm_row(int i, int La, int Lb, double Q, double a, double b, double sgn, double* out) {
+  const double p = a + b, h = 0.5 / p, xpa = -b * Q / p, xpb = a * Q / p;
+  double e[NE + 1];
+#pragma unroll
+  for (int t = 0; t <= NE; ++t) e[t] = 0.0;
+  e[0] = exp(-a * b / p * Q * Q);
+  auto raise = [&](double x) {
+    double lo = 0.0;                                   // E_(t-1) of the row below
+#pragma unroll
+    for (int t = 0; t < NE; ++t) {
+      const double c = e[t];
+      e[t] = x * c + h * lo + (t + 1) * e[t + 1];
+      lo = c;
+    }
+  };
+  for (int k = 0; k < i; ++k) raise(xpa);
+  const int nt = La + Lb + 1;
+  double* o = out + (int64_t)i * (Lb + 1) * nt;
+  for (int j = 0; j <= Lb; ++j) {
+    if (j) raise(xpb);
+    double s = 1.0;
+#pragma unroll
+    for (int t = 0; t < NE; ++t) {
+      if (t < nt) o[j * nt + t] = s * e[t];
+      s *= sgn;
+    }
+  }
+}
+
+// F_n(T) for one order (boys_fn's two ranges; erf(sqrt T) = 1 in doubles from T = 36 on).
+__device__ double boys_one(int n, double T) {
+  if (T < BOYS_TMAX) {
+    const double x = T * BOYS_DENS;
+    const int k = (int)(x + 0.5);
+    const double d = ((double)k - x) / BOYS_DENS;
+    const double* g = g_boys[k] + n;
+    double f = g[6];
+    f = g[5] + d * f * (1.0 / 6.0);
+    f = g[4] + d * f * (1.0 / 5.0);
+    f = g[3] + d * f * (1.0 / 4.0);
+    f = g[2] + d * f * (1.0 / 3.0);
+    f = g[1] + d * f * (1.0 / 2.0);
+    return g[0] + d * f;
+  }
+  const double e = exp(-T), r = 0.5 / T;
+  double F = 0.5 * sqrt(M_PI / T);
+  for (int m = 0; m < n; ++m) F = ((2 * m + 1) * F - e) * r;
+  return F;
+}
+
+__global__ __launch_bounds__(256, 4) void eri_kernel(int64_t ngeom, int64_t natom, const double* __restrict__ centers,
+                                                  EriTab T, int sym, int grouped, double2* __restrict__ out) {
+  __shared__ EriShared S;
+  extern __shared__ uint16_t starts[];               // group starts, then the join flags (grouped only)
+  const int tid = threadIdx.x;
+  const int64_t n0 = T.n[0], n1 = T.n[1], n2 = T.n[2], n3 = T.n[3], full = n0 * n1 * n2 * n3;
+
+  // ---- once a workgroup: the tables' groups (ERI_ALL: one table, ERI_KET: the ket's twice), index tables
+  const int ntab = sym == ERI_ALL ? 1 : sym == ERI_KET ? 3 : 4;
+  int64_t tot = 0, off[5];
+  for (int x = 0; x < 4; ++x) { off[x] = tot; if (x < ntab) tot += T.n[x] + 1; }
+  if (grouped) {
+    uint8_t* joins = (uint8_t*)(starts + tot);
+    for (int x = 0; x < ntab; ++x)
+      for (int64_t i = tid; i < T.n[x]; i += 256) {
+        const apy_gto& f = T.f[x][i];
+        bool same = false;
+        if (i > 0 && gto_ok(f, natom)) {
+          const apy_gto& e = T.f[x][i - 1];
+          same = gto_ok(e, natom) && e.atom == f.atom && e.nprim == f.nprim;
+          for (int k = 0; same && k < f.nprim; ++k) same = e.exps[k] == f.exps[k];
+        }
+        joins[off[x] + i] = same;
+      }
+    __syncthreads();
+    if (tid < ntab) S.ngrp[tid] = find_groups(T.n[tid], joins + off[tid], starts + off[tid]);
+  } else if (tid < 4) {
+    S.ngrp[tid] = (int)T.n[tid];
+  }
+  for (int r = tid; r < ENR; r += 256) {
+    int s = 0, w = 0;
+    while (tuv_count(s) <= r) ++s;
+    const int q = r - (s > 0 ? tuv_count(s - 1) : 0);
+    while ((w + 1) * (w + 2) / 2 <= q) ++w;
+    const int v = q - w * (w + 1) / 2;
+    S.tuv[r][0] = (uint8_t)(s - w); S.tuv[r][1] = (uint8_t)(w - v); S.tuv[r][2] = (uint8_t)v;
+  }
+  if (tid <= LQ) {
+    double a = 1.0;
+    for (int i = 0; 2 * i <= tid; ++i) {
+      S.herm[tid][i] = a;
+      a *= (double)((tid - 2 * i) * (tid - 2 * i - 1)) / (2.0 * (i + 1));
+    }
+  }
+  __syncthreads();
+  // slot x's groups are those of table tx[x]
+  const int tx[4] = {0, sym == ERI_ALL ? 0 : 1, sym == ERI_ALL ? 0 : 2, sym == ERI_ALL ? 0 : sym == ERI_KET ? 2 : 3};
+  int64_t ng[4];
+  for (int x = 0; x < 4; ++x) ng[x] = uniform(S.ngrp[tx[x]]);
+  const int64_t pk = sym == ERI_NONE ? ng[2] * ng[3] : ng[2] * (ng[2] + 1) / 2;
+  const int64_t per = sym == ERI_ALL ? pk * (pk + 1) / 2 : ng[0] * ng[1] * pk;
+
+  for (int64_t item = blockIdx.x; item < ngeom * per; item += gridDim.x) {
+    const int64_t g = item / per, r0 = item % per;
+    int64_t G[4];
     if (sym == ERI_ALL) {
       int64_t bra, ket;
-      tri_split(r, bra, ket);
-      tri_split(bra, i, j);
-      tri_split(ket, k, l);
-    } else if (sym == ERI_KET) {
-      tri_split(r % pc, k, l);
-      j = (r / pc) % nb;
-      i = r / (pc * nb);
+      tri_split(r0, bra, ket);
+      tri_split(bra, G[0], G[1]);
+      tri_split(ket, G[2], G[3]);
     } else {
-      l = r % nd; k = (r / nd) % nc; j = (r / (nd * nc)) % nb; i = r / (nd * nc * nb);
+      if (sym == ERI_KET) {
+        tri_split(r0 % pk, G[2], G[3]);
+      } else {
+        G[2] = (r0 % pk) / ng[3]; G[3] = r0 % ng[3];
+      }
+      G[1] = (r0 / pk) % ng[1];
+      G[0] = r0 / (pk * ng[1]);
     }
-    double2* o = out + g * full;
-    // element (p, q, s, t) of the [na][nb][nc][nd] output
-    auto at = [&](int64_t p, int64_t q, int64_t s2, int64_t t) { return ((p * nb + q) * nc + s2) * nd + t; };
-    auto put = [&](double v) {
-      const double2 w = make_double2(v, 0.0);
-      o[at(i, j, k, l)] = w;
-      if (sym == ERI_NONE) return;
-      o[at(i, j, l, k)] = w;
-      if (sym == ERI_KET) return;
-      o[at(j, i, k, l)] = w;
-      o[at(j, i, l, k)] = w;
-      o[at(k, l, i, j)] = w;
-      o[at(l, k, i, j)] = w;
-      o[at(k, l, j, i)] = w;
-      o[at(l, k, j, i)] = w;
-    };
-    const apy_gto& A = fa[i];
-    const apy_gto& B = fb[j];
-    const apy_gto& C = fc[k];
-    const apy_gto& D = fd[l];
-    if (!gto_ok(A, natom) || !gto_ok(B, natom) || !gto_ok(C, natom) || !gto_ok(D, natom) ||
-        !quartet_ok(A, B, C, D)) {
-      if (lane == 0) put(kNaN);
-      continue;
+    // ---- the four groups into LDS
+    __syncthreads();                                  // the previous item's elements are done with LDS
+    if (tid < 4) {
+      const int x = tid;
+      const int64_t b = grouped ? starts[off[tx[x]] + G[x]] : G[x];
+      const int64_t e = grouped ? starts[off[tx[x]] + G[x] + 1] : b + 1;
+      const apy_gto& f = T.f[x][b];
+      const bool ok = gto_ok(f, natom);
+      S.first[x] = (int)b;
+      S.size[x] = (int)(e - b);
+      S.nprim[x] = ok ? f.nprim : 0;
+      int L = 0;
+      for (int64_t m = b; m < e && ok; ++m)
+        for (int t = 0; t < T.f[x][m].nterm; ++t) L = max(L, lsum(T.f[x][m].lmn[t]));
+      S.L[x] = L;
+      for (int k = 0; k < 3; ++k) S.cen[x][k] = ok ? centers[3 * (natom * g + f.atom) + k] : 0.0;
     }
-    const double* cen = centers + 3 * natom * g;
-    const double* ca = cen + 3 * A.atom;
-    const double* cb = cen + 3 * B.atom;
-    const double* cc = cen + 3 * C.atom;
-    const double* cd = cen + 3 * D.atom;
-    const double qab[3] = {ca[0] - cb[0], ca[1] - cb[1], ca[2] - cb[2]};
-    const double qcd[3] = {cc[0] - cd[0], cc[1] - cd[1], cc[2] - cd[2]};
-    // quartet w = ((((((ta nbt + tb) nct + tc) ndt + td) npa + pa) npb + pb) npc + pc) npd + pd
-    const int nt = A.nterm * B.nterm * C.nterm * D.nterm;
-    const int np = A.nprim * B.nprim * C.nprim * D.nprim;
-    double acc = 0.0;
-    for (int w = lane; w < nt * np; w += 64) {
-      int x = w;
-      const int pd = x % D.nprim; x /= D.nprim;
-      const int pc = x % C.nprim; x /= C.nprim;
-      const int pb = x % B.nprim; x /= B.nprim;
-      const int pa = x % A.nprim; x /= A.nprim;
-      const int td = x % D.nterm; x /= D.nterm;
-      const int tc = x % C.nterm; x /= C.nterm;
-      const int tb = x % B.nterm; x /= B.nterm;
-      const int ta = x;
-      acc += eri_prim(A, B, C, D, ta, tb, tc, td, pa, pb, pc, pd, ca, cb, cc, cd, qab, qcd);
+    __syncthreads();
+    for (int w = tid; w < 4 * EG * 2 * APY_GTO_MAXPRIM; w += 256) {
+      const int k = w % APY_GTO_MAXPRIM, t = (w / APY_GTO_MAXPRIM) % 2, m = (w / (2 * APY_GTO_MAXPRIM)) % EG,
+                x = w / (2 * APY_GTO_MAXPRIM * EG);
+      if (m >= S.size[x]) continue;
+      const apy_gto& f = T.f[x][S.first[x] + m];
+      S.coef[x][m][t][k] = f.coefs[t][k];
+      if (m == 0 && t == 0) S.exps[x][k] = f.exps[k];
+      if (k < 3) S.lmn[x][m][t][k] = (int8_t)f.lmn[t][k];
+      if (k == 3 && t == 0) S.nterm[x][m] = (uint8_t)f.nterm;
     }
-    for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
-    if (lane == 0) put(acc);
+    if (tid < 2 * EPP) {
+      const int x = tid / EPP, b = tid % EPP, n = S.nprim[2 * x + 1];
+      if (n > 0) { S.prim[x][b][0] = (uint8_t)(b / n); S.prim[x][b][1] = (uint8_t)(b % n); }
+    }
+    __syncthreads();
+    const int La = uniform(S.L[0]), Lb = uniform(S.L[1]), Lc = uniform(S.L[2]), Ld = uniform(S.L[3]);
+    const int sz1 = uniform(S.size[1]), sz3 = uniform(S.size[3]);
+    const int nbc = uniform(S.size[0]) * sz1, nkc = uniform(S.size[2]) * sz3;
+    const int nbp = uniform(S.nprim[0] * S.nprim[1]), nkp = uniform(S.nprim[2] * S.nprim[3]);
+    const bool bad = nbp * nkp == 0;
+    const int L1 = La + Lb, L = min(L1 + Lc + Ld, LQ), nr = tuv_count(L), nr1 = tuv_count(min(L1, L));
+    const int eb = 3 * (La + 1) * (Lb + 1) * (L1 + 1), ek = 3 * (Lc + 1) * (Ld + 1) * (Lc + Ld + 1);
+    const int wsz = 4 * (L + 1) + nr;
+    // batches of primitive pairs, ket elements of a slice (all of them but for f functions)
+    const int ks = min(nkc, EH / nr1);
+    const int Kb = max(1, min(nkp, min(EE / ek, EW / wsz)));
+    const int Bb = max(1, min(min(nbp, EE / eb), min(EW / (wsz * Kb), EH / (nr1 * ks))));
+    const int nbt = La + Lb + 1, nkt = Lc + Ld + 1;
+    const SmallDiv dL(L + 1), dR(nr), dR1(nr1), dA(La + 1), dC(Lc + 1), d3(3), dsz1(sz1), dsz3(sz3);
+
+    for (int k0 = 0; k0 < nkc; k0 += ks) {
+      const int nks = min(ks, nkc - k0), nel = nbc * nks;
+      const SmallDiv dK(nks);
+      for (int w = tid; w < nel; w += 256) S.acc[w] = 0.0;
+      for (int b0 = 0; b0 < nbp && !bad; b0 += Bb) {
+        const int nb = min(Bb, nbp - b0);
+        for (int w = tid; w < nb * nks * nr1; w += 256) S.H[w] = 0.0;
+        for (int q0 = 0; q0 < nkp; q0 += Kb) {
+          const int nq = min(Kb, nkp - q0), nbq = nb * nq;
+          const SmallDiv dq(nq);
+          // 1. E of the bra batch (once) and of the ket batch (again only if it changes), G and powers
+          const int nEb = q0 == 0 ? nb * 3 * (La + 1) : 0;
+          const int nEk = (Kb < nkp || b0 == 0) ? nq * 3 * (Lc + 1) : 0;
+          for (int w = tid; w < nEb + nEk + nbq * (L + 1); w += 256) {
+            if (w < nEb) {
+              const int y = dA.div(w), i = dA.mod(w), b = d3.div(y), ax = d3.mod(y);
+              herm_row(i, La, Lb, S.cen[0][ax] - S.cen[1][ax], S.exps[0][S.prim[0][b0 + b][0]],
+                       S.exps[1][S.prim[0][b0 + b][1]], 1.0, S.Eb + b * eb + ax * (eb / 3));
+            } else if (w < nEb + nEk) {
+              const int y = dC.div(w - nEb), i = dC.mod(w - nEb), b = d3.div(y), ax = d3.mod(y);
+              herm_row(i, Lc, Ld, S.cen[2][ax] - S.cen[3][ax], S.exps[2][S.prim[1][q0 + b][0]],
+                       S.exps[3][S.prim[1][q0 + b][1]], -1.0, S.Ek + b * ek + ax * (ek / 3));
+            } else {
+              const int bq = dL.div(w - nEb - nEk), n = dL.mod(w - nEb - nEk), b = b0 + dq.div(bq),
+                        q = q0 + dq.mod(bq);
+              const double xa = S.exps[0][S.prim[0][b][0]], xb = S.exps[1][S.prim[0][b][1]], p = xa + xb;
+              const double xc = S.exps[2][S.prim[1][q][0]], xd = S.exps[3][S.prim[1][q][1]], s = xc + xd;
+              const double alpha = p * s / (p + s);
+              double* Wq = S.W + bq * wsz;
+              double r2 = 0.0;
+              for (int ax = 0; ax < 3; ++ax) {
+                const double d = (xa * S.cen[0][ax] + xb * S.cen[1][ax]) / p -
+                                 (xc * S.cen[2][ax] + xd * S.cen[3][ax]) / s;
+                r2 += d * d;
+                double pw = 1.0;
+                for (int k = 0; k < n; ++k) pw *= d;
+                Wq[(ax + 1) * (L + 1) + n] = pw;
+              }
+              double G_ = 2.0 * M_PI * M_PI * sqrt(M_PI) / (p * s * sqrt(p + s)) * boys_one(n, alpha * r2);
+              for (int k = 0; k < n; ++k) G_ *= -2.0 * alpha;
+              Wq[n] = G_;
+            }
+          }
+          __syncthreads();
+          // 2. R_tuv
+          for (int w = tid; w < nbq * nr; w += 256) {
+            const int rr = dR.mod(w);
+            double* Wq = S.W + dR.div(w) * wsz;
+            const int t = S.tuv[rr][0], u = S.tuv[rr][1], v = S.tuv[rr][2];
+            const double* X = Wq + (L + 1);
+            const double* Y = X + (L + 1);
+            const double* Z = Y + (L + 1);
+            double sx = 0.0;
+            for (int i = 0; 2 * i <= t; ++i) {
+              double sy = 0.0;
+              for (int j = 0; 2 * j <= u; ++j) {
+                double sz = 0.0;
+                for (int k = 0; 2 * k <= v; ++k) sz += S.herm[v][k] * Z[v - 2 * k] * Wq[t + u + v - i - j - k];
+                sy += S.herm[u][j] * Y[u - 2 * j] * sz;
+              }
+              sx += S.herm[t][i] * X[t - 2 * i] * sy;
+            }
+            Wq[4 * (L + 1) + rr] = sx;
+          }
+          __syncthreads();
+          // 3. the ket contraction; where the items are few, 2^sh neighbouring lanes share one
+          const int items = nb * nks * nr1;
+          int sh = 0;
+          while (sh < 6 && (items << (sh + 1)) <= 256 && (1 << sh) < nq) ++sh;
+          const int sub = tid & ((1 << sh) - 1);
+          for (int w = tid >> sh; w < items; w += 256 >> sh) {
+            const int y = dR1.div(w), rr = dR1.mod(w), b = dK.div(y), kc = k0 + dK.mod(y);
+            const int mc = dsz3.div(kc), md = dsz3.mod(kc);
+            const int t = S.tuv[rr][0], u = S.tuv[rr][1], v = S.tuv[rr][2];
+            double h = 0.0;
+            for (int tc = 0; tc < S.nterm[2][mc]; ++tc)
+              for (int td = 0; td < S.nterm[3][md]; ++td) {
+                const int8_t* lc = S.lmn[2][mc][tc];
+                const int8_t* ld = S.lmn[3][md][td];
+                const int lx = lc[0] + ld[0], ly = lc[1] + ld[1], lz = lc[2] + ld[2];
+                if (t + u + v + lx + ly + lz > L) continue;   // read by elements past LQ only (NaN)
+                const int ox = (lc[0] * (Ld + 1) + ld[0]) * nkt, oy = ek / 3 + (lc[1] * (Ld + 1) + ld[1]) * nkt,
+                          oz = 2 * (ek / 3) + (lc[2] * (Ld + 1) + ld[2]) * nkt;
+                for (int q = sub; q < nq; q += 1 << sh) {
+                  const double* R = S.W + (b * nq + q) * wsz + 4 * (L + 1);
+                  const double* E = S.Ek + q * ek;
+                  double sx = 0.0;
+                  for (int i = 0; i <= lx; ++i) {
+                    double sy = 0.0;
+                    for (int j = 0; j <= ly; ++j) {
+                      double sz = 0.0;
+                      for (int k = 0; k <= lz; ++k) sz += E[oz + k] * R[tuv_index(t + i, u + j, v + k)];
+                      sy += E[oy + j] * sz;
+                    }
+                    sx += E[ox + i] * sy;
+                  }
+                  h += S.coef[2][mc][tc][S.prim[1][q0 + q][0]] * S.coef[3][md][td][S.prim[1][q0 + q][1]] * sx;
+                }
+              }
+            for (int o = (1 << sh) >> 1; o > 0; o >>= 1) h += __shfl_xor(h, o, 64);   // lanes of one item: all here
+            if (sub == 0) S.H[w] += h;
+          }
+          __syncthreads();
+        }
+        // the bra contraction of this batch
+        for (int w = tid; w < nel; w += 256) {
+          const int kc = dK.mod(w), bc = dK.div(w), ma = dsz1.div(bc), mb = dsz1.mod(bc);
+          double h = 0.0;
+          for (int ta = 0; ta < S.nterm[0][ma]; ++ta)
+            for (int tb = 0; tb < S.nterm[1][mb]; ++tb) {
+              const int8_t* la = S.lmn[0][ma][ta];
+              const int8_t* lb = S.lmn[1][mb][tb];
+              const int lx = la[0] + lb[0], ly = la[1] + lb[1], lz = la[2] + lb[2];
+              if (lx + ly + lz > L) continue;
+              const int ox = (la[0] * (Lb + 1) + lb[0]) * nbt, oy = eb / 3 + (la[1] * (Lb + 1) + lb[1]) * nbt,
+                        oz = 2 * (eb / 3) + (la[2] * (Lb + 1) + lb[2]) * nbt;
+              for (int b = 0; b < nb; ++b) {
+                const double* Hq = S.H + (b * nks + kc) * nr1;
+                const double* E = S.Eb + b * eb;
+                double sx = 0.0;
+                for (int i = 0; i <= lx; ++i) {
+                  double sy = 0.0;
+                  for (int j = 0; j <= ly; ++j) {
+                    double sz = 0.0;
+                    for (int k = 0; k <= lz; ++k) sz += E[oz + k] * Hq[tuv_index(i, j, k)];
+                    sy += E[oy + j] * sz;
+                  }
+                  sx += E[ox + i] * sy;
+                }
+                h += S.coef[0][ma][ta][S.prim[0][b0 + b][0]] * S.coef[1][mb][tb][S.prim[0][b0 + b][1]] * sx;
+              }
+            }
+          S.acc[w] += h;
+        }
+        __syncthreads();                              // H and E of this batch are read
+      }
+      // ---- out: the value of a canonical element to every image under the launch's symmetry
+      for (int w = tid; w < nel; w += 256) {
+        const int kc = k0 + dK.mod(w), bc = dK.div(w);
+        const int e0 = dsz1.div(bc), e1 = dsz1.mod(bc), e2 = dsz3.div(kc), e3 = dsz3.mod(kc);
+        const int64_t i = S.first[0] + e0, j = S.first[1] + e1, k = S.first[2] + e2, l = S.first[3] + e3;
+        // one element an image class: an order of functions is asked for where the group quartet leaves one open
+        if (sym != ERI_NONE && k < l) continue;
+        if (sym == ERI_ALL && i < j) continue;
+        if (sym == ERI_ALL && G[0] == G[2] && G[1] == G[3] && (i < k || (i == k && j < l))) continue;
+        double v = S.acc[w];
+        if (bad) {
+          v = kNaN;
+        } else {
+          int Lm[4];
+          const int em[4] = {e0, e1, e2, e3};
+          for (int x = 0; x < 4; ++x) {
+            Lm[x] = 0;
+            for (int t = 0; t < S.nterm[x][em[x]]; ++t) {
+              const int8_t* c = S.lmn[x][em[x]][t];
+              Lm[x] = max(Lm[x], c[0] + c[1] + c[2]);
+            }
+          }
+          if (Lm[0] + Lm[1] + Lm[2] + Lm[3] > LQ) v = kNaN;
+        }
+        const double2 y = make_double2(v, 0.0);
+        double2* o = out + g * full;
+        auto at = [&](int64_t p, int64_t q, int64_t s, int64_t t) { return ((p * n1 + q) * n2 + s) * n3 + t; };
+        o[at(i, j, k, l)] = y;
+        if (sym == ERI_NONE) continue;
+        o[at(i, j, l, k)] = y;
+        if (sym == ERI_KET) continue;
+        o[at(j, i, k, l)] = y;
+        o[at(j, i, l, k)] = y;
+        o[at(k, l, i, j)] = y;
+        o[at(l, k, i, j)] = y;
+        o[at(k, l, j, i)] = y;
+        o[at(l, k, j, i)] = y;
+      }
+    }
   }
 }
 
@@ -486,12 +766,17 @@ int apy_eri_gto(int64_t ngeom, int64_t natom, const double* centers, const apy_g
   const int sym = (fa == fb && fb == fc && fc == fd && na == nb && nb == nc && nc == nd) ? ERI_ALL
                   : (fc == fd && nc == nd)                                             ? ERI_KET
                                                                                        : ERI_NONE;
-  const int64_t pc = nc * (nc + 1) / 2;
-  const int64_t per = sym == ERI_ALL ? pc * (pc + 1) / 2 : sym == ERI_KET ? na * nb * pc : na * nb * nc * nd;
-  const int64_t total = ngeom * per;
+  if (na > INT32_MAX || nb > INT32_MAX || nc > INT32_MAX || nd > INT32_MAX) return APY_E_ARG;
   if (const int rc = ensure_boys_table((hipStream_t)stream); rc != APY_OK) return rc;
-  eri_kernel<<<apy_grid1d(64 * total), 256, 0, (hipStream_t)stream>>>(ngeom, natom, centers, fa, na, fb, nb, fc, nc, fd,
-                                                                  nd, sym, (double2*)out);
+  const EriTab T = {{fa, fb, fc, fd}, {na, nb, nc, nd}};
+  // tables whose group starts do not fit LDS are taken function by function
+  const int64_t tot = na + 1 + (sym == ERI_ALL ? 0 : nb + nc + 2 + (sym == ERI_KET ? 0 : nd + 1));
+  const int grouped = tot <= ETAB;
+  // a resident grid (four workgroups a CU): the groups are found once a workgroup
+  const double bound = (double)ngeom * na * nb * nc * nd;
+  const unsigned grid = (unsigned)std::min(bound, 4.0 * 256.0);
+  const size_t lds = grouped ? (size_t)tot * (sizeof(uint16_t) + 1) : 0;
+  eri_kernel<<<grid, 256, lds, (hipStream_t)stream>>>(ngeom, natom, centers, T, sym, grouped, (double2*)out);
   APY_LAUNCH_CHECK();
   return APY_OK;
 }

@@ -23,50 +23,59 @@ from .gaussian import assemble_deriv1, center_derivative
 from .kernels import stream_of
 
 
-def _entry(atom, terms):
-    """One apy_gto entry from (lmn, coefs) terms sharing exps."""
-    g = _lib.Gto()
-    exps = terms[0][2]
-    if len(exps) > _lib.APY_GTO_MAXPRIM or not 1 <= len(terms) <= 2:
+_GTO = np.dtype([("atom", "i4"), ("nprim", "i4"), ("nterm", "i4"), ("lmn", "i4", (2, 3)), ("pad", "i4"),
+                 ("exps", "f8", (_lib.APY_GTO_MAXPRIM,)), ("coefs", "f8", (2, _lib.APY_GTO_MAXPRIM))])
+assert _GTO.itemsize == ctypes.sizeof(_lib.Gto)
+
+
+def _table(atoms, functions, device):
+    """Device apy_gto table: entry i at centre atoms[i] with the terms functions[i], one or two objects with
+    lmn, exps and coefs that share exps.  Filled a field at a time: an entry at a time through ctypes took
+    12 us a function, 0.4 ms of host time for 34 functions whose integrals take 0.2 ms."""
+    n, mp = len(functions), _lib.APY_GTO_MAXPRIM
+    tab = np.zeros(n, dtype=_GTO)
+    nterm = [len(t) for t in functions]
+    first = [t[0] for t in functions]
+    nprim = [len(f.exps) for f in first]
+    if n and (max(nprim) > mp or min(nterm) < 1 or max(nterm) > 2):
         raise ValueError("function outside the integral kernel's limits")
-    g.atom, g.nprim, g.nterm = int(atom), len(exps), len(terms)
-    for k, (lmn, coefs, e) in enumerate(terms):
-        if sum(lmn) > _lib.APY_GTO_MAXL or not np.array_equal(e, exps):
+    tab["atom"], tab["nprim"], tab["nterm"] = atoms, nprim, nterm
+    used = np.arange(mp) < np.asarray(nprim, dtype=np.int64).reshape(n, 1)
+    if n:
+        tab["exps"][used] = np.concatenate([f.exps for f in first])
+    for k in range(2):
+        rows = [i for i in range(n) if nterm[i] > k]
+        if not rows:
+            continue
+        terms = [functions[i][k] for i in rows]
+        lmn = np.array([f.lmn for f in terms], dtype=np.int64)
+        if lmn.sum(axis=1).max() > _lib.APY_GTO_MAXL or any(
+                k and f.exps is not first[i].exps and not np.array_equal(f.exps, first[i].exps)
+                for i, f in zip(rows, terms)):
             raise ValueError("function outside the integral kernel's limits")
-        for x in range(3):
-            g.lmn[k][x] = int(lmn[x])
-        for p in range(len(exps)):
-            g.coefs[k][p] = float(coefs[p])
-    for p in range(len(exps)):
-        g.exps[p] = float(exps[p])
-    return g
-
-
-def _upload(entries, device):
-    arr = (_lib.Gto * len(entries))(*entries)
-    buf = np.frombuffer(bytes(arr), dtype=np.uint8).copy()
-    return torch.from_numpy(buf).to(device)
+        tab["lmn"][rows, k] = lmn
+        at = np.nonzero(used[rows])
+        tab["coefs"][np.asarray(rows)[at[0]], k, at[1]] = np.concatenate(
+            [f.coefs[:len(f.exps)] for f in terms])
+    return torch.from_numpy(tab.view(np.uint8)).to(device)
 
 
 def basis_table(functions, atom_of, device):
     """Device apy_gto table of the basis functions."""
-    return _upload([_entry(a, [(f.lmn, f.coefs, f.exps)]) for f, a in zip(functions, atom_of)], device)
+    return _table(list(atom_of), [(f,) for f in functions], device)
 
 
 def derivative_table(functions, atom_of, axis, device):
     """Device apy_gto table of d f / dA_axis for every basis function f
     (centred at A; gaussian.center_derivative's terms)."""
-    out = []
-    for f, a in zip(functions, atom_of):
-        out.append(_entry(a, [(t.lmn, t.coefs, t.exps) for t in center_derivative(f, axis)]))
-    return _upload(out, device)
+    return _table(list(atom_of), [center_derivative(f, axis) for f in functions], device)
 
 
 def function_table(functions, device):
     """Device apy_gto table in which every function is its own centre
     (entry i at centre i), and the [n, 3] host array of those centres: the
     form for function lists that carry their centres (mixed overlaps)."""
-    tab = _upload([_entry(i, [(f.lmn, f.coefs, f.exps)]) for i, f in enumerate(functions)], device)
+    tab = _table(list(range(len(functions))), [(f,) for f in functions], device)
     return tab, np.stack([np.asarray(f.center, dtype=np.float64) for f in functions])
 
 

@@ -238,3 +238,49 @@ def test_eri_symmetric_launches_match_general_launch(dev, geom, basis):
     for perm in ((1, 0, 2, 3), (0, 1, 3, 2), (2, 3, 0, 1), (3, 2, 1, 0)):
         assert np.array_equal(G8, G8.transpose(perm))
     assert np.array_equal(G2, G2.transpose(0, 1, 3, 2))
+
+
+@pytest.mark.parametrize("case", ["f_shell_split", "six_primitives", "interleaved_centres", "bad_entry"])
+def test_eri_function_groups(dev, case):
+    """Neighbouring functions with one centre and the same exponents are computed together, up to six at a
+    time and in batches of primitive pairs: a shell of ten f functions, six-primitive s, p and d functions
+    sharing exponents (36 primitive pairs a side), equal exponents on alternating centres (groups of one)
+    and a shell with an entry outside the limits inside it.  Elements past a total angular momentum of 9
+    and those of the bad entry are NaN, every other one is the host's.  The sums have up to 1296 terms of
+    like magnitude at most 1e2 times the result: 1e-12 covers their rounding."""
+    rng = np.random.default_rng(5)
+    cen = np.array([[0.1, -0.2, 0.3], [0.9, 0.4, -0.5]])
+    six = np.array([23.0, 8.0, 3.1, 1.3, 0.6, 0.25])
+    R = gaussian.RawGaussian
+    lmns = lambda L: [(x, y, L - x - y) for x in range(L, -1, -1) for y in range(L - x, -1, -1)]
+    if case == "f_shell_split":
+        spec = [(0, l, [1.1, 0.4]) for l in lmns(3)] + [(1, l, [0.8, 0.3]) for l in lmns(1) + lmns(0)]
+    elif case == "six_primitives":
+        spec = [(0, l, six) for l in lmns(0) + lmns(1)] + [(1, l, six) for l in lmns(2)]
+    elif case == "interleaved_centres":
+        spec = [(k % 2, l, [0.9, 0.35]) for k, l in enumerate(lmns(2) + lmns(1))]
+    else:
+        spec = [(0, l, [0.9, 0.35, 0.2]) for l in lmns(2) + lmns(1)]
+    fns = [R(cen[a], l, np.asarray(e, dtype=float), rng.uniform(0.5, 1.5, len(e))) for a, l, e in spec]
+    tab = basis_table(fns, [a for a, _, _ in spec], dev)
+    n, bad = len(fns), -1
+    if case == "bad_entry":
+        bad, size = 3, ctypes.sizeof(_lib.Gto)
+        g = _lib.Gto.from_buffer_copy(bytes(tab[bad * size:(bad + 1) * size].cpu().numpy()))
+        g.lmn[0][0] = _lib.APY_GTO_MAXL + 1
+        tab[bad * size:(bad + 1) * size] = torch.from_numpy(np.frombuffer(bytes(g), dtype=np.uint8).copy()).to(dev)
+    copy = tab.clone()
+    for tabs in ((tab, tab, tab, tab), (copy, copy, tab, tab), (copy, copy, copy, tab)):
+        G = eri(*tabs, (n,) * 4, cen[None], dev).cpu().numpy()[0].real
+        L = np.array([sum(f.lmn) for f in fns])
+        nan = sum(np.ix_(*[L] * 4)) > 9
+        for ax in range(4):
+            sl = [slice(None)] * 4
+            sl[ax] = bad
+            if bad >= 0:
+                nan[tuple(sl)] = True
+        assert np.array_equal(np.isnan(G), nan)
+        good = np.argwhere(~nan)
+        for p in good[rng.integers(0, len(good), 120)]:
+            want = gaussian.eri(*[fns[q] for q in p])
+            assert abs(G[tuple(p)] - want) < 1e-12 * max(1.0, abs(want)), (case, p)
