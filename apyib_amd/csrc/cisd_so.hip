@@ -205,36 +205,45 @@ __global__ void so_fock_kernel(int64_t m, int64_t nb, const double2* fmo, double
 // Every sigma works from the packed doubles T_p[(i<j)][(a<b)] (the packed
 // input itself, or pack_t2 of a dense input); the dense images the GEMMs
 // need are expanded from it with the antisymmetry signs.
-__global__ __launch_bounds__(256) void pack_t2(const double2* __restrict__ t2, double2* __restrict__ tp, int64_t O,
-                                               int64_t V) {
-  const int64_t Po = npair(O), Pv = npair(V), total = Po * Pv;
-  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total; t += (int64_t)gridDim.x * blockDim.x) {
-    int64_t i, j, a, b;
-    pdec(t / Pv, O, i, j);
-    pdec(t % Pv, V, a, b);
-    tp[t] = t2[((i * O + j) * V + a) * V + b];
-  }
-}
+//
+// One launch forms all of them: the grid is cut into sections (in blocks), so that the small copies of a
+// step do not follow each other at a launch's latency each (five launches of 2 to 5 us at O=10 V=4 and
+// O=18 V=50 alike).  A dense input is read at its i < j, a < b elements, which are T_p.
+struct PrepArgs {
+  int64_t O, V;
+  const double2* t2;       // dense input [i][j][a][b] (NULL: tp_in is read)
+  const double2* tp_in;    // packed input
+  double2* tp;             // T_p of a dense input
+  double2* tr;             // T'[(i,a),(k,c)]
+  double2* th;             // Th[i][j][(c<b)] (NULL: none)
+  const double2* ov;       // ovoo_p (NULL: no transposes)
+  double2* ovT;            // [(i<j)][k][b] = <kb||ij>
+  const double2* oo;       // ooov
+  double2* ooT;            // [k][i][(j,b)] = <kj||ib>
+  int32_t ring, pack, half, ovb;   // ends of the sections in blocks; the rest: ooT
+};
 
 __device__ inline int64_t pidx(int64_t p, int64_t q, int64_t N) { return prow(p, N) + q - p - 1; }
 
-// T'[(i,a),(k,c)] = t2[i,k,a,c] from T_p: +T_p[(ik),(ac)] when i<k and a<c
-// (or both reversed), minus when one pair is reversed, zero on i == k or a == c.
-// One workgroup per (i, k, 32 x 32 tile of (a, c)): the packed row (ik) is read in two passes, the
-// a < c half with c fastest and the a > c half with a fastest, so that both read along the packed
-// row; the tile goes through LDS and out along c.
-constexpr int RT = 32;
-__global__ __launch_bounds__(256) void ring_perm_packed(const double2* __restrict__ tp, double2* __restrict__ tr,
-                                                        int64_t O, int64_t V) {
+constexpr int RT = 32;      // edge of a ring tile
+constexpr int PREP_E = 512; // elements of a block of the other sections
+
+__global__ __launch_bounds__(256) void prep_kernel(PrepArgs p) {
   __shared__ double2 T[RT][RT + 1];
-  const int64_t Pv = npair(V), OV = O * V, nt = (V + RT - 1) / RT, tiles = O * O * nt * nt;
-  const int tx = threadIdx.x % RT, ty = threadIdx.x / RT;
-  for (int64_t w = blockIdx.x; w < tiles; w += gridDim.x) {
-    const int64_t tc = w % nt, ta = (w / nt) % nt, k = (w / (nt * nt)) % O, i = w / (nt * nt * O);
-    const int64_t a0 = ta * RT, c0 = tc * RT;
-    const double2* row = i != k ? tp + pidx(i < k ? i : k, i < k ? k : i, O) * Pv : nullptr;
+  const int64_t O = p.O, V = p.V, Po = npair(O), Pv = npair(V), OV = O * V;
+  const int blk = (int)blockIdx.x;
+  if (blk < p.ring) {
+    // T'[(i,a),(k,c)] = t2[i,k,a,c]: +T_p[(ik),(ac)] when i<k and a<c (or both reversed), minus when one
+    // pair is reversed, zero on i == k or a == c.  One block per (i, k, 32 x 32 tile of (a, c)): the row
+    // (ik) is read in two passes, the a < c half with c fastest and the a > c half with a fastest, so that
+    // both read along it; the tile goes through LDS and out along c.
+    const int64_t nt = (V + RT - 1) / RT;
+    const int tx = threadIdx.x % RT, ty = threadIdx.x / RT;
+    const int64_t tc = blk % nt, ta = (blk / nt) % nt, k = (blk / (nt * nt)) % O, i = blk / (nt * nt * O);
+    const int64_t a0 = ta * RT, c0 = tc * RT, lo = i < k ? i : k, hi = i < k ? k : i;
+    const double2* row = i == k ? nullptr : p.t2 ? p.t2 + (lo * O + hi) * V * V : p.tp_in + pidx(lo, hi, O) * Pv;
+    auto at = [&](int64_t x, int64_t y) { return p.t2 ? x * V + y : pidx(x, y, V); };   // x < y
     const double su = i < k ? 1.0 : -1.0;     // sign of the a < c half; the a > c half has -su
-    __syncthreads();                            // the previous tile has been written out
 #pragma unroll
     for (int r = 0; r < RT / 8; ++r) {
       const int ra = ty + 8 * r;
@@ -243,7 +252,7 @@ __global__ __launch_bounds__(256) void ring_perm_packed(const double2* __restric
       if (!(row && a < V && c < V && a > c)) {
         double2 x = make_double2(0.0, 0.0);
         if (row && a < V && c < V && a < c) {
-          const double2 y = row[pidx(a, c, V)];
+          const double2 y = row[at(a, c)];
           x = make_double2(su * y.x, su * y.y);
         }
         T[ra][tx] = x;
@@ -251,7 +260,7 @@ __global__ __launch_bounds__(256) void ring_perm_packed(const double2* __restric
       // lower pass (a fastest): a > c
       const int64_t al = a0 + tx, cl = c0 + ra;
       if (row && al < V && cl < V && al > cl) {
-        const double2 y = row[pidx(cl, al, V)];
+        const double2 y = row[at(cl, al)];
         T[tx][ra] = make_double2(-su * y.x, -su * y.y);
       }
     }
@@ -259,50 +268,63 @@ __global__ __launch_bounds__(256) void ring_perm_packed(const double2* __restric
 #pragma unroll
     for (int r = 0; r < RT / 8; ++r) {
       const int64_t a = a0 + ty + 8 * r, c = c0 + tx;
-      if (a < V && c < V) tr[(i * V + a) * OV + k * V + c] = T[ty + 8 * r][tx];
+      if (a < V && c < V) p.tr[(i * V + a) * OV + k * V + c] = T[ty + 8 * r][tx];
+    }
+    return;
+  }
+  const int first = blk < p.pack ? p.ring : blk < p.half ? p.pack : blk < p.ovb ? p.half : p.ovb;
+#pragma unroll
+  for (int u = 0; u < PREP_E / 256; ++u) {
+    const int64_t t = (int64_t)(blk - first) * PREP_E + u * 256 + threadIdx.x;
+    if (blk < p.pack) {                        // T_p of a dense input
+      if (t >= Po * Pv) return;
+      int64_t i, j, a, b;
+      pdec(t / Pv, O, i, j);
+      pdec(t % Pv, V, a, b);
+      p.tp[t] = p.t2[((i * O + j) * V + a) * V + b];
+    } else if (blk < p.half) {                 // Th[i][j][(c<b)] = t2[i,j,c,b], zero rows for i == j
+      if (t >= O * O * Pv) return;
+      const int64_t P = t % Pv, j = (t / Pv) % O, i = t / (Pv * O), lo = i < j ? i : j, hi = i < j ? j : i;
+      double2 v = make_double2(0.0, 0.0);
+      if (i != j) {
+        if (p.t2) {
+          int64_t c, b;
+          pdec(P, V, c, b);
+          v = p.t2[((lo * O + hi) * V + c) * V + b];
+        } else {
+          v = p.tp_in[pidx(lo, hi, O) * Pv + P];
+        }
+        if (i > j) v = make_double2(-v.x, -v.y);
+      }
+      p.th[t] = v;
+    } else if (blk < p.ovb) {                  // ovT
+      if (t >= Po * OV) return;
+      const int64_t b = t % V, k = (t / V) % O, P = t / OV;
+      p.ovT[t] = p.ov[(k * V + b) * Po + P];
+    } else {                                   // ooT
+      if (t >= O * O * OV) return;
+      const int64_t b = t % V, j = (t / V) % O, i = (t / OV) % O, k = t / (OV * O);
+      p.ooT[t] = p.oo[((k * O + j) * O + i) * V + b];
     }
   }
 }
 
-// Th[i][j][(c<b)] = t2[i,j,c,b] from T_p (zero rows for i == j).
-__global__ __launch_bounds__(256) void half_pack_packed(const double2* __restrict__ tp, double2* __restrict__ th,
-                                                        int64_t O, int64_t Pv) {
-  const int64_t total = O * O * Pv;
-  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total; t += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t P = t % Pv, r = t / Pv;
-    const int64_t j = r % O, i = r / O;
-    double2 v = make_double2(0.0, 0.0);
-    if (i != j) {
-      const double2 w = tp[pidx(i < j ? i : j, i < j ? j : i, O) * Pv + P];
-      v = i < j ? w : make_double2(-w.x, -w.y);
-    }
-    th[t] = v;
-  }
-}
-
-// ovT[(i<j)][k][b] = ovoo_p[k][b][(i<j)] = <kb||ij>
-__global__ __launch_bounds__(256) void ovoo_transpose(const double2* __restrict__ ov, double2* __restrict__ ovT,
-                                                      int64_t O, int64_t V) {
-  const int64_t Po = npair(O), total = Po * O * V;
-  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total; t += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t b = t % V, r = t / V;
-    const int64_t k = r % O, P = r / O;
-    ovT[t] = ov[(k * V + b) * Po + P];
-  }
-}
-
-// ooovT[k][i][(j,b)] = ooov[k][j][i][b] = <kj||ib>
-__global__ __launch_bounds__(256) void ooov_transpose(const double2* __restrict__ x, double2* __restrict__ y,
-                                                      int64_t O, int64_t V) {
-  const int64_t total = O * O * O * V;
-  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total; t += (int64_t)gridDim.x * blockDim.x) {
-    int64_t r = t;
-    const int64_t b = r % V; r /= V;
-    const int64_t j = r % O; r /= O;
-    const int64_t i = r % O;
-    const int64_t k = r / O;
-    y[t] = x[((k * O + j) * O + i) * V + b];
-  }
+int launch_prep(PrepArgs p, hipStream_t st) {
+  const int64_t nt = (p.V + RT - 1) / RT, Po = npair(p.O), Pv = npair(p.V), OV = p.O * p.V;
+  auto blocks = [](int64_t n) { return (n + PREP_E - 1) / PREP_E; };
+  int64_t e = p.O * p.O * nt * nt;
+  p.ring = (int32_t)e;
+  e += p.t2 ? blocks(Po * Pv) : 0;
+  p.pack = (int32_t)e;
+  e += p.th ? blocks(p.O * p.O * Pv) : 0;
+  p.half = (int32_t)e;
+  e += p.ov ? blocks(Po * OV) : 0;
+  p.ovb = (int32_t)e;
+  e += p.ov ? blocks(p.O * p.O * OV) : 0;
+  if (e > 0x7fffffffLL) return APY_E_ARG;
+  prep_kernel<<<(unsigned)e, 256, 0, st>>>(p);
+  APY_LAUNCH_CHECK();
+  return APY_OK;
 }
 
 __global__ __launch_bounds__(256) void ring_fock_kernel(int64_t O, int64_t V, const double2* __restrict__ F,
@@ -380,6 +402,10 @@ struct Epi2Args {
   double2* tn;             // residual mode: t + r/D, same layout as out
   int mode;
   int packed;
+  const double2* s1;       // singles accumulator (NULL: no singles in this launch)
+  double2* out1;
+  double2* tn1;
+  int32_t doubles;         // blocks of the doubles (0: singles only); the singles' blocks follow
 };
 
 __device__ inline void epi_dense_transposed(const Epi2Args& e, double2 (*L)[ET + 1], double2* base, int64_t i,
@@ -398,7 +424,7 @@ __device__ inline void epi_dense_transposed(const Epi2Args& e, double2 (*L)[ET +
   }
 }
 
-__global__ __launch_bounds__(256) void epi2_doubles(Epi2Args e) {
+__device__ __forceinline__ void epi2_doubles(const Epi2Args& e) {
   __shared__ double2 L[ET][ET + 1];
   __shared__ double2 sA[EKC][ET], sB[EKC][ET], oA[EKC][ET], oB[EKC][ET];
   const int tid = threadIdx.x, tx = tid & (ET - 1), ty = tid >> 5;
@@ -537,31 +563,49 @@ __global__ __launch_bounds__(256) void epi2_doubles(Epi2Args e) {
   }
 }
 
-__global__ void epi_singles(int64_t O, int64_t V, int64_t n, const double2* __restrict__ F,
-                            const double* __restrict__ eps, const double2* E, double c0r, double c0i,
-                            const double2* __restrict__ s1, const double2* t1, double2* t1n, double2* out1,
-                            int mode, const double2* c0p) {
-  const int64_t total = O * V;
-  if (c0p) { c0r = c0p->x; c0i = c0p->y; }
-  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total; t += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t i = t / V, a = t % V;
-    double2 f = F[(O + a) * n + i];
-    double2 s = s1[t];
-    s.x += c0r * f.x - c0i * f.y;
-    s.y += c0r * f.y + c0i * f.x;
-    if (mode == APY_MODE_RESIDUAL) {
-      const double2 tv = t1[t];
-      const double2 Ev = *E;
-      double2 r = s;
-      r.x -= Ev.x * tv.x - Ev.y * tv.y;
-      r.y -= Ev.x * tv.y + Ev.y * tv.x;
-      const double D = eps[i] - eps[O + a];
-      t1n[t] = make_double2(tv.x + r.x / D, tv.y + r.y / D);
-      out1[t] = r;
-    } else {
-      out1[t] = s;
-    }
+__device__ __forceinline__ void epi_singles(const Epi2Args& e, int64_t t) {
+  const int64_t O = e.O, V = e.V;
+  if (t >= O * V) return;
+  const double2 c0 = e.c0p ? *e.c0p : make_double2(e.c0r, e.c0i);
+  const int64_t i = t / V, a = t % V;
+  const double2 f = e.F[(O + a) * e.n + i];
+  double2 s = e.s1[t];
+  s.x += c0.x * f.x - c0.y * f.y;
+  s.y += c0.x * f.y + c0.y * f.x;
+  if (e.mode == APY_MODE_RESIDUAL) {
+    const double2 tv = e.t1[t], E = *e.E;
+    s.x -= E.x * tv.x - E.y * tv.y;
+    s.y -= E.x * tv.y + E.y * tv.x;
+    const double D = e.eps[i] - e.eps[O + a];
+    e.tn1[t] = make_double2(tv.x + s.x / D, tv.y + s.y / D);
   }
+  e.out1[t] = s;
+}
+
+__global__ __launch_bounds__(256) void epi_kernel(Epi2Args e) {
+  if ((int)blockIdx.x >= e.doubles) {
+    epi_singles(e, (int64_t)((int)blockIdx.x - e.doubles) * 256 + threadIdx.x);
+    return;
+  }
+  epi2_doubles(e);
+}
+
+// Both epilogues in one launch, unless the singles are written over the t1 that the doubles still read
+// (a step with t_new == t).
+int launch_epi(Epi2Args e, int64_t t_len, hipStream_t st) {
+  const int64_t nt = (e.V + ET - 1) / ET, nd = npair(e.O) * (nt * (nt + 1) / 2), ns = (e.O * e.V + 255) / 256;
+  if (nd + ns > 0x7fffffffLL) return APY_E_ARG;
+  auto hits = [&](const double2* p) { return p && p < e.t1 + t_len && e.t1 < p + t_len; };
+  e.doubles = (int32_t)nd;
+  const bool split = e.s1 && (hits(e.out1) || (e.mode == APY_MODE_RESIDUAL && hits(e.tn1)));
+  epi_kernel<<<(unsigned)(nd + (e.s1 && !split ? ns : 0)), 256, 0, st>>>(e);
+  APY_LAUNCH_CHECK();
+  if (split) {
+    e.doubles = 0;
+    epi_kernel<<<(unsigned)ns, 256, 0, st>>>(e);
+    APY_LAUNCH_CHECK();
+  }
+  return APY_OK;
 }
 
 // Energy partial sums: terms l < OV are t1[i,a] f[i,O+a]; the rest 1/4 t2*oovv
@@ -632,6 +676,25 @@ __global__ void finalize_sum(const double2* __restrict__ partial, int np, double
 }
 
 constexpr int ENERGY_BLOCKS = 1024;
+
+// Blocks of the energy's partial sums over n terms: four terms a thread, and one block (which then writes
+// the energy itself) where a second launch would take longer than the terms do.
+inline int energy_blocks(int64_t n) {
+  if (n <= 4096) return 1;
+  return (int)std::min<int64_t>(ENERGY_BLOCKS, (n + 1023) / 1024);
+}
+
+int launch_energy(int64_t O, int64_t V, int singles, int packed, const double2* F, const double2* oovv,
+                  const double2* t, double2* part, double2* energy, hipStream_t st) {
+  const int nb = energy_blocks(O * V + (packed ? npair(O) * npair(V) : O * O * V * V));
+  energy_partial<<<nb, 256, 0, st>>>(O, V, O + V, singles, packed, F, oovv, t, nb > 1 ? part : energy);
+  APY_LAUNCH_CHECK();
+  if (nb > 1) {
+    finalize_sum<<<1, 256, 0, st>>>(part, nb, energy);
+    APY_LAUNCH_CHECK();
+  }
+  return APY_OK;
+}
 
 inline size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 
@@ -723,15 +786,17 @@ void sigma_gemms(int64_t O, int64_t V, int nb, int singles, const apy_so_ints* I
 }
 
 // exact = 1 sizes the GEMM region for the plans that would run now instead of
-// every plan the tuner may pick (the no-allocation entry point).
+// every plan the tuner may pick (the no-allocation entry point); grouped = 1 for
+// the products in one launch (a query's size: a step takes less, one product after
+// another then).
 SigmaWS carve(int64_t O, int64_t V, int nb, int singles, int dense_in, const void* ring_f, void* base,
-              int exact = 0) {
+              int exact = 0, int grouped = 0) {
   const int64_t Po = npair(O), Pv = npair(V), OV = O * V;
   SigmaWS w{};
   size_t off = 0;
-  char* b = (char*)base;
+  char* b = base ? (char*)base : (char*)256;     // a query's addresses are only compared with each other
   auto take = [&](size_t elems) -> double2* {
-    double2* p = b ? (double2*)(b + off) : nullptr;
+    double2* p = (double2*)(b + off);
     off += al256(elems * sizeof(double2));
     return p;
   };
@@ -752,7 +817,8 @@ SigmaWS carve(int64_t O, int64_t V, int nb, int singles, int dense_in, const voi
   sigma_gemms(O, V, nb, singles, nullptr, nullptr, nullptr, nullptr, ring_f, w, G);
   size_t g = 0;
   for (const apy_gemm_desc& d : G) g = std::max(g, exact ? apy_zgemm_plan_ws_bytes(&d) : apy_zgemm_ws_bytes(&d));
-  w.gemm = b ? (void*)(b + off) : nullptr;
+  if (grouped) g = std::max(g, apy_zgemm_group_ws_bytes(G.data(), (int)G.size()));
+  w.gemm = (void*)(b + off);
   w.gemm_bytes = g;
   off += al256(g);
   w.total = off;
@@ -773,33 +839,26 @@ int sigma_body(int64_t O, int64_t V, int nb, int singles, const apy_so_ints* I, 
   if (singles && nb == 1) w.t1 = (double2*)t[0];   // one instance: t1 read in place
   for (int k = 0; k < nb; ++k) {
     double2* tpk = w.tp + k * PP;
-    if (!packed_in) {
-      pack_t2<<<apy_grid1d(PP, 1 << 20), 256, 0, st>>>(t[k] + OV, tpk, O, V);
-      APY_LAUNCH_CHECK();
+    PrepArgs p{};
+    p.O = O; p.V = V;
+    p.t2 = packed_in ? nullptr : t[k] + OV;
+    p.tp_in = tpk;
+    p.tp = tpk;
+    p.tr = w.tr + k * OV * OV;
+    if (singles) p.th = w.th + k * O * O * Pv;
+    if (singles && k == 0) {
+      p.ov = (const double2*)I->ovoo_p; p.ovT = w.ovT;
+      p.oo = (const double2*)I->ooov; p.ooT = w.ooT;
     }
-    ring_perm_packed<<<(unsigned)std::min<int64_t>(O * O * ((V + RT - 1) / RT) * ((V + RT - 1) / RT), 1 << 20), 256, 0, st>>>(
-        tpk, w.tr + k * OV * OV, O, V);
-    APY_LAUNCH_CHECK();
-    if (singles) {
-      half_pack_packed<<<apy_grid1d(O * O * Pv, 1 << 20), 256, 0, st>>>(tpk, w.th + k * O * O * Pv, O, Pv);
-      APY_LAUNCH_CHECK();
-      if (nb > 1)
-        APY_HIP_TRY(hipMemcpyAsync(w.t1 + k * OV, t[k], OV * sizeof(double2), hipMemcpyDeviceToDevice, st));
-    }
-  }
-  if (singles) {
-    ovoo_transpose<<<apy_grid1d(Po * OV), 256, 0, st>>>((const double2*)I->ovoo_p, w.ovT, O, V);
-    APY_LAUNCH_CHECK();
-    ooov_transpose<<<apy_grid1d(O * O * OV), 256, 0, st>>>((const double2*)I->ooov, w.ooT, O, V);
-    APY_LAUNCH_CHECK();
+    const int s = launch_prep(p, st);
+    if (s != APY_OK) return s;
+    if (singles && nb > 1)
+      APY_HIP_TRY(hipMemcpyAsync(w.t1 + k * OV, t[k], OV * sizeof(double2), hipMemcpyDeviceToDevice, st));
   }
   std::vector<apy_gemm_desc> G;
   sigma_gemms(O, V, nb, singles, I, F, hoo, t, ring_f, w, G, g3);
-  for (size_t q = 0; q < G.size(); ++q) {
-    const int s = q == 0 ? apy_zgemm_launch(&G[q], w.gemm, w.gemm_bytes, st, ev0, ev1)
-                         : apy_zgemm_launch(&G[q], w.gemm, w.gemm_bytes, st);
-    if (s != APY_OK) return s;
-  }
+  const int s = apy_zgemm_group(G.data(), (int)G.size(), w.gemm, w.gemm_bytes, st, ev0, ev1);
+  if (s != APY_OK) return s;
   return APY_OK;
 }
 
@@ -820,11 +879,6 @@ Epi2Args epi_args(int64_t O, int64_t V, int nb, int k, int singles, const apy_so
   e.fov = (singles && fov) ? 1 : 0;
   e.Tp = w.tp + k * Po * Pv;
   return e;
-}
-
-inline unsigned epi_grid(int64_t O, int64_t V) {
-  const int64_t nt = (V + ET - 1) / ET;
-  return (unsigned)(npair(O) * (nt * (nt + 1) / 2));
 }
 
 }  // namespace
@@ -889,8 +943,10 @@ int apy_cisd_so_ring_fock(int64_t O, int64_t V, const void* fock, const void* ri
 
 size_t apy_cisd_so_workspace(int64_t O, int64_t V, int singles) {
   if (O < 0 || V < 0) return 0;
-  // sized for a dense input and no ring_f: covers every call of this (O, V)
-  return carve(O, V, 1, singles ? 1 : 0, 1, nullptr, nullptr).total;
+  // a dense input, without and with ring_f (any non-null address here): covers every call of this (O, V)
+  const int sg = singles ? 1 : 0;
+  return std::max(carve(O, V, 1, sg, 1, nullptr, nullptr, 0, 1).total,
+                  carve(O, V, 1, sg, 1, (const void*)256, nullptr, 0, 1).total);
 }
 
 }  // extern "C"
@@ -915,8 +971,9 @@ int apy_cisd_so_step_ws(const apy_cisd_so_args* A, void* workspace, size_t ws_by
   hipStream_t st = (hipStream_t)stream;
   SigmaWS w = carve(O, V, 1, singles, !packed, A->ring_f, workspace, exact);
   if (!workspace || ws_bytes < w.total) return APY_E_WORKSPACE;
+  w.gemm_bytes = ws_bytes - (size_t)((char*)w.gemm - (char*)workspace);
 
-  const int64_t OV = O * V, n = O + V;
+  const int64_t OV = O * V;
   const double2* t = (const double2*)A->t;
   double2* tn = (double2*)A->t_new;
   double2* out = (double2*)A->out;
@@ -939,14 +996,10 @@ int apy_cisd_so_step_ws(const apy_cisd_so_args* A, void* workspace, size_t ws_by
   e.tn = tn ? tn + OV : nullptr;
   e.mode = A->mode;
   e.packed = packed;
-  epi2_doubles<<<epi_grid(O, V), 256, 0, st>>>(e);
-  APY_LAUNCH_CHECK();
-  if (singles) {
-    epi_singles<<<apy_grid1d(OV), 256, 0, st>>>(O, V, n, F, A->eps, (const double2*)A->energy, c0r, c0i, w.s1, t, tn,
-                                                out, A->mode, c0p);
-    APY_LAUNCH_CHECK();
-  }
-  return APY_OK;
+  e.s1 = singles ? w.s1 : nullptr;
+  e.out1 = out;
+  e.tn1 = tn;
+  return launch_epi(e, OV, st);
 }
 
 size_t apy_cisd_so_ws_exact(const apy_cisd_so_args* A) {
@@ -987,12 +1040,8 @@ static int energy_impl(int64_t O, int64_t V, int singles, int packed, const void
   if (O < 0 || V < 0 || !fock || !oovv || !t || !energy) return APY_E_ARG;
   if (!workspace || ws_bytes < ENERGY_BLOCKS * sizeof(double2)) return APY_E_WORKSPACE;
   hipStream_t st = (hipStream_t)stream;
-  energy_partial<<<ENERGY_BLOCKS, 256, 0, st>>>(O, V, O + V, singles, packed, (const double2*)fock,
-                                                (const double2*)oovv, (const double2*)t, (double2*)workspace);
-  APY_LAUNCH_CHECK();
-  finalize_sum<<<1, 256, 0, st>>>((const double2*)workspace, ENERGY_BLOCKS, (double2*)energy);
-  APY_LAUNCH_CHECK();
-  return APY_OK;
+  return launch_energy(O, V, singles, packed, (const double2*)fock, (const double2*)oovv, (const double2*)t,
+                       (double2*)workspace, (double2*)energy, st);
 }
 
 int apy_cisd_so_energy(int64_t O, int64_t V, int singles, const void* fock, const void* oovv, const void* t,
@@ -1031,7 +1080,7 @@ int apy_cisd_so_sigma_batch(const apy_cisd_so_sigma_batch_args* A, void* workspa
   SigmaWS w = carve(O, V, nb, singles, 1, nullptr, workspace);
   if (!workspace || ws_bytes < w.total) return APY_E_WORKSPACE;
   hipStream_t st = (hipStream_t)stream;
-  const int64_t OV = O * V, n = O + V;
+  const int64_t OV = O * V;
   std::vector<const double2*> F(nb), T(nb);
   std::vector<const void*> H(nb);
   for (int k = 0; k < nb; ++k) {
@@ -1049,13 +1098,10 @@ int apy_cisd_so_sigma_batch(const apy_cisd_so_sigma_batch_args* A, void* workspa
     e.out = out + OV;
     e.mode = APY_MODE_SIGMA;
     e.packed = 0;
-    epi2_doubles<<<epi_grid(O, V), 256, 0, st>>>(e);
-    APY_LAUNCH_CHECK();
-    if (singles) {
-      epi_singles<<<apy_grid1d(OV), 256, 0, st>>>(O, V, n, F[k], nullptr, nullptr, e.c0r, e.c0i, w.s1 + k * OV,
-                                                  T[k], nullptr, out, APY_MODE_SIGMA, nullptr);
-      APY_LAUNCH_CHECK();
-    }
+    e.s1 = singles ? w.s1 + k * OV : nullptr;
+    e.out1 = out;
+    const int qs = launch_epi(e, OV, st);
+    if (qs != APY_OK) return qs;
   }
   return APY_OK;
 }
@@ -1105,13 +1151,13 @@ void fock_gemms(int64_t O, int64_t V, const double2* F, const void* hoo, const d
   G.push_back(d);
 }
 
-FockWS carve_fock(int64_t O, int64_t V, void* base) {
+FockWS carve_fock(int64_t O, int64_t V, void* base, int grouped = 0) {
   const int64_t Po = npair(O), Pv = npair(V), OV = O * V;
   FockWS w{};
   size_t off = 0;
-  char* b = (char*)base;
+  char* b = base ? (char*)base : (char*)256;
   auto take = [&](size_t elems) -> double2* {
-    double2* p = b ? (double2*)(b + off) : nullptr;
+    double2* p = (double2*)(b + off);
     off += al256(elems * sizeof(double2));
     return p;
   };
@@ -1124,7 +1170,8 @@ FockWS carve_fock(int64_t O, int64_t V, void* base) {
   fock_gemms(O, V, nullptr, nullptr, nullptr, w, G);
   size_t g = 0;
   for (const apy_gemm_desc& d : G) g = std::max(g, apy_zgemm_ws_bytes(&d));
-  w.gemm = b ? (void*)(b + off) : nullptr;
+  if (grouped) g = std::max(g, apy_zgemm_group_ws_bytes(G.data(), (int)G.size()));
+  w.gemm = (void*)(b + off);
   w.gemm_bytes = g;
   off += al256(g);
   w.total = off;
@@ -1137,7 +1184,7 @@ extern "C" {
 
 size_t apy_cisd_so_fock_sigma_workspace(int64_t O, int64_t V) {
   if (O < 2 || V < 2) return 0;
-  return carve_fock(O, V, nullptr).total;
+  return carve_fock(O, V, nullptr, 1).total;
 }
 
 int apy_cisd_so_fock_sigma(const apy_cisd_so_fock_sigma_args* A, void* workspace, size_t ws_bytes, void* stream) {
@@ -1153,18 +1200,18 @@ int apy_cisd_so_fock_sigma(const apy_cisd_so_fock_sigma_args* A, void* workspace
   const int64_t Po = npair(O), Pv = npair(V), OV = O * V, n = O + V, PP = Po * Pv;
   const double2* t = (const double2*)A->t;
   const double2* c0p = t + OV + PP;
-  ring_perm_packed<<<(unsigned)std::min<int64_t>(O * O * ((V + RT - 1) / RT) * ((V + RT - 1) / RT), 1 << 20), 256, 0, st>>>(
-      t + OV, w.tr, O, V);
-  APY_LAUNCH_CHECK();
+  PrepArgs pa{};
+  pa.O = O; pa.V = V; pa.tp_in = t + OV; pa.tr = w.tr;
+  const int ps = launch_prep(pa, st);
+  if (ps != APY_OK) return ps;
   std::vector<apy_gemm_desc> G;
   for (int f = 0; f < nf; ++f) {
     const double2* F = (const double2*)A->fock[f];
     double2* out = (double2*)A->out[f];
     fock_gemms(O, V, F, A->hoo[f], t, w, G);
-    for (const apy_gemm_desc& d : G) {
-      const int s = apy_zgemm_launch(&d, w.gemm, w.gemm_bytes, st);
-      if (s != APY_OK) return s;
-    }
+    const int gs = apy_zgemm_group(G.data(), (int)G.size(), w.gemm,
+                                   ws_bytes - (size_t)((char*)w.gemm - (char*)workspace), st);
+    if (gs != APY_OK) return gs;
     Epi2Args e{};
     e.O = O; e.V = V; e.Po = Po; e.Pv = Pv; e.n = n;
     e.ntile = (int)((V + ET - 1) / ET);
@@ -1182,15 +1229,12 @@ int apy_cisd_so_fock_sigma(const apy_cisd_so_fock_sigma_args* A, void* workspace
     e.out = out + OV;
     e.mode = APY_MODE_SIGMA;
     e.packed = 1;
-    epi2_doubles<<<epi_grid(O, V), 256, 0, st>>>(e);
-    APY_LAUNCH_CHECK();
-    epi_singles<<<apy_grid1d(OV), 256, 0, st>>>(O, V, n, F, nullptr, nullptr, 0.0, 0.0, w.s1, t, nullptr, out,
-                                                APY_MODE_SIGMA, c0p);
-    APY_LAUNCH_CHECK();
-    energy_partial<<<ENERGY_BLOCKS, 256, 0, st>>>(O, V, n, 1, 1, F, nullptr, t, w.part);
-    APY_LAUNCH_CHECK();
-    finalize_sum<<<1, 256, 0, st>>>(w.part, ENERGY_BLOCKS, out + OV + PP);
-    APY_LAUNCH_CHECK();
+    e.s1 = w.s1;
+    e.out1 = out;
+    const int qs = launch_epi(e, OV, st);
+    if (qs != APY_OK) return qs;
+    const int es = launch_energy(O, V, 1, 1, F, nullptr, t, w.part, out + OV + PP, st);
+    if (es != APY_OK) return es;
   }
   return APY_OK;
 }

@@ -33,8 +33,6 @@
 #include "common.h"
 
 #include <algorithm>
-#include <map>
-#include <mutex>
 
 namespace {
 
@@ -190,26 +188,6 @@ __global__ __launch_bounds__(256) void sp_ladder_kernel(Dirac g, int64_t o, int6
   }
 }
 
-// T+[(i<=j)][(c<=d)] = (t_ijcd + t_ijdc)/2, T-[(i<j)][(c<d)] = (t_ijcd - t_ijdc)/2
-// T+ / T- of nb amplitude vectors (stride L, doubles at offset o*v) into [nb][(i<=j)][(c<=d)] and
-// [nb][(i<j)][(c<d)]
-__global__ __launch_bounds__(256) void sp_pack_kernel(int64_t o, int64_t v, int64_t nb, int64_t L,
-                                                      const double2* __restrict__ tv, double2* __restrict__ ts,
-                                                      double2* __restrict__ ta) {
-  const int64_t per = o * o * v * v, total = nb * per, sv = nsym(v), av = nanti(v), so = nsym(o), ao = nanti(o);
-  for (int64_t u = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; u < total; u += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t q = u / per, t = u % per;
-    const int64_t d = t % v, c = (t / v) % v, j = (t / (v * v)) % o, i = t / (v * v * o);
-    if (i > j || c > d) continue;
-    const double2* t2 = tv + q * L + o * v;
-    const double2 x = t2[t], y = t2[((i * o + j) * v + d) * v + c];
-    ts[q * so * sv + isym(i, j, o) * sv + isym(c, d, v)] =
-        c == d ? x : make_double2(0.5 * (x.x + y.x), 0.5 * (x.y + y.y));
-    if (i < j && c < d)
-      ta[q * ao * av + ianti(i, j, o) * av + ianti(c, d, v)] = make_double2(0.5 * (x.x - y.x), 0.5 * (x.y - y.y));
-  }
-}
-
 // Hoo[(i,j)][(k,l)] = <kl|ij> - F[k][i] d(l,j) - F[l][j] d(k,i);  g = [2 F_ov | -F_ov]
 __global__ __launch_bounds__(256) void sp_prepare_kernel(int64_t o, int64_t v, const double2* __restrict__ F,
                                                          const double2* __restrict__ oooo, double2* __restrict__ hoo,
@@ -231,18 +209,40 @@ __global__ __launch_bounds__(256) void sp_prepare_kernel(int64_t o, int64_t v, c
   }
 }
 
-// TU[q][(i,a)][(k,c)] = t_ikac, TU[q][(i,a)][ov + (k,c)] = t_ikca = t_kiac for the nb vectors (stride L)
-__global__ __launch_bounds__(256) void sp_tu_kernel(int64_t o, int64_t v, int64_t nb, int64_t L,
-                                                    const double2* __restrict__ tv, double2* __restrict__ TU) {
-  const int64_t ov = o * v, per = 2 * ov * ov, total = nb * per;
+// The images of nb amplitude vectors (stride L, doubles at offset o*v) that the products read, in one
+// launch (sections of the element range, each 1 to 5 us by itself):
+//   TU[q][(i,a)][(k,c)] = t_ikac, TU[q][(i,a)][ov + (k,c)] = t_ikca = t_kiac,
+//   T+[q][(i<=j)][(c<=d)] = (t_ijcd + t_ijdc)/2, T-[q][(i<j)][(c<d)] = (t_ijcd - t_ijdc)/2,
+//   T1[q][(i,a)] = t1 of vector q, stacked for one product (T1 NULL: none).
+__global__ __launch_bounds__(256) void sp_prep_kernel(int64_t o, int64_t v, int64_t nb, int64_t L,
+                                                      const double2* __restrict__ tv, double2* __restrict__ TU,
+                                                      double2* __restrict__ ts, double2* __restrict__ ta,
+                                                      double2* __restrict__ T1) {
+  const int64_t ov = o * v, d2 = ov * ov, sv = nsym(v), av = nanti(v), so = nsym(o), ao = nanti(o);
+  const int64_t total = nb * (3 * d2 + (T1 ? ov : 0));
   for (int64_t u = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; u < total; u += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t q = u / per, t = u % per;
-    const int64_t row = t / (2 * ov), col = t % (2 * ov);
-    const int64_t i = row / v, a = row % v;
-    const int64_t cc = col % ov, k = cc / v, c = cc % v;
-    const double2* t2 = tv + q * L + ov;
-    // t_ikca = t_kiac by the pair symmetry: both halves read along c
-    TU[u] = col < ov ? t2[((i * o + k) * v + a) * v + c] : t2[((k * o + i) * v + a) * v + c];
+    if (u < nb * 2 * d2) {
+      const int64_t q = u / (2 * d2), t = u % (2 * d2);
+      const int64_t row = t / (2 * ov), col = t % (2 * ov);
+      const int64_t i = row / v, a = row % v;
+      const int64_t cc = col % ov, k = cc / v, c = cc % v;
+      const double2* t2 = tv + q * L + ov;
+      // t_ikca = t_kiac by the pair symmetry: both halves read along c
+      TU[u] = col < ov ? t2[((i * o + k) * v + a) * v + c] : t2[((k * o + i) * v + a) * v + c];
+    } else if (u < nb * 3 * d2) {
+      const int64_t q = (u - nb * 2 * d2) / d2, t = (u - nb * 2 * d2) % d2;
+      const int64_t d = t % v, c = (t / v) % v, j = (t / (v * v)) % o, i = t / (v * v * o);
+      if (i > j || c > d) continue;
+      const double2* t2 = tv + q * L + ov;
+      const double2 x = t2[t], y = t2[((i * o + j) * v + d) * v + c];
+      ts[q * so * sv + isym(i, j, o) * sv + isym(c, d, v)] =
+          c == d ? x : make_double2(0.5 * (x.x + y.x), 0.5 * (x.y + y.y));
+      if (i < j && c < d)
+        ta[q * ao * av + ianti(i, j, o) * av + ianti(c, d, v)] = make_double2(0.5 * (x.x - y.x), 0.5 * (x.y - y.y));
+    } else {
+      const int64_t w = u - nb * 3 * d2;
+      T1[w] = tv[(w / ov) * L + w % ov];
+    }
   }
 }
 
@@ -298,13 +298,6 @@ __global__ __launch_bounds__(256) void sp_to_so_kernel(int64_t o, int64_t v, int
   }
 }
 
-// T1[q][(i,a)] = t1 of vector q (stride L): the singles of nb vectors stacked for one product
-__global__ __launch_bounds__(256) void sp_t1_stack(int64_t ov, int64_t nb, int64_t L, const double2* __restrict__ tv,
-                                                   double2* __restrict__ T1) {
-  for (int64_t u = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; u < nb * ov; u += (int64_t)gridDim.x * blockDim.x)
-    T1[u] = tv[(u / ov) * L + u % ov];
-}
-
 // Epilogue operands; every per-instance array is instance 0's, the others follow at the region
 // strides (so*sv for Ps, ao*av for Pa, (ov)^2 for R, Y, X1, X2, Q1, Q2; L for the vectors).
 struct SpEpi {
@@ -329,6 +322,16 @@ struct SpEpi {
   double2 rs;
   const double2* es;
   int64_t s_eps, s_vvoo;  // per-instance strides of eps and vvoo (0: shared by the instances)
+  // singles: F and its instance stride, their accumulator [nb][ov] (NULL: CID, zeros are written), vectors
+  const double2* fock;
+  int64_t s_fock;
+  const double2* acc;
+  const double2* t1;
+  const double2* rb1;
+  const double2* rt1;
+  double2* t1_new;
+  double2* r1;
+  int32_t doubles;        // blocks of the doubles; the singles' blocks follow
 };
 
 // scalar of the response term of instance q: re[q] + rs + es[q] (null arrays read as zero)
@@ -345,13 +348,13 @@ constexpr int SET = 32;  // edge of the (a, b) tile of the doubles epilogue
 // a > b half of the ladder) are summed while reading them along a, into one LDS tile, and read
 // back along b; every other operand is read along b directly.  All global reads and writes are
 // along the contiguous index.
-__global__ __launch_bounds__(256) void sp_epi_doubles(SpEpi e) {
+__device__ __forceinline__ void sp_epi_doubles(const SpEpi& e) {
   __shared__ double2 T[SET][SET + 1];  // T[b - b0][a - a0]: the transposed terms of output (a, b)
   const int64_t o = e.o, v = e.v, ov = o * v, vv = v * v, per = ov * ov;
   const int64_t nt = (v + SET - 1) / SET, tiles = e.nb * o * o * nt * nt;
   const int64_t so = nsym(o), sv = nsym(v), ao = nanti(o), av = nanti(v);
   const int tx = threadIdx.x % SET, ty = threadIdx.x / SET;
-  for (int64_t w = blockIdx.x; w < tiles; w += gridDim.x) {
+  for (int64_t w = blockIdx.x; w < tiles; w += e.doubles) {
     int64_t r = w;
     const int64_t tb = r % nt; r /= nt;
     const int64_t ta = r % nt; r /= nt;
@@ -452,41 +455,37 @@ __global__ __launch_bounds__(256) void sp_epi_doubles(SpEpi e) {
 }
 
 // r1 = F[a][i] + acc - E t1 (ci_wfn.py:457-464); t1_new = t1 + r1 / D_ia, per instance (acc [nb][ov],
-// vectors L apart)
-__global__ __launch_bounds__(256) void sp_epi_singles(int64_t o, int64_t v, int64_t nb, int64_t L,
-                                                      const double* __restrict__ eps, const double2* __restrict__ F,
-                                                      const double2* __restrict__ acc, const double2* __restrict__ t1,
-                                                      const double2* __restrict__ energy, double2* __restrict__ t1_new,
-                                                      double2* __restrict__ r1, const double2* __restrict__ rb,
-                                                      const double2* __restrict__ rt, const double2* __restrict__ re,
-                                                      double2 rs, const double2* __restrict__ es, int64_t s_eps,
-                                                      int64_t s_fock) {
-  const int64_t n = o + v, ov = o * v, total = nb * ov;
-  for (int64_t u = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; u < total; u += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t q = u / ov, t = u % ov, qv = q * L;
-    const int64_t i = t / v, a = t % v;
-    const double2 E = energy[q];
-    const double2 f = F[q * s_fock + (o + a) * n + i], s = acc[u], x = t1[qv + t];
-    double2 r = make_double2(f.x + s.x - (E.x * x.x - E.y * x.y), f.y + s.y - (E.x * x.y + E.y * x.x));
-    if (rb) {
-      const double2 c = resp_scalar(re, rs, es, q), bb = rb[qv + t], y = rt[t];
-      r.x += bb.x - (c.x * y.x - c.y * y.y);
-      r.y += bb.y - (c.x * y.y + c.y * y.x);
-    }
-    const double D = eps[q * s_eps + i] - eps[q * s_eps + o + a];
-    r1[qv + t] = r;
-    t1_new[qv + t] = make_double2(x.x + r.x / D, x.y + r.y / D);
+// vectors L apart); CID keeps the singles block of the vectors at zero
+__device__ __forceinline__ void sp_epi_singles(const SpEpi& e, int64_t u) {
+  const int64_t o = e.o, v = e.v, n = o + v, ov = o * v;
+  if (u >= e.nb * ov) return;
+  const int64_t q = u / ov, t = u % ov, qv = q * e.L;
+  if (!e.acc) {
+    e.t1_new[qv + t] = make_double2(0.0, 0.0);
+    e.r1[qv + t] = make_double2(0.0, 0.0);
+    return;
   }
+  const int64_t i = t / v, a = t % v;
+  const double2 E = e.energy[q];
+  const double2 f = e.fock[q * e.s_fock + (o + a) * n + i], s = e.acc[u], x = e.t1[qv + t];
+  double2 r = make_double2(f.x + s.x - (E.x * x.x - E.y * x.y), f.y + s.y - (E.x * x.y + E.y * x.x));
+  if (e.rb1) {
+    const double2 c = resp_scalar(e.re, e.rs, e.es, q), bb = e.rb1[qv + t], y = e.rt1[t];
+    r.x += bb.x - (c.x * y.x - c.y * y.y);
+    r.y += bb.y - (c.x * y.y + c.y * y.x);
+  }
+  const double D = e.eps[q * e.s_eps + i] - e.eps[q * e.s_eps + o + a];
+  e.r1[qv + t] = r;
+  e.t1_new[qv + t] = make_double2(x.x + r.x / D, x.y + r.y / D);
 }
 
-// zero the first n entries of nb vectors L apart in a and b (the CID singles block)
-__global__ __launch_bounds__(256) void sp_zero_kernel(int64_t n, int64_t nb, int64_t L, double2* __restrict__ a,
-                                                      double2* __restrict__ b) {
-  for (int64_t u = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; u < nb * n; u += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t at = (u / n) * L + u % n;
-    a[at] = make_double2(0.0, 0.0);
-    b[at] = make_double2(0.0, 0.0);
+// Both epilogues in one launch: neither reads what the other writes.
+__global__ __launch_bounds__(256) void sp_epi_kernel(SpEpi e) {
+  if ((int)blockIdx.x >= e.doubles) {
+    sp_epi_singles(e, (int64_t)((int)blockIdx.x - e.doubles) * 256 + threadIdx.x);
+    return;
   }
+  sp_epi_doubles(e);
 }
 
 constexpr int EN_BLOCKS = 256;
@@ -558,26 +557,8 @@ apy_gemm_desc gd(int64_t m, int64_t nn, int64_t k, int al, const void* a, int64_
 // Workspace regions: each holds nb instances one after another (R, Y, X1, X2, Q1, Q2: (ov)^2 each;
 // TU: 2 (ov)^2; Ts/Ps: so*sv; Ta/Pa: ao*av; acc, T1: ov), then the GEMM scratch.
 struct SpWS {
-  size_t R, Y, X1, X2, TU, Ts, Ta, Ps, Pa, Q1, Q2, acc, t1, gemm, gemm2, total;
+  size_t R, Y, X1, X2, TU, Ts, Ta, Ps, Pa, Q1, Q2, acc, t1, gemm, total;
 };
-
-// One side stream per device (default priority).  A step's products fall into two chains with no
-// data between them once TU and T+/- exist (below): the second runs on this stream, so the small
-// products of a single vector (ladders with M = o(o+1)/2 rows, rings with M = ov) fill the chip
-// together instead of one after another.
-hipStream_t sp_side_stream() {
-  static std::mutex mu;
-  static std::map<int, hipStream_t> streams;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return nullptr;
-  std::lock_guard<std::mutex> lock(mu);
-  auto it = streams.find(dev);
-  if (it != streams.end()) return it->second;
-  hipStream_t s = nullptr;
-  if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) return nullptr;
-  streams[dev] = s;
-  return s;
-}
 
 constexpr int NSPG = 14;
 
@@ -680,7 +661,7 @@ int sp_gemms(int64_t o, int64_t v, int singles, int64_t nb, int64_t L, const apy
   return q;
 }
 
-SpWS sp_carve(int64_t o, int64_t v, int singles, int64_t nb, bool multi = false) {
+SpWS sp_carve(int64_t o, int64_t v, int singles, int64_t nb, bool multi = false, bool grouped = false) {
   const size_t z = 16, ov = (size_t)(o * v), d2 = ov * ov * z, B = (size_t)nb;
   auto rnd = [](size_t b) { return (b + 255) / 256 * 256; };
   SpWS w{};
@@ -709,9 +690,18 @@ SpWS sp_carve(int64_t o, int64_t v, int singles, int64_t nb, bool multi = false)
     const int q = sp_gemms(o, v, singles, nb, (int64_t)(ov + ov * ov), nullptr, nullptr, &w, g, multi ? &S : nullptr,
                            form == 1);
     for (int k = 0; k < q; ++k) m = std::max(m, apy_zgemm_ws_bytes(&g[k]));
+    // the products in one launch, without and with F_vv folded into the ring operator
+    for (int fold = 0; grouped && fold < 2; ++fold) {
+      apy_cisd_sp_args A{};
+      apy_sp_ints I{};
+      A.ints = &I;
+      A.w21_f = fold ? (void*)256 : nullptr;
+      const int qg = sp_gemms(o, v, singles, nb, (int64_t)(ov + ov * ov), &A, (char*)256, &w, g, multi ? &S : nullptr,
+                              form == 1);
+      m = std::max(m, apy_zgemm_group_ws_bytes(g, qg));
+    }
   }
-  w.gemm2 = off + rnd(std::max(m, (size_t)EN_BLOCKS * z));   // split-K region of the side chain
-  w.total = w.gemm2 + std::max(m, (size_t)256);
+  w.total = off + rnd(std::max(m, (size_t)EN_BLOCKS * z));
   return w;
 }
 
@@ -747,52 +737,13 @@ int sp_step_impl(const apy_cisd_sp_args* A, int64_t nb, const void* resp_shift, 
   hipStream_t st = (hipStream_t)stream;
   char* base = (char*)workspace;
   const double2* t = (const double2*)A->t;
-  sp_tu_kernel<<<apy_grid1d(nb * 2 * ov * ov), 256, 0, st>>>(o, v, nb, L, t, (double2*)(base + w.TU));
+  double2* T1 = singles && !multi && nb > 1 ? (double2*)(base + w.t1) : nullptr;
+  sp_prep_kernel<<<apy_grid1d(nb * (3 * ov * ov + (T1 ? ov : 0))), 256, 0, st>>>(
+      o, v, nb, L, t, (double2*)(base + w.TU), (double2*)(base + w.Ts), (double2*)(base + w.Ta), T1);
   APY_LAUNCH_CHECK();
-  sp_pack_kernel<<<apy_grid1d(nb * ov * ov), 256, 0, st>>>(o, v, nb, L, t, (double2*)(base + w.Ts),
-                                                            (double2*)(base + w.Ta));
-  APY_LAUNCH_CHECK();
-  if (singles && !multi && nb > 1) {
-    sp_t1_stack<<<apy_grid1d(nb * ov), 256, 0, st>>>(ov, nb, L, t, (double2*)(base + w.t1));
-    APY_LAUNCH_CHECK();
-  }
   apy_gemm_desc g[NSPG];
   const int q = sp_gemms(o, v, singles, nb, L, A, base, &w, g, multi ? &S : nullptr, !multi && I->w4t);
-  // Two chains with no data between them: P+, HHL (+ Y), X1, Q1 on the caller's stream; P-, X2, Q2 and
-  // the singles accumulator products (one after another into acc) forked onto the side stream and
-  // joined before the epilogues.  Under stream capture everything stays on the caller's stream.
-  auto on_side = [&](const apy_gemm_desc& d) {
-    const char* c = (const char*)d.c;
-    return c == base + w.Pa || c == base + w.X2 || (singles && (c == base + w.Q2 || c == base + w.acc));
-  };
-  hipStream_t ss = nullptr;
-  {
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone) ss = sp_side_stream();
-  }
-  hipEvent_t evf = nullptr, evj = nullptr;
-  if (ss) {
-    if (hipEventCreateWithFlags(&evf, hipEventDisableTiming) != hipSuccess) return APY_E_HIP;
-    if (hipEventCreateWithFlags(&evj, hipEventDisableTiming) != hipSuccess) {
-      (void)hipEventDestroy(evf);
-      return APY_E_HIP;
-    }
-    APY_HIP_TRY(hipEventRecord(evf, st));
-    APY_HIP_TRY(hipStreamWaitEvent(ss, evf, 0));
-  }
-  int status = APY_OK;
-  const size_t gb = w.gemm2 - w.gemm;
-  for (int k = 0; k < q && status == APY_OK; ++k)
-    if (ss && on_side(g[k])) status = apy_zgemm_launch(&g[k], base + w.gemm2, ws_bytes - w.gemm2, ss);
-  if (ss && hipEventRecord(evj, ss) != hipSuccess && status == APY_OK) status = APY_E_HIP;
-  for (int k = 0; k < q && status == APY_OK; ++k)
-    if (!ss || !on_side(g[k])) status = apy_zgemm_launch(&g[k], base + w.gemm, gb, st);
-  if (ss) {
-    // join even after a failed launch, so no later work on the caller's stream races the side stream
-    if (hipStreamWaitEvent(st, evj, 0) != hipSuccess && status == APY_OK) status = APY_E_HIP;
-    (void)hipEventDestroy(evf);
-    (void)hipEventDestroy(evj);
-  }
+  const int status = apy_zgemm_group(g, q, base + w.gemm, ws_bytes - w.gemm, st);
   if (status != APY_OK) return status;
   const double2* rb = (const double2*)A->resp_b;
   const double2* rt = (const double2*)A->resp_t;
@@ -805,18 +756,12 @@ int sp_step_impl(const apy_cisd_sp_args* A, int64_t nb, const void* resp_shift, 
           singles ? (const double2*)(base + w.Q1) : nullptr, singles ? (const double2*)(base + w.Q2) : nullptr,
           t + ov, (const double2*)A->energy, (double2*)A->t_new + ov, (double2*)A->out + ov,
           rb ? rb + ov : nullptr, rb ? rt + ov : nullptr, re, rs, es, multi ? S.eps : 0,
-          multi ? S.blk[S_VVOO] : 0};
-  const int64_t nt = (v + SET - 1) / SET;
-  sp_epi_doubles<<<(unsigned)std::min<int64_t>(nb * o * o * nt * nt, 1 << 20), 256, 0, st>>>(e);
-  APY_LAUNCH_CHECK();
-  if (singles) {
-    sp_epi_singles<<<apy_grid1d(nb * ov), 256, 0, st>>>(o, v, nb, L, A->eps, (const double2*)A->fock,
-                                                        (const double2*)(base + w.acc), t, (const double2*)A->energy,
-                                                        (double2*)A->t_new, (double2*)A->out, rb, rt, re, rs, es,
-                                                        multi ? S.eps : 0, multi ? S.fock : 0);
-  } else {  // CID keeps the singles block of the vectors at zero
-    sp_zero_kernel<<<apy_grid1d(nb * ov), 256, 0, st>>>(ov, nb, L, (double2*)A->t_new, (double2*)A->out);
-  }
+          multi ? S.blk[S_VVOO] : 0,
+          (const double2*)A->fock, multi ? S.fock : 0, singles ? (const double2*)(base + w.acc) : nullptr, t, rb, rt,
+          (double2*)A->t_new, (double2*)A->out, 0};
+  const int64_t nt = (v + SET - 1) / SET, ns = (nb * ov + 255) / 256;
+  e.doubles = (int32_t)std::min<int64_t>(nb * o * o * nt * nt, 1 << 20);
+  sp_epi_kernel<<<(unsigned)(e.doubles + ns), 256, 0, st>>>(e);
   APY_LAUNCH_CHECK();
   return APY_OK;
 }
@@ -827,11 +772,16 @@ int sp_energy_impl(int64_t o, int64_t v, int singles, int64_t nb, const void* g,
   if (!workspace || ws_bytes < (size_t)nb * apy_cisd_sp_energy_workspace()) return APY_E_WORKSPACE;
   hipStream_t st = (hipStream_t)stream;
   const int64_t ov = o * v;
-  sp_energy_partial<<<dim3(EN_BLOCKS, (unsigned)nb), 256, 0, st>>>(ov, singles ? 1 : 0, (const double2*)g,
-                                                                    (const double2*)L, (const double2*)t,
-                                                                    ov + ov * ov, s_g, s_l, (double2*)workspace);
+  // four terms a thread; one block an instance writes the energy itself where a second launch would take
+  // longer than the terms do
+  const int64_t terms = ov + ov * ov;
+  const int np = terms <= 4096 ? 1 : (int)std::min<int64_t>(EN_BLOCKS, (terms + 1023) / 1024);
+  sp_energy_partial<<<dim3((unsigned)np, (unsigned)nb), 256, 0, st>>>(ov, singles ? 1 : 0, (const double2*)g,
+                                                                      (const double2*)L, (const double2*)t, terms, s_g,
+                                                                      s_l, (double2*)(np > 1 ? workspace : energy));
   APY_LAUNCH_CHECK();
-  sp_energy_final<<<(unsigned)nb, 256, 0, st>>>((const double2*)workspace, EN_BLOCKS, (double2*)energy);
+  if (np == 1) return APY_OK;
+  sp_energy_final<<<(unsigned)nb, 256, 0, st>>>((const double2*)workspace, np, (double2*)energy);
   APY_LAUNCH_CHECK();
   return APY_OK;
 }
@@ -899,7 +849,7 @@ int apy_cisd_sp_prepare(int64_t o, int64_t v, const void* fock, const apy_sp_int
 
 size_t apy_cisd_sp_workspace(int64_t o, int64_t v, int singles) {
   if (o < 1 || v < 1) return 0;
-  return sp_carve(o, v, singles ? 1 : 0, 1).total;
+  return sp_carve(o, v, singles ? 1 : 0, 1, false, true).total;
 }
 
 int apy_cisd_sp_step(const apy_cisd_sp_args* A, void* workspace, size_t ws_bytes, void* stream) {
@@ -908,7 +858,7 @@ int apy_cisd_sp_step(const apy_cisd_sp_args* A, void* workspace, size_t ws_bytes
 
 size_t apy_cisd_sp_batch_workspace(int64_t o, int64_t v, int singles, int64_t nb) {
   if (o < 1 || v < 1 || nb < 1) return 0;
-  return sp_carve(o, v, singles ? 1 : 0, nb).total;
+  return sp_carve(o, v, singles ? 1 : 0, nb, false, true).total;
 }
 
 int apy_cisd_sp_step_batch(const apy_cisd_sp_args* A, int64_t nb, const void* resp_shift, void* workspace,
@@ -960,7 +910,7 @@ int apy_cisd_sp_energy_multi(int64_t o, int64_t v, int singles, int64_t nb, cons
 
 size_t apy_cisd_sp_multi_workspace(int64_t o, int64_t v, int singles, int64_t nb) {
   if (o < 1 || v < 1 || nb < 1) return 0;
-  return sp_carve(o, v, singles ? 1 : 0, nb, true).total;
+  return sp_carve(o, v, singles ? 1 : 0, nb, true, true).total;
 }
 
 int apy_cisd_sp_step_multi(const apy_cisd_sp_args* A, int64_t nb, void* workspace, size_t ws_bytes, void* stream) {

@@ -52,6 +52,12 @@ inline unsigned apy_grid1d(int64_t n, int64_t cap = 65536) {
 int apy_zgemm_launch(const apy_gemm_desc* d, void* workspace, size_t ws_bytes, hipStream_t s,
                      hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
 size_t apy_zgemm_ws_bytes(const apy_gemm_desc* d);
+// The products d[0..n) in list order: large ones by themselves, the others in one launch and one
+// reduction.  None may read another's output; outputs are equal or disjoint (else, or with a smaller
+// workspace than apy_zgemm_group_ws_bytes, or with events, one launch after another).
+int apy_zgemm_group(const apy_gemm_desc* d, int n, void* workspace, size_t ws_bytes, hipStream_t s,
+                    hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
+size_t apy_zgemm_group_ws_bytes(const apy_gemm_desc* d, int n);
 // Workspace of the plan apy_zgemm_launch would run for d now (cached or model plan).
 size_t apy_zgemm_plan_ws_bytes(const apy_gemm_desc* d);
 // apy_cisd_so_step on a caller's workspace; exact = 1: the GEMM region sized

@@ -78,8 +78,11 @@ __device__ inline double2 masked(double2 v, bool in, unsigned long long sg) {
 // G3: the Gauss form of the complex product, three real products per complex multiply-add
 // (T1 = ar br, T2 = ai bi, T3 = (ar + ai)(br + bi); re = T1 - T2, im = T3 - T1 - T2): three MFMAs
 // instead of four, one more accumulator plane, the operand sums formed in registers.
+template <int BM, int BN, int BK, bool B_NK>
+constexpr int tile_lds = 2 * (BM * (BK + 1) + (B_NK ? BN * (BK + 1) : BK * BN));  // double2 of the two stages
+
 template <int BM, int BN, int WM, int WN, int BK, bool A_MK, bool B_NK, bool G3>
-__global__ __launch_bounds__(NTHR) void zgemm_mfma(GemmArgs p) {
+__device__ __forceinline__ void zgemm_tile(const GemmArgs& p, int64_t logical, double2* lds) {
   constexpr int RB = WM / 16, CB = WN / 16;
   constexpr int BKP = BK + 1;  // padded row (complex elements) of k-contiguous LDS tiles
   constexpr int A_PER = BM * BK / NTHR;
@@ -92,15 +95,14 @@ __global__ __launch_bounds__(NTHR) void zgemm_mfma(GemmArgs p) {
   // Interleaved (re, im) tiles: one 16-byte LDS read yields both planes of
   // an MFMA operand.  Row strides of BKP complex (272 B for BK=16) keep the
   // 8-lane groups of a 128-bit LDS access on distinct banks.
-  __shared__ double2 As[2][A_LDS];
-  __shared__ double2 Bs[2][B_LDS];
+  auto As = reinterpret_cast<double2 (*)[A_LDS]>(lds);
+  auto Bs = reinterpret_cast<double2 (*)[B_LDS]>(lds + 2 * A_LDS);
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
 
-  int64_t logical = xcd_remap(blockIdx.x, p.total);
   const int64_t mt = logical % p.mtiles; logical /= p.mtiles;
   const int64_t nt = logical % p.ntiles; logical /= p.ntiles;
   const int s = (int)(logical % p.split);
@@ -285,6 +287,50 @@ __global__ __launch_bounds__(NTHR) void zgemm_mfma(GemmArgs p) {
       }
 }
 
+template <int BM, int BN, int WM, int WN, int BK, bool A_MK, bool B_NK, bool G3>
+__global__ __launch_bounds__(NTHR) void zgemm_mfma(GemmArgs p) {
+  __shared__ double2 lds[tile_lds<BM, BN, BK, B_NK>];
+  zgemm_tile<BM, BN, WM, WN, BK, A_MK, B_NK, G3>(p, xcd_remap(blockIdx.x, p.total), lds);
+}
+
+// Several independent products in one launch: the blocks of each on a range of the grid that starts at a
+// multiple of 8 (so xcd_remap sees the XCD the block is on).  A CISD step is 8 to 14 products of very
+// different sizes, most of which cannot fill the chip alone: launched one after another they ran at their
+// own latency, together they share the CUs (O=10 V=4: 22 launches, 93 us a step -> 6 launches, 38 us;
+// o=9 v=25: 157 -> 62; O=18 V=50: 372 -> 279; o=10 v=80: 679 -> 575).  Two tiles, chosen per product by padding: 64 x 64 and
+// 32 x 64, both with BK = 8 (168 registers, three blocks a CU).  G3: the 64 x 64 tile in the three-product
+// form, and only for the products that ask for it.
+constexpr int GROUP_MAX = 14;
+struct GroupArgs {
+  GemmArgs g[GROUP_MAX];
+  int32_t start[GROUP_MAX];
+  int32_t kind[GROUP_MAX];   // bit 0: A_MK, bit 1: B_NK, bit 2: the 32 x 64 tile
+  int32_t n;
+};
+
+template <bool G3>
+__global__ __launch_bounds__(NTHR, G3 ? 2 : 3) void zgemm_group(GroupArgs G) {
+  constexpr int L = tile_lds<64, 64, 8, true>;
+  static_assert(L >= tile_lds<64, 64, 8, false> && L >= tile_lds<32, 64, 8, true>, "LDS of the largest tile");
+  __shared__ double2 lds[L];
+  int q = 0;
+  while (q + 1 < G.n && (int)blockIdx.x >= G.start[q + 1]) ++q;
+  const GemmArgs& p = G.g[q];
+  const int64_t bid = (int64_t)blockIdx.x - G.start[q];
+  if (bid >= p.total) return;
+  const int64_t u = xcd_remap(bid, p.total);
+  switch (G.kind[q]) {
+    case 0: zgemm_tile<64, 64, 32, 32, 8, false, false, G3>(p, u, lds); break;
+    case 1: zgemm_tile<64, 64, 32, 32, 8, true, false, G3>(p, u, lds); break;
+    case 2: zgemm_tile<64, 64, 32, 32, 8, false, true, G3>(p, u, lds); break;
+    case 3: zgemm_tile<64, 64, 32, 32, 8, true, true, G3>(p, u, lds); break;
+    case 4: zgemm_tile<32, 64, 16, 32, 8, false, false, false>(p, u, lds); break;
+    case 5: zgemm_tile<32, 64, 16, 32, 8, true, false, false>(p, u, lds); break;
+    case 6: zgemm_tile<32, 64, 16, 32, 8, false, true, false>(p, u, lds); break;
+    default: zgemm_tile<32, 64, 16, 32, 8, true, true, false>(p, u, lds); break;
+  }
+}
+
 // C_g = beta*C_g + sum over `group` consecutive partials of ws.
 __global__ __launch_bounds__(256) void zgemm_reduce(const double2* __restrict__ ws, int64_t group, int64_t ngroups,
                                                      int64_t m, int64_t n, double2* c, int64_t ldc, int64_t sc,
@@ -348,6 +394,68 @@ __global__ __launch_bounds__(RW_E * RW_R) void zgemm_reduce_wide(const double2* 
     }
     *cp = make_double2(xr, xi);
   }
+}
+
+// The partial sums of a grouped launch: target t is beta C + the parts of its contributions in list order
+// (K slices, and batch members where they are summed, of one product, then the next product into the same
+// C).  Few parts: a thread an element; many (wide): the layout of zgemm_reduce_wide.
+struct GroupRed {
+  struct { double2* c; int64_t total; double ber, bei; int32_t use_beta, first, count, wide, start; } t[GROUP_MAX];
+  struct { const double2* ws; int64_t parts, mn; } k[GROUP_MAX];   // [batch][parts][mn]
+  int32_t n;
+};
+
+__global__ __launch_bounds__(256) void zgemm_group_reduce(GroupRed R) {
+  int q = 0;
+  while (q + 1 < R.n && (int)blockIdx.x >= R.t[q + 1].start) ++q;
+  const auto& T = R.t[q];
+  const int64_t blk = (int64_t)blockIdx.x - T.start, total = T.total;
+  __shared__ double sr[RW_R][RW_E], si[RW_R][RW_E];
+  double xr = 0.0, xi = 0.0;
+  int64_t e;
+  bool own;
+  if (!T.wide) {
+    e = blk * 256 + threadIdx.x;
+    own = e < total;
+    if (own)
+      for (int u = T.first; u < T.first + T.count; ++u) {
+        const int64_t np = R.k[u].parts, mn = R.k[u].mn;
+        const double2* w = R.k[u].ws + (mn == total ? e : e / mn * np * mn + e % mn);
+        for (int64_t s = 0; s < np; ++s) { const double2 v = w[s * mn]; xr += v.x; xi += v.y; }
+      }
+  } else {
+    const int j = threadIdx.x % RW_E, r = threadIdx.x / RW_E;
+    e = blk * RW_E + j;
+    double ar[4] = {0.0, 0.0, 0.0, 0.0}, ai[4] = {0.0, 0.0, 0.0, 0.0};
+    if (e < total)
+      for (int u = T.first; u < T.first + T.count; ++u) {
+        const int64_t np = R.k[u].parts, mn = R.k[u].mn;
+        const double2* w = R.k[u].ws + (mn == total ? e : e / mn * np * mn + e % mn);
+        int64_t s = r;
+        for (; s + 3 * RW_R < np; s += 4 * RW_R) {
+          const double2 v0 = w[s * mn], v1 = w[(s + RW_R) * mn], v2 = w[(s + 2 * RW_R) * mn],
+                        v3 = w[(s + 3 * RW_R) * mn];
+          ar[0] += v0.x; ai[0] += v0.y; ar[1] += v1.x; ai[1] += v1.y;
+          ar[2] += v2.x; ai[2] += v2.y; ar[3] += v3.x; ai[3] += v3.y;
+        }
+#pragma unroll
+        for (int x = 0; x < 3; ++x, s += RW_R)
+          if (s < np) { const double2 v = w[s * mn]; ar[x] += v.x; ai[x] += v.y; }
+      }
+    sr[r][j] = (ar[0] + ar[1]) + (ar[2] + ar[3]);
+    si[r][j] = (ai[0] + ai[1]) + (ai[2] + ai[3]);
+    __syncthreads();
+    own = r == 0 && e < total;
+    if (own)
+      for (int k = 0; k < RW_R; ++k) { xr += sr[k][j]; xi += si[k][j]; }
+  }
+  if (!own) return;
+  if (T.use_beta) {
+    const double2 old = T.c[e];
+    xr += T.ber * old.x - T.bei * old.y;
+    xi += T.ber * old.y + T.bei * old.x;
+  }
+  T.c[e] = make_double2(xr, xi);
 }
 
 // ------------------------------------------------------------ tile configs
@@ -670,6 +778,211 @@ int apy_zgemm_launch(const apy_gemm_desc* d, void* workspace, size_t ws_bytes, h
     return APY_OK;
   }
   return run_plan(d, make_plan(d), workspace, ws_bytes, s, ev0, ev1);
+}
+
+// ------------------------------------------------------------ grouped products
+namespace {
+
+// A product of this size fills the chip for several rounds by itself and keeps its own (tuned) plan.
+constexpr double GROUP_ALONE_FLOP = 2.0e10;   // about 0.3 ms
+constexpr int64_t GROUP_MIN_K = 64;           // shortest K slice: eight stages against the prologue
+constexpr double GROUP_PART_BYTES = 6.4e7;    // partial sums of one product at most
+
+struct Group {
+  int n = 0;                 // products in the launch
+  int idx[GROUP_MAX];        // their descriptors, longest blocks first
+  int kind[GROUP_MAX], split[GROUP_MAX];
+  int64_t kchunk[GROUP_MAX], parts[GROUP_MAX];
+  int nt = 0;                // targets, in list order
+  int target[GROUP_MAX];     // of descriptor idx
+  bool alone[GROUP_MAX];     // by descriptor: launched by itself before the group
+  size_t off[GROUP_MAX];     // by descriptor: its partial sums in the workspace (SIZE_MAX: none)
+  size_t bytes = 0;
+};
+
+int64_t out_total(const apy_gemm_desc* d) { return d->m * d->n * (d->reduce_batch ? 1 : d->batch); }
+
+// Whether the list can run as alone products followed by one group, and how.  The outputs must be
+// contiguous and equal or disjoint; into one output the first product of the group brings its beta, the
+// later ones add (beta = 1).
+bool group_plan(const apy_gemm_desc* d, int n, Group& G) {
+  if (n < 1 || n > GROUP_MAX) return false;
+  const char *lo[GROUP_MAX], *hi[GROUP_MAX];
+  for (int i = 0; i < n; ++i) {
+    const apy_gemm_desc& x = d[i];
+    if (x.m < 1 || x.n < 1 || x.k < 1 || x.batch < 1 || x.ldc != x.n || x.split_k || x.tile) return false;
+    if (x.batch > 1 && !x.reduce_batch && x.stride_c != x.m * x.n) return false;
+    lo[i] = (const char*)x.c;
+    hi[i] = lo[i] + out_total(&x) * (int64_t)sizeof(double2);
+    G.off[i] = SIZE_MAX;
+    G.alone[i] = 8.0 * (double)x.m * x.n * x.k * x.batch > GROUP_ALONE_FLOP;
+    for (int j = 0; j < i && G.alone[i]; ++j)
+      if (!G.alone[j] && lo[j] < hi[i] && lo[i] < hi[j]) G.alone[i] = false;
+  }
+  int first[GROUP_MAX], count[GROUP_MAX], of[GROUP_MAX];
+  for (int i = 0; i < n; ++i) {
+    if (G.alone[i]) continue;
+    int t = -1;
+    for (int j = 0; j < G.nt && t < 0; ++j) {
+      const int f = first[j];
+      if (lo[f] == lo[i] && hi[f] == hi[i]) t = j;
+      else if (lo[f] < hi[i] && lo[i] < hi[f]) return false;
+    }
+    if (t < 0) {
+      t = G.nt++;
+      first[t] = i;
+      count[t] = 0;
+    } else if (d[i].beta_re != 1.0 || d[i].beta_im != 0.0) {
+      return false;
+    }
+    ++count[t];
+    of[i] = t;
+  }
+  // Tile by padding, then K slices that give every block the same work with one round of resident blocks.
+  int kind[GROUP_MAX];
+  double area[GROUP_MAX], T = 0.0;
+  for (int i = 0; i < n; ++i) {
+    if (G.alone[i]) continue;
+    const double c = (double)((d[i].n + 63) / 64) * 64;
+    const double a64 = (double)((d[i].m + 63) / 64) * 64 * c / CFGS[8].eff, a32 = (double)((d[i].m + 31) / 32) * 32 * c / CFGS[9].eff;
+    const bool small = !d[i].gauss3m && a32 < a64;
+    kind[i] = (d[i].a_layout == APY_MK ? 1 : 0) | (d[i].b_layout == APY_NK ? 2 : 0) | (small ? 4 : 0);
+    area[i] = small ? 32.0 * 64.0 : 64.0 * 64.0;
+    T += (small ? a32 : a64) * d[i].k * d[i].batch;
+  }
+  const double slots = 3.0 * dev_info().cus, per = T / slots;
+  double work[GROUP_MAX];
+  for (int i = 0; i < n; ++i) {
+    if (G.alone[i]) continue;
+    const double eff = CFGS[(kind[i] & 4) ? 9 : 8].eff;
+    const int64_t want = std::max<int64_t>(GROUP_MIN_K, (int64_t)(per * eff / area[i]));
+    const double bytes = (double)d[i].m * d[i].n * d[i].batch * sizeof(double2);
+    int64_t split = (d[i].k + want - 1) / want;
+    split = std::min<int64_t>(split, std::max<int64_t>(1, (int64_t)(GROUP_PART_BYTES / bytes)));
+    const int64_t kc = ((d[i].k + split - 1) / split + 15) / 16 * 16;
+    split = (d[i].k + kc - 1) / kc;
+    work[i] = area[i] / eff * (double)std::min(kc, d[i].k);
+    int at = G.n++;
+    while (at > 0 && work[G.idx[at - 1]] < work[i]) { G.idx[at] = G.idx[at - 1]; --at; }
+    G.idx[at] = i;
+    G.kind[i] = kind[i];
+    G.split[i] = (int)split;
+    G.kchunk[i] = kc;
+    G.parts[i] = split * (d[i].reduce_batch ? d[i].batch : 1);
+    G.target[i] = of[i];
+    if (G.parts[i] > 1 || count[of[i]] > 1) {
+      G.off[i] = G.bytes;
+      G.bytes += ((size_t)G.parts[i] * out_total(&d[i]) * sizeof(double2) + 255) & ~(size_t)255;
+    }
+  }
+  return true;
+}
+
+}  // namespace
+
+size_t apy_zgemm_group_ws_bytes(const apy_gemm_desc* d, int n) {
+  Group G;
+  if (!group_plan(d, n, G)) return 0;
+  size_t w = G.bytes;
+  for (int i = 0; i < n; ++i)
+    if (G.alone[i]) w = std::max(w, apy_zgemm_ws_bytes(&d[i]));
+  return w;
+}
+
+int apy_zgemm_group(const apy_gemm_desc* d, int n, void* workspace, size_t ws_bytes, hipStream_t s, hipEvent_t ev0,
+                    hipEvent_t ev1) {
+  Group G;
+  if (ev0 || !group_plan(d, n, G) || G.bytes > ws_bytes || (G.bytes && !workspace)) {
+    for (int i = 0; i < n; ++i) {
+      const int st = apy_zgemm_launch(&d[i], workspace, ws_bytes, s, i ? nullptr : ev0, i ? nullptr : ev1);
+      if (st != APY_OK) return st;
+    }
+    return APY_OK;
+  }
+  for (int i = 0; i < n; ++i) {
+    int st = check_desc(&d[i]);
+    if (st == APY_OK && G.alone[i]) st = apy_zgemm_launch(&d[i], workspace, ws_bytes, s);
+    if (st != APY_OK) return st;
+  }
+  if (G.n == 0) return APY_OK;
+  GroupArgs A;
+  GroupRed R;
+  A.n = G.n;
+  R.n = 0;
+  int64_t blocks = 0;
+  bool g3 = false;
+  for (int q = 0; q < G.n; ++q) {
+    const int i = G.idx[q];
+    const apy_gemm_desc& x = d[i];
+    const int bm = (G.kind[i] & 4) ? 32 : 64;
+    GemmArgs& a = A.g[q];
+    a = GemmArgs{};
+    a.m = x.m; a.n = x.n; a.k = x.k;
+    a.a = (const double2*)x.a; a.lda = x.lda; a.sa = x.stride_a;
+    a.b = (const double2*)x.b; a.ldb = x.ldb; a.sb = x.stride_b;
+    a.c = (double2*)x.c; a.ldc = x.ldc; a.sc = x.stride_c;
+    a.alr = x.alpha_re; a.ali = x.alpha_im; a.ber = x.beta_re; a.bei = x.beta_im;
+    a.conj_a = x.conj_a; a.conj_b = x.conj_b;
+    a.use_beta = (x.beta_re != 0.0 || x.beta_im != 0.0) ? 1 : 0;
+    a.batch = x.batch; a.split = G.split[i]; a.kchunk = G.kchunk[i];
+    a.mtiles = (x.m + bm - 1) / bm; a.ntiles = (x.n + 63) / 64;
+    a.total = a.mtiles * a.ntiles * a.split * a.batch;
+    a.ws = G.off[i] != SIZE_MAX ? (double2*)((char*)workspace + G.off[i]) : nullptr;
+    a.g3 = x.gauss3m ? 1 : 0;
+    g3 = g3 || x.gauss3m;
+    A.kind[q] = G.kind[i];
+    A.start[q] = (int32_t)blocks;
+    blocks += (a.total + 7) / 8 * 8;
+    if (blocks > 0x7fffffffLL) return APY_E_ARG;
+  }
+  if (g3) {
+    // the 64 x 64 tile of the G3 launch is for the products that ask for the three-product form
+    for (int q = 0; q < G.n; ++q)
+      if (!A.g[q].g3 && !(A.kind[q] & 4)) {
+        for (int i = 0; i < n; ++i) {
+          if (G.alone[i]) continue;
+          const int st = apy_zgemm_launch(&d[i], workspace, ws_bytes, s);
+          if (st != APY_OK) return st;
+        }
+        return APY_OK;
+      }
+    zgemm_group<true><<<(unsigned)blocks, NTHR, 0, s>>>(A);
+  } else {
+    zgemm_group<false><<<(unsigned)blocks, NTHR, 0, s>>>(A);
+  }
+  APY_LAUNCH_CHECK();
+  int64_t rb = 0;
+  int nk = 0;
+  for (int t = 0; t < G.nt; ++t) {
+    auto& X = R.t[R.n];
+    X.first = nk;
+    X.count = 0;
+    int64_t parts = 0;
+    for (int i = 0; i < n; ++i) {
+      if (G.alone[i] || G.target[i] != t || G.off[i] == SIZE_MAX) continue;
+      if (X.count++ == 0) {
+        X.c = (double2*)d[i].c;
+        X.total = out_total(&d[i]);
+        X.ber = d[i].beta_re;
+        X.bei = d[i].beta_im;
+        X.use_beta = (d[i].beta_re != 0.0 || d[i].beta_im != 0.0) ? 1 : 0;
+      }
+      R.k[nk].ws = (const double2*)((char*)workspace + G.off[i]);
+      R.k[nk].mn = d[i].m * d[i].n;
+      R.k[nk++].parts = G.parts[i];
+      parts += G.parts[i];
+    }
+    if (X.count == 0) continue;
+    X.wide = parts >= 2 * RW_R && X.total <= (1 << 18);
+    X.start = (int32_t)rb;
+    rb += X.wide ? (X.total + RW_E - 1) / RW_E : (X.total + 255) / 256;
+    if (rb > 0x7fffffffLL) return APY_E_ARG;
+    ++R.n;
+  }
+  if (R.n == 0) return APY_OK;
+  zgemm_group_reduce<<<(unsigned)rb, 256, 0, s>>>(R);
+  APY_LAUNCH_CHECK();
+  return APY_OK;
 }
 
 int apy_zgemm_tune_impl(const apy_gemm_desc* d, void* workspace, size_t ws_bytes, int reps, hipStream_t s,

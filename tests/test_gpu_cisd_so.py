@@ -50,6 +50,89 @@ def test_blocks_from_mo_spin_expansion(dev, m, Osp):
     assert np.array_equal(f_so, transforms.compute_F_SO_loop(f_mo))
 
 
+@pytest.mark.parametrize("m,Osp", [(2, 1), (33, 3), (40, 7), (70, 4), (36, 70)])
+def test_blocks_from_mo_at_tile_edges(dev, m, Osp):
+    """The spin-expanded blocks of apy_so_ints_from_mo against those of apy_so_ints_from_full (the general
+    element-wise path) on the expanded tensor: virtual spaces below, at and past one and two 32-wide spatial
+    tiles, an odd number of occupied spin orbitals, more than 32 occupied spatial orbitals.  Copies and
+    single differences: equal."""
+    n = 2 * m
+    g = torch.Generator(device=dev).manual_seed(m)
+    E = torch.randn((m,) * 4, dtype=torch.complex128, device=dev, generator=g)
+    if n > 80:                       # the expanded tensor of 80 spin orbitals is 0.7 GB: larger ones by blocks
+        names = ("ring", "vovv_p", "vvvo_p")
+        got = SOIntegrals.from_mo(E, Osp, blocks=names)
+        V = n - Osp
+        o, v = torch.arange(Osp, device=dev), Osp + torch.arange(V, device=dev)
+        a, b = torch.triu_indices(V, V, 1, device=dev) + Osp
+
+        def anti(p, q, r, s):
+            z = torch.zeros((), dtype=torch.complex128, device=dev)
+            d = torch.where(((p ^ r) & 1 == 0) & ((q ^ s) & 1 == 0), E[p >> 1, r >> 1, q >> 1, s >> 1], z)
+            return d - torch.where(((p ^ s) & 1 == 0) & ((q ^ r) & 1 == 0), E[p >> 1, s >> 1, q >> 1, r >> 1], z)
+
+        ring = torch.stack([anti(o[None, :, None], v[:, None, None], v[None, None, :], j) for j in o])
+        assert torch.equal(got["ring"], ring.reshape(-1))
+        vovv = got["vovv_p"].view(V, Osp, -1)
+        vvvo = got["vvvo_p"].view(-1, Osp, V)
+        for k in range(0, V, 7):
+            assert torch.equal(vovv[k], anti(v[k], o[:, None], a[None], b[None]))
+        for k in range(0, a.numel(), 997):
+            assert torch.equal(vvvo[k], anti(a[k], b[k], v[None], o[:, None]))
+        return
+    p = torch.arange(n, device=dev)
+    same = (p[:, None] & 1) == (p[None, :] & 1)
+    h = p >> 1
+    D = E[h][:, h][:, :, h][:, :, :, h] * (same[:, :, None, None] & same[None, None])     # (pr|qs) spin-expanded
+    A = D.permute(0, 2, 1, 3) - D.permute(0, 2, 3, 1)                                     # <pq||rs>
+    got, want = SOIntegrals.from_mo(E, Osp), SOIntegrals.from_full(A, Osp)
+    for name in want.blocks:
+        assert torch.equal(got[name], want[name]), name
+
+
+@pytest.mark.parametrize("O,V", [(2, 2), (3, 5), (5, 33), (10, 4), (9, 64), (13, 41)])
+@pytest.mark.parametrize("singles,fov,fold,packed", [(True, False, True, False), (True, True, True, True),
+                                                     (True, True, False, False), (False, False, True, False)])
+def test_grouped_products_match_one_after_another(dev, O, V, singles, fov, fold, packed):
+    """A step's products in one launch (the workspace the library asks for) against the same products one
+    launch after another (the smaller workspace the step still takes, found by bisection): two orders of
+    sums of up to O V^2 terms of order one."""
+    import ctypes
+    from apyib_amd import _lib
+    lib = _lib.load()
+    F, eps = synthetic.fock(O, V, 3)
+    ints = SOIntegrals.synthetic(O, V, 3, device=dev)
+    ci = SOCI(ints, _dev(F, dev), eps, singles=singles, fov_coupling=fov, fold_fvv=fold)
+    g = torch.Generator(device=dev).manual_seed(O * V)
+    t = torch.randn(ci.Lp if packed else ci.L, dtype=torch.complex128, device=dev, generator=g) * 0.1
+    mode = _lib.APY_MODE_SIGMA if packed or fov else _lib.APY_MODE_RESIDUAL
+
+    def run(nbytes):
+        out, tn = torch.full_like(t, 7.0), torch.full_like(t, 7.0)
+        a = _lib.CisdSoArgs(O, V, ci.fock.data_ptr(), ci.eps.data_ptr(), ctypes.pointer(ints.struct), ci.hoo.data_ptr(),
+                            int(singles), int(mode), int(fov), ci.energy_dev.data_ptr(), 1.0, 0.0, t.data_ptr(),
+                            tn.data_ptr(), out.data_ptr(), None, None, None,
+                            ci.ring_f.data_ptr() if fold else None, int(packed), 0)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        rc = lib.apy_cisd_so_step(ctypes.byref(a), ctypes.c_void_p(ws.data_ptr()), nbytes,
+                                  ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        return rc, out, tn
+
+    full = ci.ws_bytes
+    rc, out, tn = run(full)
+    assert rc == 0
+    lo, hi = 0, full                 # run(lo) refused, run(hi) accepted
+    while hi - lo > 256:
+        mid = (lo + hi) // 2
+        lo, hi = (lo, mid) if run(mid)[0] == 0 else (mid, hi)
+    rc, out1, tn1 = run(hi)
+    assert rc == 0
+    live = slice(None) if singles else slice(ci.OV, None)
+    for x, y in ((out, out1), (tn, tn1)):
+        assert (x[live] - y[live]).abs().max() <= 1e-13 * max(1.0, y[live].abs().max().item())
+
+
 def _system(O, V, seed, dev, brill=False):
     F, A, eps = synthetic.system(O, V, seed)
     if brill:
