@@ -163,6 +163,109 @@ __global__ __launch_bounds__(256) void build_block(Src src, int kind, int64_t O,
   }
 }
 
+// The four large blocks of <pq||rs> from spatial MO integrals.  For one spatial pair (P, Q) the block's
+// rows are the matrix M[x][y] = (Px|Qy) = E[P][x][Q][y] and its transpose:
+//   <pq||rs> = d(p,r) d(q,s) M[R][S] - d(p,s) d(q,r) M[S][R]   (spins; capitals: p/2).
+// One workgroup takes a pair (P, Q) and a 32 x 32 tile of (R, S): it reads the tile of M and the mirrored
+// one along their rows into LDS and writes the rows of the up to four spin pairs along the output's
+// contiguous index.  build_block read M[S][R] one element a cache line (stride m^2) and decoded four
+// orbitals an element: m = 60, O = 20 (57e6 elements, 0.92 GB) 560 us in all, bound by those reads; this
+// is bound by its writes.
+//   KIND            p       q      columns                    output index
+//   K_VVVV_P        a    <  b      r = c < s = d              [(ab)][(cd)]
+//   K_VOVV          a       j      r = c < s = b              [a][j][(cb)]
+//   K_VVVO_P        a    <  b      r = c, s = j               [(ab)][j][c]
+//   K_RING          k       b      r = c, s = j               [(j,b)][(k,c)]
+constexpr int BT = 32;   // spatial tile edge
+
+template <int KIND>
+__global__ __launch_bounds__(256) void build_pair_rows(const double2* __restrict__ E, int64_t m, int64_t O, int64_t V,
+                                                       int64_t nq, int64_t nts, double2* __restrict__ out) {
+  constexpr bool TRI = KIND == K_VVVV_P || KIND == K_VOVV;      // columns r < s, both virtual
+  constexpr bool PAIR = KIND == K_VVVV_P || KIND == K_VVVO_P;   // rows a < b
+  __shared__ double2 A[BT][BT + 1], B[BT][BT + 1];              // M[R][S] and M[S][R] of the tile
+  const int64_t n = O + V, v0 = O >> 1;                          // first virtual spatial orbital (O odd: shared)
+  const int64_t Pv = npair(V), OV = O * V;
+  int64_t w = blockIdx.x;
+  int64_t tr, ts;
+  if (TRI) {                                                     // tile pairs tr <= ts
+    int64_t t = w % (nts * (nts + 1) / 2);
+    w /= nts * (nts + 1) / 2;
+    tr = 0;
+    while (t >= nts - tr) { t -= nts - tr; ++tr; }
+    ts = tr + t;
+  } else {
+    const int64_t ntv = ((n - 1) / 2 - v0) / BT + 1;
+    tr = w % ntv; w /= ntv;
+    ts = w % nts; w /= nts;
+  }
+  int64_t P, Q;
+  if (PAIR) {                                                    // P <= Q of nq virtual ones
+    const double b = 2.0 * (double)nq + 1.0;
+    P = (int64_t)((b - sqrt(b * b - 8.0 * (double)w)) * 0.5);
+    while (P > 0 && P * (2 * nq - P + 1) / 2 > w) --P;
+    while ((P + 1) * (2 * nq - P) / 2 <= w) ++P;
+    Q = v0 + P + w - P * (2 * nq - P + 1) / 2;
+    P += v0;
+  } else if (KIND == K_VOVV) {
+    P = v0 + w / nq; Q = w % nq;
+  } else {
+    P = w / nq; Q = v0 + w % nq;
+  }
+  const int64_t R0 = v0 + tr * BT, S0 = (TRI ? v0 : 0) + ts * BT;
+  const int64_t Rn = n / 2 + (n & 1), Sn = TRI ? Rn : (O + 1) / 2;   // ends of the spatial ranges
+  const double2* M = E + (P * m * m + Q) * m;                        // M[x][y] = M[x m^2 + y]
+  for (int e = threadIdx.x; e < BT * BT; e += 256) {
+    const int64_t x = e / BT, y = e % BT;
+    if (R0 + x < Rn && S0 + y < Sn) A[x][y] = M[(R0 + x) * m * m + S0 + y];
+    if (S0 + x < Sn && R0 + y < Rn) B[x][y] = M[(S0 + x) * m * m + R0 + y];
+  }
+  __syncthreads();
+  // the contiguous index of the output runs over the lanes: s for the packed columns, else r
+  const int lane = threadIdx.x & 63, grp = threadIdx.x >> 6;
+  for (int pq = 0; pq < 4; ++pq) {
+    const int64_t p = 2 * P + (pq >> 1), q = 2 * Q + (pq & 1);
+    int64_t base;
+    if (PAIR) {
+      if (p < O || q < O || p >= n || q >= n || p >= q) continue;
+      base = (prow(p - O, V) + q - p - 1) * (KIND == K_VVVV_P ? Pv : OV);
+    } else if (KIND == K_VOVV) {
+      if (p < O || p >= n || q >= O) continue;
+      base = ((p - O) * O + q) * Pv;
+    } else {
+      if (p >= O || q < O || q >= n) continue;
+      base = (q - O) * OV + p * V;
+    }
+    for (int k = grp; k < 2 * BT; k += 4) {
+      const int x = TRI ? k : lane, y = TRI ? lane : k;              // spin offsets of r and s in the tile
+      const int64_t r = 2 * R0 + x, s = 2 * S0 + y;
+      if (r < O || r >= n || (TRI ? s <= r || s >= n : s >= O)) continue;
+      double2 v = make_double2(0.0, 0.0);
+      if (((p ^ r) & 1) == 0 && ((q ^ s) & 1) == 0) v = A[x >> 1][y >> 1];
+      if (((p ^ s) & 1) == 0 && ((q ^ r) & 1) == 0) {
+        const double2 u = B[y >> 1][x >> 1];
+        v.x -= u.x;
+        v.y -= u.y;
+      }
+      const int64_t o = TRI ? prow(r - O, V) + s - r - 1 : KIND == K_VVVO_P ? s * V + r - O : s * V * OV + r - O;
+      out[base + o] = v;
+    }
+  }
+}
+
+template <int KIND>
+int launch_pair_rows(const double2* E, int64_t m, int64_t O, int64_t V, void* out, hipStream_t st) {
+  if (!out || kind_size(KIND, O, V) <= 0) return APY_OK;
+  constexpr bool TRI = KIND == K_VVVV_P || KIND == K_VOVV, PAIR = KIND == K_VVVV_P || KIND == K_VVVO_P;
+  const int64_t nv = m - O / 2, no = (O + 1) / 2, ntv = (nv + BT - 1) / BT, nto = (no + BT - 1) / BT;
+  const int64_t nq = PAIR ? nv : KIND == K_VOVV ? no : nv;
+  const int64_t pairs = PAIR ? nv * (nv + 1) / 2 : nv * no, tiles = TRI ? ntv * (ntv + 1) / 2 : ntv * nto;
+  if (pairs * tiles > 0x7fffffffLL) return APY_E_ARG;
+  build_pair_rows<KIND><<<(unsigned)(pairs * tiles), 256, 0, st>>>(E, m, O, V, nq, TRI ? ntv : nto, (double2*)out);
+  APY_LAUNCH_CHECK();
+  return APY_OK;
+}
+
 void* block_ptr(const apy_so_ints* I, int kind) {
   switch (kind) {
     case K_VVVV_P: return I->vvvv_p;
@@ -179,9 +282,11 @@ void* block_ptr(const apy_so_ints* I, int kind) {
 }
 
 template <class Src>
-int build_all(const Src& src, const apy_so_ints* I, int accumulate, double scale, hipStream_t st) {
+int build_all(const Src& src, const apy_so_ints* I, int accumulate, double scale, hipStream_t st,
+              unsigned skip = 0) {
   if (!I || I->O < 0 || I->V < 0) return APY_E_ARG;
   for (int kind = 0; kind < K_COUNT; ++kind) {
+    if (skip >> kind & 1) continue;
     double2* out = (double2*)block_ptr(I, kind);
     if (!out) continue;
     int64_t total = kind_size(kind, I->O, I->V);
@@ -899,8 +1004,17 @@ int apy_so_ints_from_full(int64_t n, const void* A, const apy_so_ints* ints, voi
 
 int apy_so_ints_from_mo(int64_t m, const void* eri_mo, const apy_so_ints* ints, void* stream) {
   if (!eri_mo || !ints || ints->O + ints->V != 2 * m) return APY_E_ARG;
-  SrcMO src{(const double2*)eri_mo, m};
-  return build_all(src, ints, 0, 0.0, (hipStream_t)stream);
+  const double2* E = (const double2*)eri_mo;
+  const int64_t O = ints->O, V = ints->V;
+  hipStream_t st = (hipStream_t)stream;
+  if (O < 0 || V < 0) return APY_E_ARG;
+  int s = launch_pair_rows<K_VVVV_P>(E, m, O, V, ints->vvvv_p, st);
+  if (s == APY_OK) s = launch_pair_rows<K_VVVO_P>(E, m, O, V, ints->vvvo_p, st);
+  if (s == APY_OK) s = launch_pair_rows<K_VOVV>(E, m, O, V, ints->vovv_p, st);
+  if (s == APY_OK) s = launch_pair_rows<K_RING>(E, m, O, V, ints->ring, st);
+  if (s != APY_OK) return s;
+  SrcMO src{E, m};
+  return build_all(src, ints, 0, 0.0, st, 1u << K_VVVV_P | 1u << K_VVVO_P | 1u << K_VOVV | 1u << K_RING);
 }
 
 int apy_synth_so_ints(uint64_t seed, uint64_t tag, double sd, int accumulate, double scale, int real_only,
