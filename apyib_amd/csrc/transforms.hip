@@ -11,6 +11,8 @@
 // the AO integrals with the density, one block per output element pair.
 #include "common.h"
 
+#include <algorithm>
+
 namespace {
 
 // F[m,n] = h[m,n] + sum_{l,s} D[l,s] (2 (mn|ls) - (ml|ns))  (times `scale`
@@ -81,6 +83,130 @@ __global__ __launch_bounds__(256) void eri_so_kernel(int64_t m, const double2* _
   }
 }
 
+// One quarter transform with the coefficient matrix resident in LDS, for small dimensions up to 96:
+//   ROWS:  Y[x][p] = sum_k X[x][k] op(C)[k][p]            (x: `total` rows ldx apart, k contiguous)
+//   else:  Y[b][p][s] = sum_k op(C)[k][p] X[b][k][s]      (columns (b, s), N to a batch member: `total` of them)
+// A wave takes 16 rows or columns of the streamed operand (a column's batch member is found per lane, so
+// short batch members leave no lane idle) and all p: the streamed elements go from memory into the MFMA
+// lanes directly, four k steps ahead, C comes from LDS as the other operand, and no barrier follows the
+// first.  As tiles of the general GEMM the K of one AO dimension is five stages: their prologue and the
+// padding to 32 or 64 held nbf = 90 at 41 TFLOP/s (4.45 ms the four), nbf = 34 at 16.
+// MFMA f64 16x16x4 lanes: A[l%16][l/16], B[l/16][l%16], D[l/16 + 4r][l%16].
+constexpr int QT = 512;        // eight waves share one C
+constexpr int QS = 4;          // k steps (of 4) in flight
+
+template <int NB, bool ROWS>
+__global__ __launch_bounds__(QT, 2) void quarter_kernel(int K, int M, const double2* __restrict__ C, int64_t ldc,
+                                                        int conj, const double2* __restrict__ X, int64_t total,
+                                                        int64_t N, int64_t sx, int64_t ldx, double2* __restrict__ Y,
+                                                        int64_t sy, int64_t ldy) {
+  extern __shared__ double2 Cs[];                     // [K rounded up to 4][16 NB]
+  constexpr int LD = 16 * NB;
+  const int Kp = (K + 3) & ~3;
+  for (int e = threadIdx.x; e < Kp * LD; e += QT) {
+    const int k = e / LD, p = e % LD;
+    double2 v = make_double2(0.0, 0.0);
+    if (k < K && p < M) v = C[k * ldc + p];
+    if (conj) v.y = -v.y;
+    Cs[e] = v;
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & 63, lo = lane & 15, hi = lane >> 4;
+  const int64_t ntask = (total + 15) / 16, nw = (int64_t)gridDim.x * (QT / 64);
+  for (int64_t task = (int64_t)blockIdx.x * (QT / 64) + (threadIdx.x >> 6); task < ntask; task += nw) {
+    const int64_t c = min(task * 16 + lo, total - 1);
+    const int64_t b = ROWS ? 0 : c / N, col = ROWS ? 0 : c - b * N;
+    const double2* x = ROWS ? X + c * ldx : X + b * sx + col;
+    auto load = [&](int k) {                          // past K: the last element, masked to zero
+      const int kk = min(k + hi, K - 1);
+      double2 v = x[ROWS ? (int64_t)kk : kk * ldx];
+      if (k + hi >= K) v = make_double2(0.0, 0.0);
+      return v;
+    };
+    v4d re[NB], im[NB];
+#pragma unroll
+    for (int p = 0; p < NB; ++p) { re[p] = (v4d){0, 0, 0, 0}; im[p] = (v4d){0, 0, 0, 0}; }
+    double2 cur[QS], nxt[QS];
+#pragma unroll
+    for (int u = 0; u < QS; ++u) cur[u] = load(4 * u);
+    for (int k0 = 0; k0 < Kp; k0 += 4 * QS) {
+#pragma unroll
+      for (int u = 0; u < QS; ++u) nxt[u] = load(k0 + 4 * (QS + u));
+#pragma unroll
+      for (int u = 0; u < QS; ++u) {
+        if (k0 + 4 * u >= Kp) break;
+        const double2 xv = cur[u];
+        const double2* cr = Cs + (k0 + 4 * u + hi) * LD + lo;
+#pragma unroll
+        for (int p = 0; p < NB; ++p) {
+          const double2 cv = cr[16 * p];
+          if (ROWS) {
+            re[p] = __builtin_amdgcn_mfma_f64_16x16x4f64(xv.x, cv.x, re[p], 0, 0, 0);
+            im[p] = __builtin_amdgcn_mfma_f64_16x16x4f64(xv.x, cv.y, im[p], 0, 0, 0);
+            re[p] = __builtin_amdgcn_mfma_f64_16x16x4f64(-xv.y, cv.y, re[p], 0, 0, 0);
+            im[p] = __builtin_amdgcn_mfma_f64_16x16x4f64(xv.y, cv.x, im[p], 0, 0, 0);
+          } else {
+            re[p] = __builtin_amdgcn_mfma_f64_16x16x4f64(cv.x, xv.x, re[p], 0, 0, 0);
+            im[p] = __builtin_amdgcn_mfma_f64_16x16x4f64(cv.x, xv.y, im[p], 0, 0, 0);
+            re[p] = __builtin_amdgcn_mfma_f64_16x16x4f64(-cv.y, xv.y, re[p], 0, 0, 0);
+            im[p] = __builtin_amdgcn_mfma_f64_16x16x4f64(cv.y, xv.x, im[p], 0, 0, 0);
+          }
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < QS; ++u) cur[u] = nxt[u];
+    }
+#pragma unroll
+    for (int p = 0; p < NB; ++p)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const double2 v = make_double2(re[p][r], im[p][r]);
+        if (ROWS) {
+          const int64_t row = task * 16 + hi + 4 * r;
+          if (row < total && 16 * p + lo < M) Y[row * ldy + 16 * p + lo] = v;
+        } else {
+          const int q = 16 * p + hi + 4 * r;
+          if (task * 16 + lo < total && q < M) Y[b * sy + q * ldy + col] = v;
+        }
+      }
+  }
+}
+
+constexpr size_t QLDS = 150 * 1024;   // of a CU's 160 KB
+
+size_t quarter_lds(int64_t K, int64_t M) { return (size_t)((K + 3) / 4 * 4) * ((M + 15) / 16 * 16) * sizeof(double2); }
+
+// The resident form: C within LDS and at most six 16-wide blocks of accumulators (96: 96 registers each
+// of re and im with the next k steps in flight).  Larger ones take the general GEMM, whose K is long enough.
+bool quarter_fits(int64_t nbf, int64_t nact) { return nact <= 96 && quarter_lds(nbf, nact) <= QLDS; }
+
+template <int NB, bool ROWS>
+int quarter_nb(int K, int M, const double2* C, int64_t ldc, int conj, const double2* X, int64_t total, int64_t N,
+               int64_t sx, int64_t ldx, double2* Y, int64_t sy, int64_t ldy, hipStream_t st) {
+  const size_t lds = quarter_lds(K, M);
+  if (lds > 64 * 1024)
+    APY_HIP_TRY(hipFuncSetAttribute((const void*)quarter_kernel<NB, ROWS>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)QLDS));
+  const int64_t need = ((total + 15) / 16 + QT / 64 - 1) / (QT / 64);
+  const int64_t fit = std::max<int64_t>(1, std::min<int64_t>(NB <= 2 ? 4 : 2, (int64_t)(160 * 1024 / lds)));
+  quarter_kernel<NB, ROWS><<<(unsigned)std::min<int64_t>(need, 256 * fit), QT, lds, st>>>(K, M, C, ldc, conj, X, total,
+                                                                                        N, sx, ldx, Y, sy, ldy);
+  APY_LAUNCH_CHECK();
+  return APY_OK;
+}
+
+template <bool ROWS, class... T>
+int quarter(int K, int M, T... a) {
+  switch ((M + 15) / 16) {
+    case 1: return quarter_nb<1, ROWS>(K, M, a...);
+    case 2: return quarter_nb<2, ROWS>(K, M, a...);
+    case 3: return quarter_nb<3, ROWS>(K, M, a...);
+    case 4: return quarter_nb<4, ROWS>(K, M, a...);
+    case 5: return quarter_nb<5, ROWS>(K, M, a...);
+    default: return quarter_nb<6, ROWS>(K, M, a...);
+  }
+}
+
 apy_gemm_desc gd(int64_t m, int64_t n, int64_t k, int al, const void* a, int64_t lda, int bl, const void* b,
                  int64_t ldb, void* c, int64_t ldc) {
   apy_gemm_desc d{};
@@ -144,6 +270,21 @@ int apy_eri_mo(int64_t nbf, int64_t nact, const void* eri_ao, const void* C, voi
   void* x1 = w;
   void* x2 = w + al256(P0.x_bytes);
   void* gw = w + 2 * al256(P0.x_bytes);
+  if (quarter_fits(nbf, nact)) {
+    const int K = (int)nbf, M = (int)nact;
+    const int64_t n = nbf, a = nact;
+    const double2 *c = (const double2*)C, *E = (const double2*)eri_ao;
+    double2 *X1 = (double2*)x1, *X2 = (double2*)x2, *out = (double2*)eri_mo;
+    hipStream_t st = (hipStream_t)stream;
+    int s = quarter<true>(K, M, c, a, 0, E, n * n * n, (int64_t)1, (int64_t)0, n, X1, (int64_t)0, a, st);
+    if (s == APY_OK) s = quarter<false>(K, M, c, a, 1, (const double2*)X1, n * n * a, a, n * a, a, X2, a * a, a, st);
+    if (s == APY_OK)
+      s = quarter<false>(K, M, c, a, 0, (const double2*)X2, n * a * a, a * a, n * a * a, a * a, X1, a * a * a, a * a, st);
+    if (s == APY_OK)
+      s = quarter<false>(K, M, c, a, 1, (const double2*)X1, a * a * a, a * a * a, (int64_t)0, a * a * a, out, (int64_t)0,
+                         a * a * a, st);
+    return s;
+  }
   EriPlan P = eri_plan(nbf, nact, eri_ao, C, x1, x2, eri_mo);
   for (int q = 0; q < 4; ++q) {
     int s = apy_zgemm_launch(&P.g[q], gw, P0.gemm_bytes, (hipStream_t)stream);
