@@ -16,16 +16,15 @@
 // formed only for i<j, a<b.
 //
 // Two kernels per step cover every instance.  nc_z_kernel forms
-// Z_ij[(ab)] = sum_m Foo(m,j) x_im[(ab)] for all ordered pairs (i,j): a
-// workgroup takes one (instance, i, slice of the (a<b) pairs), holds the O
-// amplitudes x_im of each element in registers (read once, coalesced) and
-// writes Z_ij for every j.  ncp_step_kernel then gives a workgroup one
-// (instance, pair i<j, 32 x 32 tile pair A <= B of the virtual plane): it
+// W_ij[(ab)] = -Z_ij + Z_ji, Z_ij = sum_m Foo(m,j) x_im, for the pairs i<j: a
+// workgroup takes one (instance, slab of the (a<b) pairs) with a thread to each
+// (i, pair) and joins the two orders in LDS.  ncp_step_kernel then gives a
+// workgroup one (instance, pair i<j, tile pair A <= B of the virtual plane): it
 // forms Y_ij[a,b] - Y_ij[b,a] over the tile on the FP64 matrix cores with
 // K = e staged in 8-wide chunks through LDS (the tile's rows of x_ij expanded
 // from the packed row with the antisymmetry signs, and the matching columns
-// of Fvv), adds the driver and -Z_ij + Z_ji (two coalesced reads), applies the
-// update and writes its partial residual norm; per_instance_sum reduces
+// of Fvv), adds the driver and W, applies the update and writes its partial
+// residual norm; per_instance_sum reduces
 // those per instance in a fixed order.  All tables live in the workspace, written once
 // by apy_mp2_nc_batched_setup, so a sequence of steps can be captured in a
 // HIP graph.
@@ -52,16 +51,24 @@ struct Item {
   int32_t inst, pij, ta, tb;
 };
 
-constexpr int ZS = 2 * BLK;  // (a<b) elements per Z work item
-constexpr int ZMAX_O = 32;   // largest O of the matrix-core Z path (two 16-row j blocks, Foo in LDS)
+// The slab of W that a work item forms in LDS: SP pairs (ab) by all (i<j), at most one thread an (i, ab);
+// 0: it does not fit (O > 66), BLK pairs (ab) an item then.
+constexpr int SLAB = 2192;
+__host__ __device__ inline int slab_of(int64_t O) {
+  const int64_t po = O * (O - 1) / 2;
+  if (O < 2 || po > SLAB) return 0;
+  const int64_t a = BLK / (O < BLK ? O : BLK), b = SLAB / po;
+  return (int)(a < b ? a : b);
+}
+inline int64_t zspan(int64_t O) { return slab_of(O) ? slab_of(O) : BLK; }
 
 struct ZItem {
-  int32_t inst, i, p0, pad;
+  int32_t inst, p0;
 };
 
 struct Header {
   int64_t n, items, zitems;
-  int64_t zitem_off, z_off;   // byte offsets of the Z work items and of the Z blocks
+  int64_t zitem_off, z_off;   // byte offsets of the W work items and of the W blocks
 };
 
 inline size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
@@ -86,8 +93,8 @@ __device__ inline void pdec(int64_t P, int64_t N, int64_t& p, int64_t& q) {
 // Workspace: header, instance table, item table, per-instance item offsets,
 // item partial norms, energy partial sums, per-instance offsets of the Z
 // blocks, then (at byte offsets the header holds, so the step needs only
-// (n, items) on the host) the Z work items and the Z blocks themselves
-// (sum_k O_k^2 Pv_k complex).
+// (n, items) on the host) the W work items and the W blocks themselves
+// (sum_k Po_k Pv_k complex).
 struct WsLayout {
   size_t inst, item, off, part, epart, zoff, zitem, z, total;
 };
@@ -111,8 +118,8 @@ int64_t count_zitems(int n, const apy_mp2_nc_instance* inst, int64_t* zelems) {
   for (int k = 0; k < n; ++k) {
     if (inst[k].O < 2 || inst[k].V < 2) continue;
     const int64_t Pv = npair(inst[k].V);
-    z += inst[k].O * ((Pv + ZS - 1) / ZS);
-    e += inst[k].O * inst[k].O * Pv;
+    z += (Pv + zspan(inst[k].O) - 1) / zspan(inst[k].O);
+    e += npair(inst[k].O) * Pv;
   }
   if (zelems) *zelems = e;
   return z;
@@ -135,131 +142,191 @@ __device__ inline void cfma(double2& acc, double2 a, double2 b) {
   acc.y = fma(a.y, b.x, acc.y);
 }
 
-// x_(pq)[c, d] of the packed amplitudes for any p != q, c != d (zero otherwise)
-__device__ inline double2 xget(const double2* x, int64_t O, int64_t Pv, int64_t V, int64_t p, int64_t q, int64_t c,
-                               int64_t d) {
-  if (p == q || c == d) return make_double2(0.0, 0.0);
-  const double2 v = x[pidx(p < q ? p : q, p < q ? q : p, O) * Pv + pidx(c < d ? c : d, c < d ? d : c, V)];
-  return ((p < q) == (c < d)) ? v : make_double2(-v.x, -v.y);
-}
+// F read through the scalar cache: every address is uniform over the workgroup and no kernel of a step
+// writes F.
+typedef const __attribute__((address_space(4))) double* SF;
 
-// Z of one work item on the FP64 matrix cores: Z_ij[P] = sum_m Foo(m,j) x_im[P] as 16 x 16 blocks
-// D[j][P] = sum_m A[j][m] B[m][P] with A = Foo^T (from LDS) and B the rows x_im (read along P, 16
-// consecutive P per 16 lanes); each wave takes ZS / 64 blocks of 16 P, every j block (O <= 32) and
-// K = m in steps of 4.  MFMA f64 16x16x4 lanes: A[l%16][l/16], B[l/16][l%16], D[l/16 + 4r][l%16].
-__device__ __forceinline__ void z_item_mfma(const double2* __restrict__ fo, const double2* __restrict__ x,
-                                            double2* Z, int O, int64_t Pv, int i, int64_t p0) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int nj = (O + 15) / 16, nk = (O + 3) / 4;
-  for (int pb = wave; pb < ZS / 16; pb += BLK / 64) {
-    const int64_t P = p0 + 16 * pb + (lane & 15);
-    v4d re[2], im[2];
+// Z_ij[P] = sum_m Foo(m,j) x_im[P] of one (i, P) a thread, JB values of j from j0: x_im from memory, Foo in
+// scalar registers, JB complex sums in vector registers.  The vector units do FP64 at the matrix units'
+// rate, and this form has no padding: 16 x 16 x 4 blocks spent 2 x 5 of them on the 18 x 18 product of
+// O = 18.
+template <int JB, bool TF>
+__device__ __forceinline__ void z_rows(SF Fr, const double2* __restrict__ x, int O, int n, int64_t Pv, int i, int j0,
+                                       int64_t P, double2 (&acc)[JB]) {
 #pragma unroll
-    for (int jb = 0; jb < 2; ++jb) { re[jb] = (v4d){0, 0, 0, 0}; im[jb] = (v4d){0, 0, 0, 0}; }
-    double2 bvs[ZMAX_O / 4];                            // B[m][P] = x_im[P] for every k step, loaded up front
+  for (int j = 0; j < JB; ++j) acc[j] = make_double2(0.0, 0.0);
+  int off[JB];                                         // past the end: a sum that is not taken
 #pragma unroll
-    for (int kb = 0; kb < ZMAX_O / 4; ++kb) {
-      const int m = 4 * kb + (lane >> 4);
-      double2 bv = make_double2(0.0, 0.0);
-      if (kb < nk && m < O && m != i && P < Pv) {
-        bv = x[pidx(i < m ? i : m, i < m ? m : i, O) * Pv + P];
-        if (m < i) bv = make_double2(-bv.x, -bv.y);
-      }
-      bvs[kb] = bv;
-    }
+  for (int j = 0; j < JB; ++j) off[j] = 2 * min(j0 + j, O - 1) * n;
+  const int ri = (int)prow(i, O) - i - 1;              // pair (i, m), m > i: ri + m; (m, i): prow(m) + i - m - 1
+  auto load = [&](int m) {
+    const int mm = min(m, O - 1), r = mm > i ? ri + mm : mm < i ? (int)prow(mm, O) + i - mm - 1 : 0;
+    return x[(int64_t)r * Pv + P];
+  };
+  // two x_im ahead: an L2 read takes as long as the sums of two m over the waves of a SIMD
+  double2 cur[2] = {load(0), load(1)}, nxt[2];
+  for (int m0 = 0; m0 < O; m0 += 2) {
+    nxt[0] = load(m0 + 2);
+    nxt[1] = load(m0 + 3);
 #pragma unroll
-    for (int kb = 0; kb < ZMAX_O / 4; ++kb) {
-      if (kb >= nk) break;
-      const int m = 4 * kb + (lane >> 4);
-      const double2 bv = bvs[kb];
+    for (int u = 0; u < 2; ++u) {
+      const int m = m0 + u;
+      if (m >= O) break;
+      double2 v = cur[u];
+      v.x = m == i ? 0.0 : m < i ? -v.x : v.x;
+      v.y = m == i ? 0.0 : m < i ? -v.y : v.y;
+      // row m of F_oo from j0 (F^T: its column): the non-transposed row is read on past O, still inside F
+      // (m <= O - 1, V >= 2), so that its loads are of four elements each
+      const SF Fm = Fr + 2 * (TF ? m : m * n + j0);
 #pragma unroll
-      for (int jb = 0; jb < 2; ++jb) {
-        if (jb >= nj) break;
-        const int j = 16 * jb + (lane & 15);
-        const double2 av = (m < O && j < O) ? fo[m * O + j] : make_double2(0.0, 0.0);   // A[j][m] = Foo(m, j)
-        re[jb] = __builtin_amdgcn_mfma_f64_16x16x4f64(av.x, bv.x, re[jb], 0, 0, 0);
-        im[jb] = __builtin_amdgcn_mfma_f64_16x16x4f64(av.x, bv.y, im[jb], 0, 0, 0);
-        re[jb] = __builtin_amdgcn_mfma_f64_16x16x4f64(-av.y, bv.y, re[jb], 0, 0, 0);
-        im[jb] = __builtin_amdgcn_mfma_f64_16x16x4f64(av.y, bv.x, im[jb], 0, 0, 0);
-      }
-    }
-    if (P < Pv) {
-#pragma unroll
-      for (int jb = 0; jb < 2; ++jb) {
-        if (jb >= nj) break;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int j = 16 * jb + (lane >> 4) + 4 * r;
-          if (j < O) Z[j * Pv + P] = make_double2(re[jb][r], im[jb][r]);
-        }
+      for (int j = 0; j < JB; ++j) {
+        const int o = TF ? off[j] : 2 * j;
+        const double fr = Fm[o], fi = Fm[o + 1];
+        acc[j].x = fma(fr, v.x, acc[j].x);
+        acc[j].x = fma(-fi, v.y, acc[j].x);
+        acc[j].y = fma(fr, v.y, acc[j].y);
+        acc[j].y = fma(fi, v.x, acc[j].y);
       }
     }
+    cur[0] = nxt[0];
+    cur[1] = nxt[1];
   }
 }
 
-// Z_k[i][j][(ab)] = sum_m Foo(m,j) x_im[(ab)] for every instance, row i and slice of
-// ZS pairs (ab) (grid-stride over the Z work list, whose length is in the header).
+// W_(i<j)[P] = -Z_ij[P] + Z_ji[P] for the SP pairs (ab) from p0: thread (i, P) forms Z_ij for all j and
+// stores the j > i of them to the slab in LDS, then, after a barrier, adds its j < i to the rows that
+// thread (j, P) stored; rows past the first pass of threads find every smaller row stored.  With more than
+// one block of j (O > JB) both are additions to zeros.  The slab leaves LDS along P.  Kept as one array: as
+// Z_ij and Z_ji of every ordered pair this kernel's writes and the step's reads were twice as long.
+template <int JB, bool TF>
+__device__ __forceinline__ void w_slab(SF Fr, const double2* __restrict__ x, double2* __restrict__ W, double2* slab,
+                                       int O, int n, int64_t Pv, int64_t p0, int SP) {
+  const int tid = threadIdx.x, rows = BLK / SP, pl = tid % SP, il = tid / SP, Po = (int)npair(O);
+  const int64_t P = min(p0 + pl, Pv - 1);
+  const bool multi = O > JB;
+  if (multi) {
+    for (int e = tid; e < Po * SP; e += blockDim.x) slab[e] = make_double2(0.0, 0.0);
+    __syncthreads();
+  }
+  for (int i0 = 0; i0 < O; i0 += rows) {
+    const int i = i0 + il;
+    const bool own = il < rows && i < O;
+    for (int j0 = 0; j0 < O; j0 += JB) {
+      double2 acc[JB];
+      if (own) {
+        z_rows<JB, TF>(Fr, x, O, n, Pv, i, j0, P, acc);
+#pragma unroll
+        for (int j = 0; j < JB; ++j)
+          if (j0 + j > i && j0 + j < O) {
+            double2& w = slab[(int)pidx(i, j0 + j, O) * SP + pl];
+            w = multi ? make_double2(w.x - acc[j].x, w.y - acc[j].y) : make_double2(-acc[j].x, -acc[j].y);
+          }
+      }
+      __syncthreads();
+      if (own) {
+#pragma unroll
+        for (int j = 0; j < JB; ++j)
+          if (j0 + j < i) {
+            double2& w = slab[(int)pidx(j0 + j, i, O) * SP + pl];
+            w.x += acc[j].x;
+            w.y += acc[j].y;
+          }
+      }
+      if (multi) __syncthreads();
+    }
+  }
+  __syncthreads();
+  const int np = (int)min((int64_t)SP, Pv - p0);
+  for (int e = tid; e < Po * SP; e += blockDim.x) {
+    const int r = e / SP, c = e % SP;
+    if (c < np) W[r * Pv + p0 + c] = slab[e];
+  }
+}
+
+// W_k[(i<j)][(ab)] = sum_m (Foo(m,i) x_jm - Foo(m,j) x_im)[(ab)] for every instance and slice of pairs
+// (ab) (grid-stride over the work list, whose length is in the header).
 __device__ __forceinline__ void nc_z_phase(char* __restrict__ ws, const apy_mp2_nc_instance* __restrict__ insts,
-                                           const int64_t* __restrict__ zoff, int reverse) {
-  __shared__ double2 fo[ZMAX_O * ZMAX_O];
+                                           const int64_t* __restrict__ zoff, int reverse, double2* slab) {
   const Header* hdr = (const Header*)ws;
   const int64_t nz = hdr->zitems;
   const ZItem* zitems = (const ZItem*)(ws + hdr->zitem_off);
   double2* zbase = (double2*)(ws + hdr->z_off);
   for (int64_t w = blockIdx.x; w < nz; w += gridDim.x) {
     const ZItem it = zitems[w];
-    const apy_mp2_nc_instance I = insts[it.inst];
-    const int64_t O = I.O, V = I.V, n = O + V, Pv = npair(V), i = it.i;
-    const int transpose_f = I.transpose_f;
-    const double2* F = (const double2*)I.fock;
+    const int inst = __builtin_amdgcn_readfirstlane(it.inst);
+    const apy_mp2_nc_instance& I = insts[inst];
+    const int O = __builtin_amdgcn_readfirstlane((int)I.O), n = O + __builtin_amdgcn_readfirstlane((int)I.V);
+    const int64_t Pv = npair(I.V);
     const double2* x = (const double2*)(reverse ? I.x_new : I.x);
-    double2* Z = zbase + zoff[it.inst] + i * O * Pv;
-    auto foo = [&](int64_t m, int64_t j) { return transpose_f ? F[j * n + m] : F[m * n + j]; };
-    if (O <= ZMAX_O) {
-      __syncthreads();                                   // fo of the previous item is no longer read
-      for (int64_t q = threadIdx.x; q < O * O; q += BLK) fo[q] = foo(q / O, q % O);   // fo[m O + j]
-      __syncthreads();
-      z_item_mfma(fo, x, Z, (int)O, Pv, (int)i, it.p0);
-    } else {
-      for (int q = 0; q < ZS / BLK; ++q) {
-        const int64_t P = it.p0 + threadIdx.x + (int64_t)BLK * q;
-        if (P >= Pv) continue;
-        for (int64_t j = 0; j < O; ++j) {
-          double2 z = make_double2(0.0, 0.0);
-          for (int64_t m = 0; m < O; ++m) {
-            if (m == i) continue;
-            double2 v = x[pidx(i < m ? i : m, i < m ? m : i, O) * Pv + P];
-            if (m < i) v = make_double2(-v.x, -v.y);
-            cfma(z, foo(m, j), v);
+    double2* W = zbase + zoff[inst];
+    // the pointer of F in scalar registers
+    const uint64_t fp = (uint64_t)I.fock;
+    const SF Fr = (SF)((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)fp) |
+                       (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(fp >> 32)) << 32);
+    const int SP = slab_of(O);
+    if (SP == 0) {                                     // more pairs (ij) than LDS holds: an element a thread
+      const double2* F = (const double2*)I.fock;
+      auto foo = [&](int m, int j) { return I.transpose_f ? F[(int64_t)j * n + m] : F[(int64_t)m * n + j]; };
+      const int64_t P = it.p0 + threadIdx.x;
+      if (threadIdx.x >= BLK || P >= Pv) continue;
+      for (int64_t r = 0; r < npair(O); ++r) {
+        int64_t i, j;
+        pdec(r, O, i, j);
+        double2 z = make_double2(0.0, 0.0);
+        for (int m = 0; m < O; ++m) {
+          if (m != i) {
+            const double2 v = x[pidx(i < m ? i : m, i < m ? m : i, O) * Pv + P];
+            cfma(z, foo(m, (int)j), i < m ? make_double2(-v.x, -v.y) : v);
           }
-          Z[j * Pv + P] = z;
+          if (m != j) {
+            const double2 v = x[pidx(j < m ? j : m, j < m ? m : j, O) * Pv + P];
+            cfma(z, foo(m, (int)i), j < m ? v : make_double2(-v.x, -v.y));
+          }
         }
+        W[r * Pv + P] = z;
       }
+      continue;
     }
+    __syncthreads();                                   // the slab of the previous item is written out
+    // the smallest block of j that covers O in as few passes as blocks of 20 do
+    const int jb = (O + (O + 19) / 20 - 1) / ((O + 19) / 20);
+    auto run = [&](auto c) {
+      constexpr int JB = decltype(c)::value;
+      if (I.transpose_f) w_slab<JB, true>(Fr, x, W, slab, O, n, Pv, it.p0, SP);
+      else w_slab<JB, false>(Fr, x, W, slab, O, n, Pv, it.p0, SP);
+    };
+    if (jb <= 8) run(std::integral_constant<int, 8>{});
+    else if (jb <= 12) run(std::integral_constant<int, 12>{});
+    else if (jb <= 16) run(std::integral_constant<int, 16>{});
+    else if (jb <= 18) run(std::integral_constant<int, 18>{});
+    else run(std::integral_constant<int, 20>{});
   }
 }
 
-__global__ __launch_bounds__(BLK) void nc_z_kernel(char* __restrict__ ws, const apy_mp2_nc_instance* __restrict__ insts,
+__global__ __launch_bounds__(BLK, 4) void nc_z_kernel(char* __restrict__ ws, const apy_mp2_nc_instance* __restrict__ insts,
                                                    const int64_t* __restrict__ zoff, int reverse) {
-  nc_z_phase(ws, insts, zoff, reverse);
+  __shared__ double2 slab[SLAB];
+  nc_z_phase(ws, insts, zoff, reverse, slab);
 }
 
 // One work item per workgroup of four waves: a 32 x 32 tile of the residual, each wave a 16 x 16
-// quarter of it on the FP64 matrix cores.  Off the diagonal (A < B) both products go into one
-// complex accumulator,
+// quarter of it on the FP64 matrix cores.  (64-wide tiles stage half the elements a product, but their
+// fewer waves left the reads of the epilogue exposed: a step of the 36-instance set 421 us with four waves
+// of 32 x 32, 330 us with eight of 32 x 16, against 322 us for 32-wide tiles.)  Off the diagonal (A < B) both products go into
+// one complex accumulator,
 //   r[a][b] += sum_e XA[a][e] GB[e][b] - sum_e GA[e][a] XB[b][e],
-// as eight v_mfma_f64_16x16x4f64 per four values of e (real and imaginary planes; the second
+// as eight v_mfma_f64_16x16x4f64 per block and four values of e (real and imaginary planes; the second
 // product with its A operand negated).  On a diagonal tile pair (A == B) the two products are one
 // matrix and its transpose, so each wave forms only Y = XA GA over its quarter (four MFMAs per
-// four e) and r = Y - Y^T is assembled through LDS.  MFMA f64 16x16x4 lanes: A[l%16][l/16],
-// B[l/16][l%16], D[l/16 + 4r][l%16].
+// four e) and r = Y - Y^T is assembled through LDS.  Quarters past V are skipped.
+// MFMA f64 16x16x4 lanes: A[l%16][l/16], B[l/16][l%16], D[l/16 + 4r][l%16].
+constexpr int STEP_LDS = 2 * MT * (MKC + 1) + 2 * MKC * (MT + 1) > MT * (MT + 1) ? 2 * MT * (MKC + 1) + 2 * MKC * (MT + 1)
+                                                                               : MT * (MT + 1);   // double2
+
 __device__ __forceinline__ void ncp_step_item(int64_t b, const apy_mp2_nc_instance* __restrict__ insts,
                                               const Item* __restrict__ items, int reverse,
                                               const char* __restrict__ ws, const int64_t* __restrict__ zoff,
-                                              double* __restrict__ part) {
-  constexpr int TILE_ELEMS = 2 * MT * (MKC + 1) + 2 * MKC * (MT + 1);
-  constexpr int SH_ELEMS = TILE_ELEMS > MT * (MT + 1) ? TILE_ELEMS : MT * (MT + 1);
-  __shared__ double2 sh[SH_ELEMS];
+                                              double* __restrict__ part, double2* sh) {
   __shared__ double red[SBLK];
   auto XA = reinterpret_cast<double2 (*)[MKC + 1]>(sh);
   auto XB = reinterpret_cast<double2 (*)[MKC + 1]>(sh + MT * (MKC + 1));
@@ -269,19 +336,17 @@ __device__ __forceinline__ void ncp_step_item(int64_t b, const apy_mp2_nc_instan
   __syncthreads();                                   // LDS of the previous item is no longer read
   const Item it = items[b];
   const apy_mp2_nc_instance I = insts[it.inst];
-  const int64_t O = I.O, V = I.V, n = O + V, Pv = npair(V);
+  const int O = (int)I.O, V = (int)I.V, n = O + V;
+  const int64_t Pv = npair(V);
   const int transpose_f = I.transpose_f;
   const double s = I.drv_scale;
   const int tid = threadIdx.x, lane = tid & 63, wm = (tid >> 6) & 1, wn = tid >> 7;
   int64_t i, j;
   pdec(it.pij, O, i, j);
   const double2* F = (const double2*)I.fock;
-  const double2* x = (const double2*)(reverse ? I.x_new : I.x);
-  double2* xn = (double2*)(reverse ? I.x : I.x_new);
-  const double2* row = x + (int64_t)it.pij * Pv;
-  const int64_t a0 = (int64_t)it.ta * MT, b0 = (int64_t)it.tb * MT;
-  // Fvv(b, e) (F^T: F[O+e][O+b])
-  auto fvv = [&](int64_t b, int64_t e) { return transpose_f ? F[(O + e) * n + O + b] : F[(O + b) * n + O + e]; };
+  const double2* row = (const double2*)(reverse ? I.x_new : I.x) + (int64_t)it.pij * Pv;
+  double2* xn = (double2*)(reverse ? I.x : I.x_new) + (int64_t)it.pij * Pv;
+  const int a0 = it.ta * MT, b0 = it.tb * MT;
 
   v4d acc_re = (v4d){0, 0, 0, 0}, acc_im = (v4d){0, 0, 0, 0};
   // diagonal tile pair (A == B): XB = XA and GB = GA, so every wave forms only Y = x Fvv^T over its
@@ -290,61 +355,75 @@ __device__ __forceinline__ void ncp_step_item(int64_t b, const apy_mp2_nc_instan
   // one e chunk of x_ij rows a0.., b0.. and of Fvv columns, fetched into registers while the previous
   // chunk is multiplied (NQ elements of each of the four tiles per thread), then stored to LDS
   constexpr int NQ = MT * MKC / SBLK;
-  const int Vi = (int)V;
-  const uint32_t V2 = 2u * (uint32_t)Vi;
+  const int am = a0 + wm * 16, bn = b0 + wn * 16;            // the wave's first row and column
+  const bool works = am < V && bn < V;
   // x_ij[p][e] is row[pidx(p, e)] above the diagonal (contiguous along e) and -row[pidx(e, p)] below it
   // (contiguous along p): each tile element is fetched by one of two passes, the upper one with e fastest
-  // across the threads and the lower one with p fastest, so that both read along the packed row.
+  // across the threads and the lower one with p fastest, so that both read along the packed row.  A pass
+  // that has no element in the chunk is left out; the addresses step with the chunk.
   double2 sxa_u[NQ], sxa_l[NQ], sxb_u[NQ], sxb_l[NQ], sga[NQ], sgb[NQ];
-  auto upper = [&](int p, int e) -> double2 {        // p <= e or out of range (zero there)
-    if (p >= Vi || e >= Vi || p >= e) return make_double2(0.0, 0.0);
-    return row[(uint32_t)p * (V2 - (uint32_t)p - 1u) / 2u + (uint32_t)(e - p - 1)];
-  };
-  auto lower = [&](int p, int e) -> double2 {        // p > e in range
-    if (p >= Vi || e >= Vi || p <= e) return make_double2(0.0, 0.0);
-    const double2 v = row[(uint32_t)e * (V2 - (uint32_t)e - 1u) / 2u + (uint32_t)(p - e - 1)];
-    return make_double2(-v.x, -v.y);
-  };
+  int up[NQ];                                          // offset of the upper row (tile A)
+  int64_t ga[NQ];                                      // of Fvv(a0 + cc, rr)
+#pragma unroll
+  for (int k = 0; k < NQ; ++k) {
+    const int q = tid + SBLK * k, p = a0 + q / MKC;
+    up[k] = p * (2 * V - p - 1) / 2 - p - 1 + q % MKC;
+    // GA[rr][cc] = Fvv(a0+cc, e0+rr), Fvv(b, e) = F[O+b][O+e] (F^T: F[O+e][O+b]), read along the contiguous
+    // index of F (e, or b for F^T)
+    const int rr = transpose_f ? q / MT : q % MKC, cc = transpose_f ? q % MT : q / MKC;
+    ga[k] = transpose_f ? (int64_t)(O + rr) * n + O + a0 + cc : (int64_t)(O + a0 + cc) * n + O + rr;
+  }
+  const int64_t ga_step = transpose_f ? n : 1, gb_off = (int64_t)(b0 - a0) * (transpose_f ? 1 : n);
   auto fetch = [&](int e0) {
+    const bool ua = e0 + MKC - 1 > a0, la = a0 + MT - 1 > e0;
+    const bool ub = e0 + MKC - 1 > b0, lb = b0 + MT - 1 > e0;
 #pragma unroll
     for (int k = 0; k < NQ; ++k) {
       const int q = tid + SBLK * k;
-      const int r = q / MKC, c = q % MKC;            // upper pass: XA[r][c] = x_ij[a0+r, e0+c], c fastest
-      sxa_u[k] = upper((int)a0 + r, e0 + c);
-      const int rl = q % MT, cl = q / MT;            // lower pass: r fastest
-      sxa_l[k] = lower((int)a0 + rl, e0 + cl);
-      // GA[rr][cc] = Fvv(a0+cc, e0+rr), read along the contiguous index of F (e, or b for F^T)
-      const int rr = transpose_f ? q / MT : q % MKC, cc = transpose_f ? q % MT : q / MKC;
-      const int e2 = e0 + rr, ca = (int)a0 + cc, cb = (int)b0 + cc;
-      sga[k] = (e2 < Vi && ca < Vi) ? fvv(ca, e2) : make_double2(0.0, 0.0);
+      const int r = q / MKC, e = e0 + q % MKC;       // upper pass: XA[r][c] = x_ij[a0+r, e0+c], c fastest
+      const int rl = q % MT, el = e0 + q / MT;       // lower pass: r fastest
+      const int lrow = el * (2 * V - el - 1) / 2 - el - 1;
+      sxa_u[k] = make_double2(0.0, 0.0);
+      sxa_l[k] = make_double2(0.0, 0.0);
+      if (ua && a0 + r < e && e < V) sxa_u[k] = row[up[k] + e0];
+      if (la && a0 + rl > el && a0 + rl < V) sxa_l[k] = row[lrow + a0 + rl];
+      const int e2 = e0 + (transpose_f ? q / MT : q % MKC), cc = transpose_f ? q % MT : q / MKC;
+      const int64_t go = ga[k] + e0 * ga_step;
+      sga[k] = make_double2(0.0, 0.0);
+      if (e2 < V && a0 + cc < V) sga[k] = F[go];
       if (!diag) {
-        sxb_u[k] = upper((int)b0 + r, e0 + c);
-        sxb_l[k] = lower((int)b0 + rl, e0 + cl);
-        sgb[k] = (e2 < Vi && cb < Vi) ? fvv(cb, e2) : make_double2(0.0, 0.0);
+        const int pb = b0 + r;
+        sxb_u[k] = make_double2(0.0, 0.0);
+        sxb_l[k] = make_double2(0.0, 0.0);
+        if (ub && pb < e && e < V) sxb_u[k] = row[pb * (2 * V - pb - 1) / 2 + e - pb - 1];
+        if (lb && b0 + rl > el && b0 + rl < V) sxb_l[k] = row[lrow + b0 + rl];
+        sgb[k] = make_double2(0.0, 0.0);
+        if (e2 < V && b0 + cc < V) sgb[k] = F[go + gb_off];
       }
     }
   };
   fetch(0);
-  for (int e0 = 0; e0 < Vi; e0 += MKC) {
+  for (int e0 = 0; e0 < V; e0 += MKC) {
     __syncthreads();                                 // the previous chunk is no longer read
 #pragma unroll
     for (int k = 0; k < NQ; ++k) {
       const int q = tid + SBLK * k;
       const int r = q / MKC, c = q % MKC, rl = q % MT, cl = q / MT;
-      const int pa = (int)a0 + r, pb = (int)b0 + r, e = e0 + c, el = e0 + cl;
+      const int e = e0 + c, el = e0 + cl;
       // each element is stored once: by the lower pass where p > e is in range, else by the upper pass
-      if (!(pa > e && pa < Vi && e < Vi)) XA[r][c] = sxa_u[k];
-      if ((int)a0 + rl > el && (int)a0 + rl < Vi && el < Vi) XA[rl][cl] = sxa_l[k];
+      if (!(a0 + r > e && a0 + r < V)) XA[r][c] = sxa_u[k];
+      if (a0 + rl > el && a0 + rl < V) XA[rl][cl] = make_double2(-sxa_l[k].x, -sxa_l[k].y);
       const int rr = transpose_f ? q / MT : q % MKC, cc = transpose_f ? q % MT : q / MKC;
       GA[rr][cc] = sga[k];
       if (!diag) {
-        if (!(pb > e && pb < Vi && e < Vi)) XB[r][c] = sxb_u[k];
-        if ((int)b0 + rl > el && (int)b0 + rl < Vi && el < Vi) XB[rl][cl] = sxb_l[k];
+        if (!(b0 + r > e && b0 + r < V)) XB[r][c] = sxb_u[k];
+        if (b0 + rl > el && b0 + rl < V) XB[rl][cl] = make_double2(-sxb_l[k].x, -sxb_l[k].y);
         GB[rr][cc] = sgb[k];
       }
     }
     __syncthreads();
-    if (e0 + MKC < Vi) fetch(e0 + MKC);              // in flight during the products below
+    if (e0 + MKC < V) fetch(e0 + MKC);               // in flight during the products below
+    if (!works) continue;                            // nothing of this wave's quarter is in range
 #pragma unroll
     for (int ks = 0; ks < MKC / 4; ++ks) {
       const int kk = ks * 4 + (lane >> 4), ra = wm * 16 + (lane & 15), cb = wn * 16 + (lane & 15);
@@ -354,13 +433,33 @@ __device__ __forceinline__ void ncp_step_item(int64_t b, const apy_mp2_nc_instan
       acc_re = __builtin_amdgcn_mfma_f64_16x16x4f64(-xa.y, gb.y, acc_re, 0, 0, 0);
       acc_im = __builtin_amdgcn_mfma_f64_16x16x4f64(xa.y, gb.x, acc_im, 0, 0, 0);
       if (!diag) {
-        const double2 ga = GA[kk][ra], xb = XB[cb][kk];   // - sum_e Fvv(a,e) x[b,e]
-        acc_re = __builtin_amdgcn_mfma_f64_16x16x4f64(-ga.x, xb.x, acc_re, 0, 0, 0);
-        acc_im = __builtin_amdgcn_mfma_f64_16x16x4f64(-ga.x, xb.y, acc_im, 0, 0, 0);
-        acc_re = __builtin_amdgcn_mfma_f64_16x16x4f64(ga.y, xb.y, acc_re, 0, 0, 0);
-        acc_im = __builtin_amdgcn_mfma_f64_16x16x4f64(-ga.y, xb.x, acc_im, 0, 0, 0);
+        const double2 ga2 = GA[kk][ra], xb = XB[cb][kk];   // - sum_e Fvv(a,e) x[b,e]
+        acc_re = __builtin_amdgcn_mfma_f64_16x16x4f64(-ga2.x, xb.x, acc_re, 0, 0, 0);
+        acc_im = __builtin_amdgcn_mfma_f64_16x16x4f64(-ga2.x, xb.y, acc_im, 0, 0, 0);
+        acc_re = __builtin_amdgcn_mfma_f64_16x16x4f64(ga2.y, xb.y, acc_re, 0, 0, 0);
+        acc_im = __builtin_amdgcn_mfma_f64_16x16x4f64(-ga2.y, xb.x, acc_im, 0, 0, 0);
       }
     }
+  }
+  // the epilogue's reads, in flight while a diagonal tile is transposed
+  const double* eps = (const double*)I.eps;
+  const double2* drv = (const double2*)I.drv + (i * O + j) * (int64_t)V * V;
+  // -sum_m Foo(m,j) x_im + sum_m Foo(m,i) x_jm
+  const double2* Wp = (const double2*)(ws + ((const Header*)ws)->z_off) + zoff[it.inst] + (int64_t)it.pij * Pv;
+  const double eij = eps[i] + eps[j];
+  const int bb = bn + (lane & 15);
+  double2 dv[4], wv[4], xv[4];
+  double ea[4];
+  const double ebb = eps[O + min(bb, V - 1)];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {                      // past the end or below the diagonal: pair (0, 1)
+    const int a = am + (lane >> 4) + 4 * r;
+    const bool in = bb < V && a < bb;
+    const int pa = in ? a : 0, pb = in ? bb : 1, Pab = pa * (2 * V - pa - 1) / 2 + pb - pa - 1;
+    dv[r] = drv[pa * V + pb];
+    wv[r] = Wp[Pab];
+    xv[r] = row[Pab];
+    ea[r] = eps[O + pa];
   }
   if (diag) {
     // every wave holds Y over its quarter of the tile (the lower-left one too): r = Y[a][b] - Y[b][a]
@@ -376,26 +475,16 @@ __device__ __forceinline__ void ncp_step_item(int64_t b, const apy_mp2_nc_instan
       acc_im[r] -= yt.y;
     }
   }
-
-  const double* eps = (const double*)I.eps;
-  const double2* drv = (const double2*)I.drv;
-  const double2* Z = (const double2*)(ws + ((const Header*)ws)->z_off) + zoff[it.inst];
-  const double eij = eps[i] + eps[j];
   double acc = 0.0;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-      const int64_t a = a0 + wm * 16 + (lane >> 4) + 4 * r, b = b0 + wn * 16 + (lane & 15);
-      if (b >= V || a >= b) continue;
-      const int64_t Pab = pidx(a, b, V);
-      const double2 d = drv[((i * O + j) * V + a) * V + b];
-      // -Z_ij + Z_ji: -sum_m Foo(m,j) x_im[a,b] + sum_m Foo(m,i) x_jm[a,b]
-      const double2 zij = Z[(i * O + j) * Pv + Pab], zji = Z[(j * O + i) * Pv + Pab];
-      const double2 rr = make_double2(s * d.x + acc_re[r] - zij.x + zji.x, s * d.y + acc_im[r] - zij.y + zji.y);
-      const double D = eij - eps[O + a] - eps[O + b];
-      const double2 xv = row[Pab];
-      xn[(int64_t)it.pij * Pv + Pab] = make_double2(xv.x + rr.x / D, xv.y + rr.y / D);
-      acc += rr.x * rr.x + rr.y * rr.y;
-    }
+    const int a = am + (lane >> 4) + 4 * r;
+    if (bb >= V || a >= bb) continue;
+    const double2 rr = make_double2(s * dv[r].x + acc_re[r] + wv[r].x, s * dv[r].y + acc_im[r] + wv[r].y);
+    const double D = eij - ea[r] - ebb;
+    xn[a * (2 * V - a - 1) / 2 + bb - a - 1] = make_double2(xv[r].x + rr.x / D, xv[r].y + rr.y / D);
+    acc += rr.x * rr.x + rr.y * rr.y;
+  }
   red[tid] = acc;
   __syncthreads();
   for (int w = SBLK / 2; w > 0; w >>= 1) {
@@ -409,17 +498,21 @@ __global__ __launch_bounds__(SBLK) void ncp_step_kernel(const apy_mp2_nc_instanc
                                                         const Item* __restrict__ items, int reverse,
                                                         const char* __restrict__ ws, const int64_t* __restrict__ zoff,
                                                         double* __restrict__ part) {
-  ncp_step_item(blockIdx.x, insts, items, reverse, ws, zoff, part);
+  __shared__ double2 sh[STEP_LDS];
+  ncp_step_item(blockIdx.x, insts, items, reverse, ws, zoff, part, sh);
 }
 
+// Called by all of a workgroup of at least BLK threads; the first BLK sum.
 __device__ __forceinline__ void instance_sum(int64_t k, const int64_t* __restrict__ off,
                                              const double* __restrict__ part, double* __restrict__ out) {
   __shared__ double red[BLK];
   __syncthreads();
   const int64_t b = off[k], e = off[k + 1];
-  double acc = 0.0;
-  for (int64_t q = b + threadIdx.x; q < e; q += BLK) acc += part[q];
-  red[threadIdx.x] = acc;
+  if (threadIdx.x < BLK) {
+    double acc = 0.0;
+    for (int64_t q = b + threadIdx.x; q < e; q += BLK) acc += part[q];
+    red[threadIdx.x] = acc;
+  }
   __syncthreads();
   for (int w = BLK / 2; w > 0; w >>= 1) {
     if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
@@ -433,7 +526,7 @@ __global__ __launch_bounds__(BLK) void per_instance_sum(const int64_t* __restric
   instance_sum(blockIdx.x, off, part, out);
 }
 
-// The whole solve in one cooperative launch: every resident workgroup loops over the Z work items,
+// The whole solve in one cooperative launch: every resident workgroup loops over the W work items,
 // the step items and the per-instance sums of an iteration with a grid barrier after each phase, then
 // reads the n residual norms and stops when sqrt(max) < tol (the test of MP2NCBatch.solve after every
 // step) or after maxit steps.  Each phase is the same per-item code as the three kernels of
@@ -448,11 +541,12 @@ __global__ __launch_bounds__(SBLK) void nc_persistent_kernel(char* __restrict__ 
                                                              int n, int64_t n_items, double tol, int maxit,
                                                              int64_t* __restrict__ iters) {
   cooperative_groups::grid_group grid = cooperative_groups::this_grid();
+  __shared__ double2 sh[SLAB > STEP_LDS ? SLAB : STEP_LDS];
   int rev = 0, it = 0;
   while (it < maxit) {
-    nc_z_phase(ws, insts, zoff, rev);
+    nc_z_phase(ws, insts, zoff, rev, sh);
     grid.sync();
-    for (int64_t b = blockIdx.x; b < n_items; b += gridDim.x) ncp_step_item(b, insts, items, rev, ws, zoff, part);
+    for (int64_t b = blockIdx.x; b < n_items; b += gridDim.x) ncp_step_item(b, insts, items, rev, ws, zoff, part, sh);
     grid.sync();
     for (int64_t k = blockIdx.x; k < n; k += gridDim.x) instance_sum(k, off, part, rnorm);
     grid.sync();
@@ -475,23 +569,41 @@ __global__ __launch_bounds__(SBLK) void nc_persistent_kernel(char* __restrict__ 
   if (blockIdx.x == 0 && threadIdx.x == 0) *iters = it;
 }
 
+// p < q of the packed pair P of N: a float root, off by one at most at these sizes, and a correction.
+__device__ inline void pdec_near(int64_t P, int N, int& p, int& q) {
+  const float b = 2.0f * (float)N - 1.0f;
+  const int64_t d = (int64_t)(2 * N - 1) * (2 * N - 1) - 8 * P;
+  int pp = min(max((int)((b - sqrtf((float)(d > 0 ? d : 0))) * 0.5f), 0), N - 2);
+  while (pp > 0 && prow(pp, N) > P) --pp;
+  while (pp < N - 2 && prow(pp + 1, N) <= P) ++pp;
+  p = pp;
+  q = (int)(P - prow(pp, N)) + pp + 1;
+}
+
 // energy[k] = scale * sum_dense w_k x_k = 4 scale * sum_(i<j, a<b) w_k x_k (w and x
 // antisymmetric), in two fixed-order passes: EN_B partial sums per instance
-// (blockIdx.y = instance), then one block per instance adds its partials.
+// (blockIdx.y = instance; a block takes every EN_B-th row (i<j), so a division and a double root an
+// element, 90 us for 36 instances of O 14-18 V 54-66, are one float root), then one block per instance
+// adds its partials.
 __global__ __launch_bounds__(BLK) void nc_energy_partial(const apy_mp2_nc_instance* __restrict__ insts, int use_x_new,
                                                          double2* __restrict__ epart) {
   __shared__ double2 red[BLK];
   const apy_mp2_nc_instance I = insts[blockIdx.y];
   const double2* w = (const double2*)I.w;
   const double2* x = (const double2*)(use_x_new ? I.x_new : I.x);
-  const int64_t O = I.O, V = I.V, Pv = npair(V), N = npair(O) * Pv;
+  const int64_t O = I.O, V = I.V, Pv = npair(V), Po = npair(O);
   double2 acc = make_double2(0.0, 0.0);
   if (w)
-    for (int64_t e = blockIdx.x * (int64_t)BLK + threadIdx.x; e < N; e += (int64_t)EN_B * BLK) {
-      int64_t i, j, a, b;
-      pdec(e / Pv, O, i, j);
-      pdec(e % Pv, V, a, b);
-      cfma(acc, w[((i * O + j) * V + a) * V + b], x[e]);
+    for (int64_t r = blockIdx.x; r < Po; r += EN_B) {
+      int64_t i, j;
+      pdec(r, O, i, j);
+      const double2* wr = w + (i * O + j) * V * V;
+      const double2* xr = x + r * Pv;
+      for (int64_t P = threadIdx.x; P < Pv; P += BLK) {
+        int a, b;
+        pdec_near(P, (int)V, a, b);
+        cfma(acc, wr[a * V + b], xr[P]);
+      }
     }
   red[threadIdx.x] = acc;
   __syncthreads();
@@ -531,16 +643,57 @@ __global__ __launch_bounds__(BLK) void t2_pack_kernel(int64_t O, int64_t V, cons
   }
 }
 
-__global__ __launch_bounds__(BLK) void t2_unpack_kernel(int64_t O, int64_t V, const double2* __restrict__ packed,
+// One workgroup per (pair i<j or diagonal i, 32 x 32 tile pair A <= B of the virtual plane): the packed
+// tile is read once and its four images written along b, the transposed two through LDS (an element at a
+// time, with its pair index from four divisions, 41 us at O=20 V=120, 92 MB written).
+__global__ __launch_bounds__(BLK) void t2_unpack_kernel(int64_t O, int64_t V, int nt, const double2* __restrict__ packed,
                                                         double2* __restrict__ dense) {
-  const int64_t total = O * O * V * V, Pv = npair(V);
-  for (int64_t t = blockIdx.x * (int64_t)BLK + threadIdx.x; t < total; t += (int64_t)gridDim.x * BLK) {
-    int64_t r = t;
-    const int64_t b = r % V; r /= V;
-    const int64_t a = r % V; r /= V;
-    const int64_t j = r % O;
-    const int64_t i = r / O;
-    dense[t] = xget(packed, O, Pv, V, i, j, a, b);
+  __shared__ double2 T[32][33];
+  const int64_t Pv = npair(V), Po = npair(O), ntp = (int64_t)nt * (nt + 1) / 2;
+  const int64_t r = blockIdx.x / ntp;
+  int t = (int)(blockIdx.x % ntp), ta = 0;
+  while (t >= nt - ta) { t -= nt - ta; ++ta; }
+  const int64_t a0 = 32 * (int64_t)ta, b0 = 32 * (int64_t)(ta + t);
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  const double2 zero = make_double2(0.0, 0.0);
+  auto at = [&](int64_t i, int64_t j, int64_t a, int64_t b) -> double2& { return dense[((i * O + j) * V + a) * V + b]; };
+  if (r >= Po) {                                        // i == j: zeros
+    const int64_t i = r - Po;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int64_t a = a0 + ty + 8 * k, b = b0 + tx, at_ = a0 + tx, bt = b0 + ty + 8 * k;
+      if (a < V && b < V) at(i, i, a, b) = zero;
+      if (t > 0 && bt < V && at_ < V) at(i, i, bt, at_) = zero;
+    }
+    return;
+  }
+  int64_t i, j;
+  pdec(r, O, i, j);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int64_t a = a0 + ty + 8 * k, b = b0 + tx;
+    double2 v = zero;
+    if (b < V && a < b) v = packed[r * Pv + pidx(a, b, V)];
+    T[ty + 8 * k][tx] = v;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int64_t a = a0 + ty + 8 * k, b = b0 + tx;     // rows of the tile, b along the lanes
+    double2 v = T[ty + 8 * k][tx];
+    if (t == 0 && a > b) v = T[tx][ty + 8 * k], v = make_double2(-v.x, -v.y);
+    if (a < V && b < V) {
+      at(i, j, a, b) = v;
+      at(j, i, a, b) = a == b ? zero : make_double2(-v.x, -v.y);
+    }
+    if (t > 0) {                                         // the mirrored tile, a along the lanes
+      const int64_t br = b0 + ty + 8 * k, ac = a0 + tx;
+      const double2 u = T[tx][ty + 8 * k];
+      if (br < V && ac < V) {
+        at(i, j, br, ac) = make_double2(-u.x, -u.y);
+        at(j, i, br, ac) = u;
+      }
+    }
   }
 }
 
@@ -565,10 +718,11 @@ int apy_t2_pack(int64_t O, int64_t V, const void* dense, void* packed, void* str
 
 int apy_t2_unpack(int64_t O, int64_t V, const void* packed, void* dense, void* stream) {
   if (O < 0 || V < 0 || !dense || !packed || dense == packed) return APY_E_ARG;
-  const int64_t total = O * O * V * V;
-  if (total == 0) return APY_OK;
-  t2_unpack_kernel<<<apy_grid1d(total, 1 << 20), BLK, 0, (hipStream_t)stream>>>(O, V, (const double2*)packed,
-                                                                                (double2*)dense);
+  if (O * V == 0) return APY_OK;
+  const int64_t nt = (V + 31) / 32, grid = (npair(O) + O) * (nt * (nt + 1) / 2);
+  if (grid > 0x7fffffffLL) return APY_E_ARG;
+  t2_unpack_kernel<<<(unsigned)grid, BLK, 0, (hipStream_t)stream>>>(O, V, (int)nt, (const double2*)packed,
+                                                                    (double2*)dense);
   APY_LAUNCH_CHECK();
   return APY_OK;
 }
@@ -609,9 +763,8 @@ int apy_mp2_nc_batched_setup(int n, const apy_mp2_nc_instance* inst, void* works
     for (int32_t p = 0; p < (int32_t)npair(inst[k].O); ++p)
       for (int32_t ta = 0; ta < nt; ++ta)
         for (int32_t tb = ta; tb < nt; ++tb) it.push_back(Item{k, p, ta, tb});
-    for (int32_t i = 0; i < (int32_t)inst[k].O; ++i)
-      for (int64_t p0 = 0; p0 < Pv; p0 += ZS) zit.push_back(ZItem{k, i, (int32_t)p0, 0});
-    zoff[k + 1] = zoff[k] + inst[k].O * inst[k].O * Pv;
+    for (int64_t p0 = 0; p0 < Pv; p0 += zspan(inst[k].O)) zit.push_back(ZItem{k, (int32_t)p0});
+    zoff[k + 1] = zoff[k] + npair(inst[k].O) * Pv;
   }
   off[n] = (int64_t)it.size();
   Header h{n, items, zitems, (int64_t)L.zitem, (int64_t)L.z};
@@ -638,7 +791,7 @@ int apy_mp2_nc_batched_step(int n, int64_t n_items, int reverse, void* rnorm, vo
   double* part = (double*)(w + L.part);
   const auto* insts = (const apy_mp2_nc_instance*)(w + L.inst);
   const int64_t* zoff = (const int64_t*)(w + L.zoff);
-  // the Z work list is grid-strided over at most 4096 workgroups
+  // the W work list is grid-strided over at most 4096 workgroups
   nc_z_kernel<<<(unsigned)std::min<int64_t>(n_items, 4096), BLK, 0, st>>>(w, insts, zoff, reverse);
   APY_LAUNCH_CHECK();
   ncp_step_kernel<<<(unsigned)n_items, SBLK, 0, st>>>(insts, (const Item*)(w + L.item), reverse, w, zoff, part);

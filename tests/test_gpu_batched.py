@@ -160,6 +160,44 @@ def test_batched_wide_instances(dev, transpose):
         assert torch.equal(g.x[k], h.x[k])
 
 
+@pytest.mark.parametrize("O,V", [(2, 32), (8, 64), (9, 65), (12, 16), (13, 31), (17, 48), (19, 80), (21, 20), (41, 7)])
+@pytest.mark.parametrize("transpose", [False, True])
+def test_batched_step_at_tile_edges(dev, O, V, transpose):
+    """One step from random amplitudes against the dense formula in torch: virtual spaces at the edges of the
+    16-wide blocks and of the 32- and 64-wide tiles, occupied spaces at the edges of the row blocks of
+    F_oo x (8, 12, 16, 18, 20 and two passes).  Sums of up to O + V terms of order one."""
+    g = torch.Generator(device=dev).manual_seed(100 * O + V)
+    cn = lambda *sh: torch.randn(*sh, dtype=torch.complex128, device=dev, generator=g)
+
+    def anti(x):
+        x = x - x.transpose(0, 1)
+        return x - x.transpose(2, 3)
+
+    n = O + V
+    F = cn(n, n)
+    eps = torch.cat([-2.0 + torch.rand(O, dtype=torch.float64, device=dev, generator=g),
+                     1.0 + torch.rand(V, dtype=torch.float64, device=dev, generator=g)])
+    drv, x = anti(cn(O, O, V, V)), anti(cn(O, O, V, V))
+    b = MP2NCBatch([Instance(O, V, F, eps, drv.reshape(-1), drv.reshape(-1), transpose_f=transpose)])
+    b.start_from(0, x)
+    b.step(0)
+    f = F.T if transpose else F
+    Y = torch.matmul(x, f[O:, O:].T)
+    Z = torch.matmul(f[:O, :O].T, x.reshape(O, O, V * V)).reshape(O, O, V, V)     # sum_m x_im f_mj
+    r = drv + Y - Y.transpose(2, 3) - Z + Z.transpose(0, 1)
+    e = eps
+    D = e[:O, None, None, None] + e[None, :O, None, None] - e[None, None, O:, None] - e[None, None, None, O:]
+    want = x + r / D
+    got = MP2NCBatch([Instance(O, V, F, eps, drv.reshape(-1), drv.reshape(-1))])
+    got.x[0].copy_(b.x_new[0])
+    got = got.amplitudes(0).reshape(O, O, V, V)
+    assert (got - want).abs().max() < 1e-13 * want.abs().max()
+    i, j = torch.triu_indices(O, O, 1, device=dev)
+    a, c = torch.triu_indices(V, V, 1, device=dev)
+    rr = (r[i, j][:, a, c].abs() ** 2).sum()
+    assert abs(b.rnorm[0] - rr) < 1e-12 * rr
+
+
 def test_packed_storage_round_trip_and_warm_start(dev):
     """The packed amplitudes expand to the antisymmetric dense tensor and
     pack back exactly; a batch started from converged amplitudes stays at
