@@ -85,12 +85,14 @@ template <int BM, int BN, int WM, int WN, int BK, bool A_MK, bool B_NK, bool G3>
 __device__ __forceinline__ void zgemm_tile(const GemmArgs& p, int64_t logical, double2* lds) {
   constexpr int RB = WM / 16, CB = WN / 16;
   constexpr int BKP = BK + 1;  // padded row (complex elements) of k-contiguous LDS tiles
-  constexpr int A_PER = BM * BK / NTHR;
+  constexpr int A_PER = (BM * BK + NTHR - 1) / NTHR;
   constexpr int B_PER = BN * BK / NTHR;
+  constexpr bool A_FULL = BM * BK % NTHR == 0;   // else the last of the A_PER elements is some threads' only
   constexpr int A_LDS = BM * BKP;
   constexpr int B_LDS = B_NK ? BN * BKP : BK * BN;
-  static_assert(BM == 2 * WM && BN == 2 * WN, "2x2 wave grid");
-  static_assert(A_PER >= 1 && B_PER >= 1, "tile too small");
+  constexpr int NWN = BN / WN;                   // waves side by side
+  static_assert((BM / WM) * NWN * 64 == NTHR && BM % WM == 0 && BN % WN == 0, "four waves");
+  static_assert(BN * BK % NTHR == 0, "tile too small");
 
   // Interleaved (re, im) tiles: one 16-byte LDS read yields both planes of
   // an MFMA operand.  Row strides of BKP complex (272 B for BK=16) keep the
@@ -101,7 +103,7 @@ __device__ __forceinline__ void zgemm_tile(const GemmArgs& p, int64_t logical, d
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
+  const int wm = wave / NWN, wn = wave % NWN;
 
   const int64_t mt = logical % p.mtiles; logical /= p.mtiles;
   const int64_t nt = logical % p.ntiles; logical /= p.ntiles;
@@ -144,7 +146,7 @@ __device__ __forceinline__ void zgemm_tile(const GemmArgs& p, int64_t logical, d
     constexpr int set = decltype(setc)::value;
 #pragma unroll
     for (int q = 0; q < A_PER; ++q) {
-      const int idx = tid + NTHR * q;
+      const int idx = A_FULL ? tid + NTHR * q : min(tid + NTHR * q, BM * BK - 1);
       int r, kk;
       if (A_MK) { r = idx / BK; kk = idx % BK; } else { kk = idx / BM; r = idx % BM; }
       const int64_t gm = min(m0 + r, p.m - 1), gk = min(k0 + kk, kend - 1);
@@ -163,7 +165,7 @@ __device__ __forceinline__ void zgemm_tile(const GemmArgs& p, int64_t logical, d
     constexpr int buf = decltype(bufc)::value, set = buf;
 #pragma unroll
     for (int q = 0; q < A_PER; ++q) {
-      const int idx = tid + NTHR * q;
+      const int idx = A_FULL ? tid + NTHR * q : min(tid + NTHR * q, BM * BK - 1);   // the last: stored alike by all
       int r, kk;
       if (A_MK) { r = idx / BK; kk = idx % BK; } else { kk = idx / BM; r = idx % BM; }
       const bool in = (m0 + r < p.m) && (k0 + kk < kend);
@@ -296,26 +298,32 @@ __global__ __launch_bounds__(NTHR) void zgemm_mfma(GemmArgs p) {
 // Several independent products in one launch: the blocks of each on a range of the grid that starts at a
 // multiple of 8 (so xcd_remap sees the XCD the block is on).  A CISD step is 8 to 14 products of very
 // different sizes, most of which cannot fill the chip alone: launched one after another they ran at their
-// own latency, together they share the CUs (O=10 V=4: 22 launches, 93 us a step -> 6 launches, 38 us;
-// o=9 v=25: 157 -> 62; O=18 V=50: 372 -> 279; o=10 v=80: 679 -> 575).  Two tiles, chosen per product by padding: 64 x 64 and
-// 32 x 64, both with BK = 8 (168 registers, three blocks a CU).  G3: the 64 x 64 tile in the three-product
-// form, and only for the products that ask for it.
+// own latency, together they share the CUs (O=10 V=4: 22 launches, 93 us a step -> 6 launches, 37 us;
+// o=9 v=25: 157 -> 58; O=18 V=50: 372 -> 241; o=10 v=80: 679 -> 520).  Five tiles, the one with the least
+// padding at its own rate for each product (168 registers and at most 44 KB of LDS: three blocks a CU);
+// 16 x 64 and 48 x 64 are for the few rows of singles and of antisymmetric pairs: with 64 x 64 and 32 x 64
+// alone o=10 v=80 took 540 us.  G3: the 64 x 64 tile in the three-product form, and only for the products
+// that ask for it.
 constexpr int GROUP_MAX = 14;
 struct GroupArgs {
   GemmArgs g[GROUP_MAX];
   int32_t start[GROUP_MAX];
-  int32_t kind[GROUP_MAX];   // bit 0: A_MK, bit 1: B_NK, bit 2: the 32 x 64 tile
+  int32_t kind[GROUP_MAX];   // bit 0: A_MK, bit 1: B_NK, then 4 x the index of the tile in GROUP_TILES
   int32_t n;
 };
 
 template <bool G3>
-__global__ __launch_bounds__(NTHR, G3 ? 2 : 3) void zgemm_group(GroupArgs G) {
-  constexpr int L = tile_lds<64, 64, 8, true>;
-  static_assert(L >= tile_lds<64, 64, 8, false> && L >= tile_lds<32, 64, 8, true>, "LDS of the largest tile");
+__global__ __launch_bounds__(NTHR, G3 ? 2 : 3) void zgemm_group(GroupArgs) {
+  // the argument block read in place (its index is uniform): through the parameter the compiler makes a
+  // private copy of all of it
+  const GroupArgs& G = *(const GroupArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  constexpr int L = tile_lds<16, 64, 16, true>;
+  static_assert(L >= tile_lds<64, 64, 8, true> && L >= tile_lds<32, 64, 8, true> && L >= tile_lds<32, 32, 16, true> &&
+                    L >= tile_lds<48, 64, 8, true>, "LDS of the largest tile");
   __shared__ double2 lds[L];
   int q = 0;
   while (q + 1 < G.n && (int)blockIdx.x >= G.start[q + 1]) ++q;
-  const GemmArgs& p = G.g[q];
+  const GemmArgs p = G.g[q];
   const int64_t bid = (int64_t)blockIdx.x - G.start[q];
   if (bid >= p.total) return;
   const int64_t u = xcd_remap(bid, p.total);
@@ -327,7 +335,19 @@ __global__ __launch_bounds__(NTHR, G3 ? 2 : 3) void zgemm_group(GroupArgs G) {
     case 4: zgemm_tile<32, 64, 16, 32, 8, false, false, false>(p, u, lds); break;
     case 5: zgemm_tile<32, 64, 16, 32, 8, true, false, false>(p, u, lds); break;
     case 6: zgemm_tile<32, 64, 16, 32, 8, false, true, false>(p, u, lds); break;
-    default: zgemm_tile<32, 64, 16, 32, 8, true, true, false>(p, u, lds); break;
+    case 7: zgemm_tile<32, 64, 16, 32, 8, true, true, false>(p, u, lds); break;
+    case 8: zgemm_tile<32, 32, 16, 16, 16, false, false, false>(p, u, lds); break;
+    case 9: zgemm_tile<32, 32, 16, 16, 16, true, false, false>(p, u, lds); break;
+    case 10: zgemm_tile<32, 32, 16, 16, 16, false, true, false>(p, u, lds); break;
+    case 11: zgemm_tile<32, 32, 16, 16, 16, true, true, false>(p, u, lds); break;
+    case 12: zgemm_tile<16, 64, 16, 16, 16, false, false, false>(p, u, lds); break;
+    case 13: zgemm_tile<16, 64, 16, 16, 16, true, false, false>(p, u, lds); break;
+    case 14: zgemm_tile<16, 64, 16, 16, 16, false, true, false>(p, u, lds); break;
+    case 15: zgemm_tile<16, 64, 16, 16, 16, true, true, false>(p, u, lds); break;
+    case 16: zgemm_tile<48, 64, 48, 16, 8, false, false, false>(p, u, lds); break;
+    case 17: zgemm_tile<48, 64, 48, 16, 8, true, false, false>(p, u, lds); break;
+    case 18: zgemm_tile<48, 64, 48, 16, 8, false, true, false>(p, u, lds); break;
+    default: zgemm_tile<48, 64, 48, 16, 8, true, true, false>(p, u, lds); break;
   }
 }
 
@@ -787,6 +807,14 @@ namespace {
 constexpr double GROUP_ALONE_FLOP = 2.0e10;   // about 0.3 ms
 constexpr int64_t GROUP_MIN_K = 64;           // shortest K slice: eight stages against the prologue
 constexpr double GROUP_PART_BYTES = 6.4e7;    // partial sums of one product at most
+// Work of a block, in shares of what one round of resident blocks would give each: a block more than a
+// round costs another whole one (o=18 v=50 by share 1: 271 us a step, 0.7: 263, 0.6: 241, 0.5: 250, 0.25:
+// 255; o=10 v=80: 523, 0.6: 521, 0.4: 513), smaller ones more partial sums.
+constexpr double GROUP_SHARE = 0.6;
+
+struct GroupTile { int bm, bn; double eff; };
+constexpr int NTILE = 5;
+constexpr GroupTile GROUP_TILES[NTILE] = {{64, 64, 0.855}, {32, 64, 0.81}, {32, 32, 0.76}, {16, 64, 0.70}, {48, 64, 0.82}};
 
 struct Group {
   int n = 0;                 // products in the launch
@@ -838,30 +866,37 @@ bool group_plan(const apy_gemm_desc* d, int n, Group& G) {
     ++count[t];
     of[i] = t;
   }
-  // Tile by padding, then K slices that give every block the same work with one round of resident blocks.
+  // Tile by padding, then K slices that give every block the same work.
+  bool g3 = false;
+  for (int i = 0; i < n; ++i) g3 = g3 || (!G.alone[i] && d[i].gauss3m);
   int kind[GROUP_MAX];
   double area[GROUP_MAX], T = 0.0;
   for (int i = 0; i < n; ++i) {
     if (G.alone[i]) continue;
-    const double c = (double)((d[i].n + 63) / 64) * 64;
-    const double a64 = (double)((d[i].m + 63) / 64) * 64 * c / CFGS[8].eff, a32 = (double)((d[i].m + 31) / 32) * 32 * c / CFGS[9].eff;
-    const bool small = !d[i].gauss3m && a32 < a64;
-    kind[i] = (d[i].a_layout == APY_MK ? 1 : 0) | (d[i].b_layout == APY_NK ? 2 : 0) | (small ? 4 : 0);
-    area[i] = small ? 32.0 * 64.0 : 64.0 * 64.0;
-    T += (small ? a32 : a64) * d[i].k * d[i].batch;
+    // the 64 x 64 tile of a G3 launch is for the products that ask for the three-product form
+    const int t0 = g3 && !d[i].gauss3m ? 1 : 0;
+    int best = t0;
+    double a = 0.0;
+    for (int t = t0; t < (d[i].gauss3m ? 1 : NTILE); ++t) {
+      const GroupTile& g = GROUP_TILES[t];
+      const double x = (double)((d[i].m + g.bm - 1) / g.bm * g.bm) * ((d[i].n + g.bn - 1) / g.bn * g.bn) / g.eff;
+      if (t == t0 || x < a) { best = t; a = x; }
+    }
+    kind[i] = (d[i].a_layout == APY_MK ? 1 : 0) | (d[i].b_layout == APY_NK ? 2 : 0) | best << 2;
+    area[i] = (double)GROUP_TILES[best].bm * GROUP_TILES[best].bn / GROUP_TILES[best].eff;
+    T += a * d[i].k * d[i].batch;
   }
-  const double slots = 3.0 * dev_info().cus, per = T / slots;
+  const double slots = (g3 ? 2.0 : 3.0) * dev_info().cus, per = T / slots * GROUP_SHARE;
   double work[GROUP_MAX];
   for (int i = 0; i < n; ++i) {
     if (G.alone[i]) continue;
-    const double eff = CFGS[(kind[i] & 4) ? 9 : 8].eff;
-    const int64_t want = std::max<int64_t>(GROUP_MIN_K, (int64_t)(per * eff / area[i]));
+    const int64_t want = std::max<int64_t>(GROUP_MIN_K, (int64_t)(per / area[i]));
     const double bytes = (double)d[i].m * d[i].n * d[i].batch * sizeof(double2);
     int64_t split = (d[i].k + want - 1) / want;
     split = std::min<int64_t>(split, std::max<int64_t>(1, (int64_t)(GROUP_PART_BYTES / bytes)));
     const int64_t kc = ((d[i].k + split - 1) / split + 15) / 16 * 16;
     split = (d[i].k + kc - 1) / kc;
-    work[i] = area[i] / eff * (double)std::min(kc, d[i].k);
+    work[i] = area[i] * (double)std::min(kc, d[i].k);
     int at = G.n++;
     while (at > 0 && work[G.idx[at - 1]] < work[i]) { G.idx[at] = G.idx[at - 1]; --at; }
     G.idx[at] = i;
@@ -914,7 +949,7 @@ int apy_zgemm_group(const apy_gemm_desc* d, int n, void* workspace, size_t ws_by
   for (int q = 0; q < G.n; ++q) {
     const int i = G.idx[q];
     const apy_gemm_desc& x = d[i];
-    const int bm = (G.kind[i] & 4) ? 32 : 64;
+    const GroupTile& tile = GROUP_TILES[G.kind[i] >> 2];
     GemmArgs& a = A.g[q];
     a = GemmArgs{};
     a.m = x.m; a.n = x.n; a.k = x.k;
@@ -925,7 +960,7 @@ int apy_zgemm_group(const apy_gemm_desc* d, int n, void* workspace, size_t ws_by
     a.conj_a = x.conj_a; a.conj_b = x.conj_b;
     a.use_beta = (x.beta_re != 0.0 || x.beta_im != 0.0) ? 1 : 0;
     a.batch = x.batch; a.split = G.split[i]; a.kchunk = G.kchunk[i];
-    a.mtiles = (x.m + bm - 1) / bm; a.ntiles = (x.n + 63) / 64;
+    a.mtiles = (x.m + tile.bm - 1) / tile.bm; a.ntiles = (x.n + tile.bn - 1) / tile.bn;
     a.total = a.mtiles * a.ntiles * a.split * a.batch;
     a.ws = G.off[i] != SIZE_MAX ? (double2*)((char*)workspace + G.off[i]) : nullptr;
     a.g3 = x.gauss3m ? 1 : 0;
@@ -936,16 +971,6 @@ int apy_zgemm_group(const apy_gemm_desc* d, int n, void* workspace, size_t ws_by
     if (blocks > 0x7fffffffLL) return APY_E_ARG;
   }
   if (g3) {
-    // the 64 x 64 tile of the G3 launch is for the products that ask for the three-product form
-    for (int q = 0; q < G.n; ++q)
-      if (!A.g[q].g3 && !(A.kind[q] & 4)) {
-        for (int i = 0; i < n; ++i) {
-          if (G.alone[i]) continue;
-          const int st = apy_zgemm_launch(&d[i], workspace, ws_bytes, s);
-          if (st != APY_OK) return st;
-        }
-        return APY_OK;
-      }
     zgemm_group<true><<<(unsigned)blocks, NTHR, 0, s>>>(A);
   } else {
     zgemm_group<false><<<(unsigned)blocks, NTHR, 0, s>>>(A);
