@@ -11,6 +11,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 namespace {
 
@@ -179,23 +180,32 @@ enum EriSym { ERI_NONE = 0, ERI_KET = 1, ERI_ALL = 2 };
 // Hermite Coulomb integrals, which is why the work is split by group quartets and not by elements: at
 // H2O2/6-31G* (34 functions, 2.1e6 primitive quartets of functions) there are 1.0e5 of groups.
 //
-// One workgroup computes the (up to EG^4) elements of a group quartet.  Primitive pairs are taken in
-// batches that fit LDS; per batch
-//   1. Hermite E coefficients of the bra and ket primitive pairs (a thread per pair, axis and bra power),
-//      G_n = pref (-2 alpha)^n F_n and the powers of P - Q (a thread per primitive quartet and order),
+// One workgroup computes the (up to EG^4) elements of a group quartet.  The expansion of a bra or ket
+// element (ab| in Hermite Gaussians is a list of slots, one for each pair of terms and (t, u, v); primitive
+// pairs are taken in batches that fit LDS; per batch
+//   1. Hermite E coefficients (a thread per primitive pair, axis and bra power), G_n = pref (-2 alpha)^n F_n
+//      and the powers of P - Q (a thread per primitive quartet and order),
 //   2. R_tuv = sum_ijk a_ti a_uj a_vk X^(t-2i) Y^(u-2j) Z^(v-2k) G_(t+u+v-i-j-k), a_ti = t!/(i!(t-2i)!2^i)
 //      (the Hermite recursion in closed form: every entry on its own, no order of evaluation between them),
-//   3. H[bra pair][ket element][tuv] += sum over the ket pairs of E^cd R, signs (-1)^t in E^cd,
-// and per bra batch acc[element] += E^ab H.  Contracting the ket pairs first makes the step
-// that touches every element run once a bra pair instead of once a primitive quartet.
-// Bound by the latency of these short phases, not by bytes or flops: 118 registers and 40 KB of LDS keep
-// four workgroups on a CU.  H2O2/6-31G*: 5040 us with a wave an element and every expansion redone for
-// each quartet of functions, 210 us so.
+//      and the slots' coefficients Lam[pair][slot] = c_a c_b E^x_t E^y_u E^z_v, signs (-1)^(t+u+v) in the ket's,
+//   3. H[bra pair][ket element][tuv] += sum over the ket pairs and the element's slots of Lam R,
+// and per bra batch acc[element] += sum over the bra pairs and the element's slots of Lam H.  Contracting the
+// ket pairs first makes the step that touches every element run once a bra pair instead of once a primitive
+// quartet.  Bound by the latency of these short phases, not by bytes or flops: the sums over slots are flat
+// loops of two slots by EU primitive pairs side by side (as loops over t, u and v with the products of E in
+// them, one sp quartet of three primitives took 165 us, now 50), and 168 registers and 52 KB of LDS keep three
+// workgroups on a CU.  H2O2/6-31G*: 5040 us with a wave an element and every expansion redone for each
+// quartet of functions, 158 us so.
 constexpr int EG = 6;                 // functions of a group
 constexpr int EPP = APY_GTO_MAXPRIM * APY_GTO_MAXPRIM;
-constexpr int EW = 1024;              // doubles: G, powers and R of a batch
-constexpr int EH = 36 * 36;           // doubles: H (a d,d pair's 35 tuv with its 36 ket elements: 1260)
+constexpr int EW = 1536;              // doubles: G, powers and R of a batch
+constexpr int EH = EG * EG * EG * EG; // doubles: H (a d,d pair's 35 tuv with its 36 ket elements: 1260)
 constexpr int EE = 448;               // doubles: E coefficients of a batch, bra or ket (f,f: 336 a pair)
+constexpr int ES = 384;               // slots by primitive pairs of a batch, bra or ket (d,d: 342 a pair; one
+                                      // element: at most 108)
+constexpr int ESUM = 2048;            // entries of the table of sums of two tuv (d,d against d,d: 1225)
+constexpr int EU = 4;                 // primitive pairs side by side
+constexpr int EACC = (EG * EG * EG * EG + 255) / 256;
 constexpr int ENR = (LQ + 1) * (LQ + 2) * (LQ + 3) / 6;   // tuv with t + u + v <= LQ
 constexpr int ETAB = 4096;            // group starts that LDS holds, all tables together
 
@@ -224,15 +234,27 @@ struct EriTab {
   int64_t n[4];
 };
 
+// A slot of an element: the places of E^x_t, E^y_u and E^z_v in a primitive pair's E block and the two
+// functions' coefficient rows (2 member + term); ca = 255 pads an element to an even count.
+struct EriSlot {
+  uint16_t e[3];
+  uint8_t ca, cb;
+};
+
 struct EriShared {
-  double W[EW], H[EH], acc[EG * EG * EG * EG], Eb[EE], Ek[EE];
+  double W[EW], H[EH], E[2][EE], Lam[2][ES];
   double exps[4][APY_GTO_MAXPRIM], cen[4][3], coef[4][EG][2][APY_GTO_MAXPRIM];
+  double pair[2][EPP][5];             // of each primitive pair: p = a + b, 1 / p and P
   double herm[LQ + 1][LQ / 2 + 1];    // a_ti
+  int16_t slot[2][EG * EG + 1];       // first slot of each element, bra and ket
   int8_t lmn[4][EG][2][3];
   uint8_t nterm[4][EG];
-  uint8_t tuv[ENR][3];
   uint8_t prim[2][EPP][2];            // primitives of pair b (bra) or q (ket)
-  int size[4], nprim[4], L[4], first[4], bad, ngrp[4];
+  uint8_t tuv[ENR][3];
+  uint8_t stuv[2][ES];                // tuv index of each slot of the slice
+  uint8_t sum[ESUM];                  // tuv index of the sum of a bra and a ket (t, u, v)
+  EriSlot rec[2][ES];
+  int size[4], nprim[4], L[4], first[4], ngrp[4];
 };
 
 // Starts of the groups of a table into `start` (start[ngrp] = n); by one thread.
@@ -248,12 +270,12 @@ __device__ int find_groups(int64_t n, const uint8_t* joins, uint16_t* start) {
 
 // E^{ij}_t of one primitive pair and axis for this i and all j <= Lb, into out[(i (Lb+1) + j) nt + t],
 // nt = La + Lb + 1, times sgn^t; the recursion of herm_E along one row, in registers.
-__device__ void herm_row(int i, int La, int Lb, double Q, double a, double b, double sgn, double* out) {
-  const double p = a + b, h = 0.5 / p, xpa = -b * Q / p, xpb = a * Q / p;
+__device__ void herm_row(int i, int La, int Lb, double Q, double a, double b, double ip, double sgn, double* out) {
+  const double h = 0.5 * ip, xpa = -b * Q * ip, xpb = a * Q * ip;
   double e[NE + 1];
 #pragma unroll
   for (int t = 0; t <= NE; ++t) e[t] = 0.0;
-  e[0] = exp(-a * b / p * Q * Q);
+  e[0] = exp(-a * b * ip * Q * Q);
   auto raise = [&](double x) {
     double lo = 0.0;                                   // E_(t-1) of the row below
 #pragma unroll
@@ -298,7 +320,7 @@ __device__ double boys_one(int n, double T) {
   return F;
 }
 
-__global__ __launch_bounds__(256, 4) void eri_kernel(int64_t ngeom, int64_t natom, const double* __restrict__ centers,
+__global__ __launch_bounds__(256, 3) void eri_kernel(int64_t ngeom, int64_t natom, const double* __restrict__ centers,
                                                   EriTab T, int sym, int grouped, double2* __restrict__ out) {
   __shared__ EriShared S;
   extern __shared__ uint16_t starts[];               // group starts, then the join flags (grouped only)
@@ -378,10 +400,7 @@ __global__ __launch_bounds__(256, 4) void eri_kernel(int64_t ngeom, int64_t nato
       S.first[x] = (int)b;
       S.size[x] = (int)(e - b);
       S.nprim[x] = ok ? f.nprim : 0;
-      int L = 0;
-      for (int64_t m = b; m < e && ok; ++m)
-        for (int t = 0; t < T.f[x][m].nterm; ++t) L = max(L, lsum(T.f[x][m].lmn[t]));
-      S.L[x] = L;
+      S.L[x] = 0;
       for (int k = 0; k < 3; ++k) S.cen[x][k] = ok ? centers[3 * (natom * g + f.atom) + k] : 0.0;
     }
     __syncthreads();
@@ -394,10 +413,7 @@ __global__ __launch_bounds__(256, 4) void eri_kernel(int64_t ngeom, int64_t nato
       if (m == 0 && t == 0) S.exps[x][k] = f.exps[k];
       if (k < 3) S.lmn[x][m][t][k] = (int8_t)f.lmn[t][k];
       if (k == 3 && t == 0) S.nterm[x][m] = (uint8_t)f.nterm;
-    }
-    if (tid < 2 * EPP) {
-      const int x = tid / EPP, b = tid % EPP, n = S.nprim[2 * x + 1];
-      if (n > 0) { S.prim[x][b][0] = (uint8_t)(b / n); S.prim[x][b][1] = (uint8_t)(b % n); }
+      if (k == 4 && S.nprim[x] > 0 && t < f.nterm) atomicMax(&S.L[x], lsum(f.lmn[t]));
     }
     __syncthreads();
     const int La = uniform(S.L[0]), Lb = uniform(S.L[1]), Lc = uniform(S.L[2]), Ld = uniform(S.L[3]);
@@ -405,20 +421,113 @@ __global__ __launch_bounds__(256, 4) void eri_kernel(int64_t ngeom, int64_t nato
     const int nbc = uniform(S.size[0]) * sz1, nkc = uniform(S.size[2]) * sz3;
     const int nbp = uniform(S.nprim[0] * S.nprim[1]), nkp = uniform(S.nprim[2] * S.nprim[3]);
     const bool bad = nbp * nkp == 0;
-    const int L1 = La + Lb, L = min(L1 + Lc + Ld, LQ), nr = tuv_count(L), nr1 = tuv_count(min(L1, L));
-    const int eb = 3 * (La + 1) * (Lb + 1) * (L1 + 1), ek = 3 * (Lc + 1) * (Ld + 1) * (Lc + Ld + 1);
+    const int L1 = La + Lb, L2 = Lc + Ld, L = min(L1 + L2, LQ), nr = tuv_count(L), nr1 = tuv_count(min(L1, L));
+    const int nr2 = tuv_count(min(L2, L));
+    const int eb = 3 * (La + 1) * (Lb + 1) * (L1 + 1), ek = 3 * (Lc + 1) * (Ld + 1) * (L2 + 1);
     const int wsz = 4 * (L + 1) + nr;
-    // batches of primitive pairs, ket elements of a slice (all of them but for f functions)
-    const int ks = min(nkc, EH / nr1);
-    const int Kb = max(1, min(nkp, min(EE / ek, EW / wsz)));
-    const int Bb = max(1, min(min(nbp, EE / eb), min(EW / (wsz * Kb), EH / (nr1 * ks))));
-    const int nbt = La + Lb + 1, nkt = Lc + Ld + 1;
-    const SmallDiv dL(L + 1), dR(nr), dR1(nr1), dA(La + 1), dC(Lc + 1), d3(3), dsz1(sz1), dsz3(sz3);
-
-    for (int k0 = 0; k0 < nkc; k0 += ks) {
-      const int nks = min(ks, nkc - k0), nel = nbc * nks;
+    const SmallDiv dL(L + 1), dR(nr), dR1(nr1), dR2(nr2), dA(La + 1), dC(Lc + 1), d3(3), dsz1(sz1), dsz3(sz3);
+    // tuv index of the sum of a bra's and a ket's; past L (read by elements past LQ only, which are NaN) 0
+    auto tuv_sum = [&](int x, int y) {
+      const int t = S.tuv[x][0] + S.tuv[y][0], u = S.tuv[x][1] + S.tuv[y][1], v = S.tuv[x][2] + S.tuv[y][2];
+      return t + u + v <= L ? tuv_index(t, u, v) : 0;
+    };
+    const bool tab = nr1 * nr2 <= ESUM;
+    // ---- per quartet: primitive pairs, the slots of every element, sums of tuv
+    if (!bad) {
+      if (tid < 128) {
+        const int x = tid >> 6, b = tid & 63, n = S.nprim[2 * x + 1];
+        if (b < (x ? nkp : nbp)) {
+          const int pa = b / n, pb = b % n;
+          const double ea = S.exps[2 * x][pa], e = S.exps[2 * x + 1][pb], p = ea + e, ip = 1.0 / p;
+          S.prim[x][b][0] = (uint8_t)pa;
+          S.prim[x][b][1] = (uint8_t)pb;
+          S.pair[x][b][0] = p;
+          S.pair[x][b][1] = ip;
+          for (int k = 0; k < 3; ++k)
+            S.pair[x][b][2 + k] = (ea * S.cen[2 * x][k] + e * S.cen[2 * x + 1][k]) / p;
+        }
+      } else {
+        const int x = (tid - 128) >> 6, e = tid & 63, ne = x ? nkc : nbc;   // waves 2 (bra) and 3 (ket)
+        int n = 0;
+        if (e < ne) {
+          const int ma = x ? dsz3.div(e) : dsz1.div(e), mb = x ? dsz3.mod(e) : dsz1.mod(e);
+          for (int ta = 0; ta < S.nterm[2 * x][ma]; ++ta)
+            for (int tb = 0; tb < S.nterm[2 * x + 1][mb]; ++tb) {
+              int c = 1;
+              for (int k = 0; k < 3; ++k) c *= S.lmn[2 * x][ma][ta][k] + S.lmn[2 * x + 1][mb][tb][k] + 1;
+              n += c;
+            }
+          n = (n + 1) & ~1;
+        }
+        int sc = n;                                    // inclusive scan over the wave
+        for (int o = 1; o < 64; o <<= 1) {
+          const int y = __shfl_up(sc, o, 64);
+          if ((tid & 63) >= o) sc += y;
+        }
+        if (e < ne) S.slot[x][e + 1] = (int16_t)sc;
+        if (e == 0) S.slot[x][0] = 0;
+      }
+      for (int w = tid; tab && w < nr1 * nr2; w += 256) S.sum[w] = (uint8_t)tuv_sum(dR2.div(w), dR2.mod(w));
+    }
+    __syncthreads();
+    const int totb = bad ? 0 : uniform(S.slot[0][nbc]), totk = bad ? 0 : uniform(S.slot[1][nkc]);
+    // slices of elements whose slots fit (all of them but for differentiated or f functions)
+    auto slice = [&](int x, int e0, int ne, int tot, int cap) {
+      if (bad) return ne - e0;
+      int n = min(ne - e0, cap);
+      if (tot > ES)
+        while (n > 1 && uniform(S.slot[x][e0 + n] - S.slot[x][e0]) > ES) --n;
+      return n;
+    };
+    for (int k0 = 0, nks; k0 < nkc; k0 += nks) {
+      nks = slice(1, k0, nkc, totk, EH / nr1);
+      for (int m0 = 0, nbs; m0 < nbc; m0 += nbs) {
+      nbs = slice(0, m0, nbc, totb, EG * EG);
+      const int nel = nbs * nks;
       const SmallDiv dK(nks);
-      for (int w = tid; w < nel; w += 256) S.acc[w] = 0.0;
+      const int sk0 = bad ? 0 : uniform(S.slot[1][k0]), sb0 = bad ? 0 : uniform(S.slot[0][m0]);
+      const int nsk = bad ? 1 : uniform(S.slot[1][k0 + nks]) - sk0, nsb = bad ? 1 : uniform(S.slot[0][m0 + nbs]) - sb0;
+      const SmallDiv dsb(nsb), dsk(nsk);
+      // the slots of the slice, a thread each
+      for (int w = tid; w < nsb + nsk && !bad; w += 256) {
+        const int x = w < nsb ? 0 : 1, sl = x ? w - nsb : w, g = sl + (x ? sk0 : sb0);
+        int e = 0, hi = x ? nkc : nbc;                   // last element whose first slot is at most g
+        while (hi - e > 1) {
+          const int mid = (e + hi) >> 1;
+          if (S.slot[x][mid] <= g) e = mid; else hi = mid;
+        }
+        const int ma = x ? dsz3.div(e) : dsz1.div(e), mb = x ? dsz3.mod(e) : dsz1.mod(e);
+        int n = g - S.slot[x][e], tuv = 0;
+        EriSlot r;
+        r.e[0] = r.e[1] = r.e[2] = 0;
+        r.ca = 255;
+        r.cb = 0;
+        for (int tt = 0; tt < S.nterm[2 * x][ma] * S.nterm[2 * x + 1][mb]; ++tt) {
+          const int ta = tt / S.nterm[2 * x + 1][mb], tb = tt % S.nterm[2 * x + 1][mb];
+          const int8_t* la = S.lmn[2 * x][ma][ta];
+          const int8_t* lb = S.lmn[2 * x + 1][mb][tb];
+          const int lx = la[0] + lb[0], ly = la[1] + lb[1], lz = la[2] + lb[2], c = (lx + 1) * (ly + 1) * (lz + 1);
+          if (n >= 0 && n < c) {
+            const int k = n % (lz + 1), j = n / (lz + 1) % (ly + 1), i = n / ((lz + 1) * (ly + 1));
+            const int l2 = (x ? Ld : Lb) + 1, nt = (x ? L2 : L1) + 1, ax = (x ? ek : eb) / 3;
+            r.e[0] = (uint16_t)((la[0] * l2 + lb[0]) * nt + i);
+            r.e[1] = (uint16_t)(ax + (la[1] * l2 + lb[1]) * nt + j);
+            r.e[2] = (uint16_t)(2 * ax + (la[2] * l2 + lb[2]) * nt + k);
+            r.ca = (uint8_t)(2 * ma + ta);
+            r.cb = (uint8_t)(2 * mb + tb);
+            tuv = tuv_index(i, j, k);
+          }
+          n -= c;
+        }
+        S.rec[x][sl] = r;
+        S.stuv[x][sl] = (uint8_t)tuv;
+      }
+      // batches of primitive pairs
+      const int Kb = max(1, min(min(nkp, ES / nsk), min(EE / ek, EW / wsz)));
+      const int Bb = max(1, min(min(nbp, ES / nsb), min(EE / eb, min(EW / (wsz * Kb), EH / (nr1 * nks)))));
+      double acc[EACC];
+#pragma unroll
+      for (int m = 0; m < EACC; ++m) acc[m] = 0.0;
       for (int b0 = 0; b0 < nbp && !bad; b0 += Bb) {
         const int nb = min(Bb, nbp - b0);
         for (int w = tid; w < nb * nks * nr1; w += 256) S.H[w] = 0.0;
@@ -426,28 +535,28 @@ __global__ __launch_bounds__(256, 4) void eri_kernel(int64_t ngeom, int64_t nato
           const int nq = min(Kb, nkp - q0), nbq = nb * nq;
           const SmallDiv dq(nq);
           // 1. E of the bra batch (once) and of the ket batch (again only if it changes), G and powers
-          const int nEb = q0 == 0 ? nb * 3 * (La + 1) : 0;
-          const int nEk = (Kb < nkp || b0 == 0) ? nq * 3 * (Lc + 1) : 0;
-          for (int w = tid; w < nEb + nEk + nbq * (L + 1); w += 256) {
-            if (w < nEb) {
-              const int y = dA.div(w), i = dA.mod(w), b = d3.div(y), ax = d3.mod(y);
-              herm_row(i, La, Lb, S.cen[0][ax] - S.cen[1][ax], S.exps[0][S.prim[0][b0 + b][0]],
-                       S.exps[1][S.prim[0][b0 + b][1]], 1.0, S.Eb + b * eb + ax * (eb / 3));
-            } else if (w < nEb + nEk) {
-              const int y = dC.div(w - nEb), i = dC.mod(w - nEb), b = d3.div(y), ax = d3.mod(y);
-              herm_row(i, Lc, Ld, S.cen[2][ax] - S.cen[3][ax], S.exps[2][S.prim[1][q0 + b][0]],
-                       S.exps[3][S.prim[1][q0 + b][1]], -1.0, S.Ek + b * ek + ax * (ek / 3));
-            } else {
-              const int bq = dL.div(w - nEb - nEk), n = dL.mod(w - nEb - nEk), b = b0 + dq.div(bq),
-                        q = q0 + dq.mod(bq);
-              const double xa = S.exps[0][S.prim[0][b][0]], xb = S.exps[1][S.prim[0][b][1]], p = xa + xb;
-              const double xc = S.exps[2][S.prim[1][q][0]], xd = S.exps[3][S.prim[1][q][1]], s = xc + xd;
-              const double alpha = p * s / (p + s);
+          const bool newb = q0 == 0, newk = Kb < nkp || b0 == 0;
+          // (a wave each for the bra's E and the ket's, two for G: in one wave their latencies would add up)
+          const int wave = tid >> 6;
+          if (wave < 2) {
+            const int x = wave, l1 = x ? Lc : La, l2 = x ? Ld : Lb, p0 = x ? q0 : b0, es = x ? ek : eb;
+            const int n = (x ? newk : newb) ? (x ? nq : nb) * 3 * (l1 + 1) : 0;
+            for (int w = tid & 63; w < n; w += 64) {
+              const int y = x ? dC.div(w) : dA.div(w), i = x ? dC.mod(w) : dA.mod(w), b = d3.div(y), ax = d3.mod(y);
+              const uint8_t* pr = S.prim[x][p0 + b];
+              herm_row(i, l1, l2, S.cen[2 * x][ax] - S.cen[2 * x + 1][ax], S.exps[2 * x][pr[0]],
+                       S.exps[2 * x + 1][pr[1]], S.pair[x][p0 + b][1], x ? -1.0 : 1.0, S.E[x] + b * es + ax * (es / 3));
+            }
+          } else {
+            for (int w = tid - 128; w < nbq * (L + 1); w += 128) {
+              const int bq = dL.div(w), n = dL.mod(w);
+              const double* B = S.pair[0][b0 + dq.div(bq)];
+              const double* Q = S.pair[1][q0 + dq.mod(bq)];
+              const double p = B[0], s = Q[0], alpha = p * s / (p + s);
               double* Wq = S.W + bq * wsz;
               double r2 = 0.0;
               for (int ax = 0; ax < 3; ++ax) {
-                const double d = (xa * S.cen[0][ax] + xb * S.cen[1][ax]) / p -
-                                 (xc * S.cen[2][ax] + xd * S.cen[3][ax]) / s;
+                const double d = B[2 + ax] - Q[2 + ax];
                 r2 += d * d;
                 double pw = 1.0;
                 for (int k = 0; k < n; ++k) pw *= d;
@@ -459,25 +568,61 @@ __global__ __launch_bounds__(256, 4) void eri_kernel(int64_t ngeom, int64_t nato
             }
           }
           __syncthreads();
-          // 2. R_tuv
-          for (int w = tid; w < nbq * nr; w += 256) {
-            const int rr = dR.mod(w);
-            double* Wq = S.W + dR.div(w) * wsz;
-            const int t = S.tuv[rr][0], u = S.tuv[rr][1], v = S.tuv[rr][2];
-            const double* X = Wq + (L + 1);
-            const double* Y = X + (L + 1);
-            const double* Z = Y + (L + 1);
-            double sx = 0.0;
-            for (int i = 0; 2 * i <= t; ++i) {
-              double sy = 0.0;
-              for (int j = 0; 2 * j <= u; ++j) {
-                double sz = 0.0;
-                for (int k = 0; 2 * k <= v; ++k) sz += S.herm[v][k] * Z[v - 2 * k] * Wq[t + u + v - i - j - k];
-                sy += S.herm[u][j] * Y[u - 2 * j] * sz;
+          // 2. R_tuv, and the slots' coefficients
+          auto coulomb = [&](auto uc) {
+            constexpr int U = decltype(uc)::value;
+            for (int w = tid; w < nr * ((nbq + U - 1) / U); w += 256) {
+              const int rr = dR.mod(w), x0 = U * dR.div(w);
+              const int t = S.tuv[rr][0], u = S.tuv[rr][1], v = S.tuv[rr][2];
+              const double* Wq[U];
+#pragma unroll
+              for (int x = 0; x < U; ++x) Wq[x] = S.W + min(x0 + x, nbq - 1) * wsz;
+              double sx[U];
+#pragma unroll
+              for (int x = 0; x < U; ++x) sx[x] = 0.0;
+              for (int i = 0; 2 * i <= t; ++i) {
+                double sy[U];
+#pragma unroll
+                for (int x = 0; x < U; ++x) sy[x] = 0.0;
+                for (int j = 0; 2 * j <= u; ++j) {
+                  double sz[U];
+#pragma unroll
+                  for (int x = 0; x < U; ++x) sz[x] = 0.0;
+                  for (int k = 0; 2 * k <= v; ++k) {
+                    const double a = S.herm[v][k];
+#pragma unroll
+                    for (int x = 0; x < U; ++x)
+                      sz[x] += a * Wq[x][3 * (L + 1) + v - 2 * k] * Wq[x][t + u + v - i - j - k];
+                  }
+                  const double a = S.herm[u][j];
+#pragma unroll
+                  for (int x = 0; x < U; ++x) sy[x] += a * Wq[x][2 * (L + 1) + u - 2 * j] * sz[x];
+                }
+                const double a = S.herm[t][i];
+#pragma unroll
+                for (int x = 0; x < U; ++x) sx[x] += a * Wq[x][L + 1 + t - 2 * i] * sy[x];
               }
-              sx += S.herm[t][i] * X[t - 2 * i] * sy;
+#pragma unroll
+              for (int x = 0; x < U; ++x)
+                if (x0 + x < nbq) S.W[(x0 + x) * wsz + 4 * (L + 1) + rr] = sx[x];
             }
-            Wq[4 * (L + 1) + rr] = sx;
+          };
+          if (nbq == 1) coulomb(std::integral_constant<int, 1>{});
+          else coulomb(std::integral_constant<int, EU>{});
+          // from the first thread on that has one R less to do
+          const int nlb = newb ? nb * nsb : 0, nlk = newk ? nq * nsk : 0;
+          const int ncoul = nbq == 1 ? nr : nr * ((nbq + EU - 1) / EU);
+          for (int w = (tid - ncoul) & 255; w < nlb + nlk; w += 256) {
+            const int x = w < nlb ? 0 : 1, y = x ? w - nlb : w;
+            const int q = x ? dsk.div(y) : dsb.div(y), sl = x ? dsk.mod(y) : dsb.mod(y);
+            const EriSlot r = S.rec[x][sl];
+            const double* E = S.E[x] + q * (x ? ek : eb);
+            const uint8_t* pr = S.prim[x][(x ? q0 : b0) + q];
+            double v = 0.0;
+            if (r.ca != 255)
+              v = (&S.coef[2 * x][0][0][0])[r.ca * APY_GTO_MAXPRIM + pr[0]] *
+                  (&S.coef[2 * x + 1][0][0][0])[r.cb * APY_GTO_MAXPRIM + pr[1]] * E[r.e[0]] * E[r.e[1]] * E[r.e[2]];
+            S.Lam[x][y] = v;
           }
           __syncthreads();
           // 3. the ket contraction; where the items are few, 2^sh neighbouring lanes share one
@@ -485,82 +630,95 @@ __global__ __launch_bounds__(256, 4) void eri_kernel(int64_t ngeom, int64_t nato
           int sh = 0;
           while (sh < 6 && (items << (sh + 1)) <= 256 && (1 << sh) < nq) ++sh;
           const int sub = tid & ((1 << sh) - 1);
-          for (int w = tid >> sh; w < items; w += 256 >> sh) {
-            const int y = dR1.div(w), rr = dR1.mod(w), b = dK.div(y), kc = k0 + dK.mod(y);
-            const int mc = dsz3.div(kc), md = dsz3.mod(kc);
-            const int t = S.tuv[rr][0], u = S.tuv[rr][1], v = S.tuv[rr][2];
-            double h = 0.0;
-            for (int tc = 0; tc < S.nterm[2][mc]; ++tc)
-              for (int td = 0; td < S.nterm[3][md]; ++td) {
-                const int8_t* lc = S.lmn[2][mc][tc];
-                const int8_t* ld = S.lmn[3][md][td];
-                const int lx = lc[0] + ld[0], ly = lc[1] + ld[1], lz = lc[2] + ld[2];
-                if (t + u + v + lx + ly + lz > L) continue;   // read by elements past LQ only (NaN)
-                const int ox = (lc[0] * (Ld + 1) + ld[0]) * nkt, oy = ek / 3 + (lc[1] * (Ld + 1) + ld[1]) * nkt,
-                          oz = 2 * (ek / 3) + (lc[2] * (Ld + 1) + ld[2]) * nkt;
-                for (int q = sub; q < nq; q += 1 << sh) {
-                  const double* R = S.W + (b * nq + q) * wsz + 4 * (L + 1);
-                  const double* E = S.Ek + q * ek;
-                  double sx = 0.0;
-                  for (int i = 0; i <= lx; ++i) {
-                    double sy = 0.0;
-                    for (int j = 0; j <= ly; ++j) {
-                      double sz = 0.0;
-                      for (int k = 0; k <= lz; ++k) sz += E[oz + k] * R[tuv_index(t + i, u + j, v + k)];
-                      sy += E[oy + j] * sz;
-                    }
-                    sx += E[ox + i] * sy;
-                  }
-                  h += S.coef[2][mc][tc][S.prim[1][q0 + q][0]] * S.coef[3][md][td][S.prim[1][q0 + q][1]] * sx;
+          auto ket = [&](auto uc) {
+            constexpr int U = decltype(uc)::value;
+            for (int w = tid >> sh; w < items; w += 256 >> sh) {
+              const int y = dR1.div(w), rr = dR1.mod(w), b = dK.div(y), kc = k0 + dK.mod(y);
+              const int f = S.slot[1][kc] - sk0, n = S.slot[1][kc + 1] - sk0;
+              const uint8_t* sm = S.sum + rr * nr2;
+              const double* R = S.W + b * nq * wsz + 4 * (L + 1);
+              double h = 0.0;
+              for (int q = sub; q < nq; q += U << sh) {
+                int lq[U], rq[U];
+                double c[U];
+#pragma unroll
+                for (int x = 0; x < U; ++x) {
+                  const int z = q + (x << sh) < nq ? q + (x << sh) : q;
+                  lq[x] = z * nsk;
+                  rq[x] = z * wsz;
+                  c[x] = 0.0;
                 }
+                for (int s = f; s < n; s += 2) {
+                  const int t0 = S.stuv[1][s], t1 = S.stuv[1][s + 1];
+                  const int r0 = tab ? sm[t0] : tuv_sum(rr, t0), r1 = tab ? sm[t1] : tuv_sum(rr, t1);
+#pragma unroll
+                  for (int x = 0; x < U; ++x)
+                    c[x] += S.Lam[1][lq[x] + s] * R[rq[x] + r0] + S.Lam[1][lq[x] + s + 1] * R[rq[x] + r1];
+                }
+#pragma unroll
+                for (int x = 0; x < U; ++x)
+                  if (q + (x << sh) < nq) h += c[x];
               }
-            for (int o = (1 << sh) >> 1; o > 0; o >>= 1) h += __shfl_xor(h, o, 64);   // lanes of one item: all here
-            if (sub == 0) S.H[w] += h;
-          }
+              for (int o = (1 << sh) >> 1; o > 0; o >>= 1) h += __shfl_xor(h, o, 64);   // one item's lanes: all here
+              if (sub == 0) S.H[w] += h;
+            }
+          };
+          if (nq <= 1 << sh) ket(std::integral_constant<int, 1>{});
+          else ket(std::integral_constant<int, EU>{});
           __syncthreads();
         }
         // the bra contraction of this batch
-        for (int w = tid; w < nel; w += 256) {
-          const int kc = dK.mod(w), bc = dK.div(w), ma = dsz1.div(bc), mb = dsz1.mod(bc);
-          double h = 0.0;
-          for (int ta = 0; ta < S.nterm[0][ma]; ++ta)
-            for (int tb = 0; tb < S.nterm[1][mb]; ++tb) {
-              const int8_t* la = S.lmn[0][ma][ta];
-              const int8_t* lb = S.lmn[1][mb][tb];
-              const int lx = la[0] + lb[0], ly = la[1] + lb[1], lz = la[2] + lb[2];
-              if (lx + ly + lz > L) continue;
-              const int ox = (la[0] * (Lb + 1) + lb[0]) * nbt, oy = eb / 3 + (la[1] * (Lb + 1) + lb[1]) * nbt,
-                        oz = 2 * (eb / 3) + (la[2] * (Lb + 1) + lb[2]) * nbt;
-              for (int b = 0; b < nb; ++b) {
-                const double* Hq = S.H + (b * nks + kc) * nr1;
-                const double* E = S.Eb + b * eb;
-                double sx = 0.0;
-                for (int i = 0; i <= lx; ++i) {
-                  double sy = 0.0;
-                  for (int j = 0; j <= ly; ++j) {
-                    double sz = 0.0;
-                    for (int k = 0; k <= lz; ++k) sz += E[oz + k] * Hq[tuv_index(i, j, k)];
-                    sy += E[oy + j] * sz;
-                  }
-                  sx += E[ox + i] * sy;
-                }
-                h += S.coef[0][ma][ta][S.prim[0][b0 + b][0]] * S.coef[1][mb][tb][S.prim[0][b0 + b][1]] * sx;
+        auto bra = [&](auto uc) {
+          constexpr int U = decltype(uc)::value;
+#pragma unroll
+          for (int m = 0; m < EACC; ++m) {
+            const int w = tid + 256 * m;
+            if (w >= nel) continue;
+            const int kc = dK.mod(w), bc = m0 + dK.div(w);
+            const int f = S.slot[0][bc] - sb0, n = S.slot[0][bc + 1] - sb0;
+            const double* Hk = S.H + kc * nr1;
+            double h = 0.0;
+            for (int b = 0; b < nb; b += U) {
+              int lq[U], hq[U];
+              double c[U];
+#pragma unroll
+              for (int x = 0; x < U; ++x) {
+                const int z = b + x < nb ? b + x : b;
+                lq[x] = z * nsb;
+                hq[x] = z * nks * nr1;
+                c[x] = 0.0;
               }
+              for (int s = f; s < n; s += 2) {
+                // a slot past the tuv of H belongs to elements past LQ (NaN)
+                const int r0 = min((int)S.stuv[0][s], nr1 - 1), r1 = min((int)S.stuv[0][s + 1], nr1 - 1);
+#pragma unroll
+                for (int x = 0; x < U; ++x)
+                  c[x] += S.Lam[0][lq[x] + s] * Hk[hq[x] + r0] + S.Lam[0][lq[x] + s + 1] * Hk[hq[x] + r1];
+              }
+#pragma unroll
+              for (int x = 0; x < U; ++x)
+                if (b + x < nb) h += c[x];
             }
-          S.acc[w] += h;
-        }
-        __syncthreads();                              // H and E of this batch are read
+            acc[m] += h;
+          }
+        };
+        if (nb == 1) bra(std::integral_constant<int, 1>{});
+        else bra(std::integral_constant<int, EU>{});
+        __syncthreads();                              // H, E and the slots of this batch are read
       }
       // ---- out: the value of a canonical element to every image under the launch's symmetry
-      for (int w = tid; w < nel; w += 256) {
-        const int kc = k0 + dK.mod(w), bc = dK.div(w);
+#pragma unroll
+      for (int m = 0; m < EACC; ++m) {
+        const int w = tid + 256 * m;
+        if (w >= nel) continue;
+        const int kc = k0 + dK.mod(w), bc = m0 + dK.div(w);
         const int e0 = dsz1.div(bc), e1 = dsz1.mod(bc), e2 = dsz3.div(kc), e3 = dsz3.mod(kc);
         const int64_t i = S.first[0] + e0, j = S.first[1] + e1, k = S.first[2] + e2, l = S.first[3] + e3;
         // one element an image class: an order of functions is asked for where the group quartet leaves one open
         if (sym != ERI_NONE && k < l) continue;
         if (sym == ERI_ALL && i < j) continue;
         if (sym == ERI_ALL && G[0] == G[2] && G[1] == G[3] && (i < k || (i == k && j < l))) continue;
-        double v = S.acc[w];
+        double v = acc[m];
         if (bad) {
           v = kNaN;
         } else {
@@ -588,6 +746,7 @@ __global__ __launch_bounds__(256, 4) void eri_kernel(int64_t ngeom, int64_t nato
         o[at(l, k, i, j)] = y;
         o[at(k, l, j, i)] = y;
         o[at(l, k, j, i)] = y;
+      }
       }
     }
   }
@@ -772,9 +931,9 @@ int apy_eri_gto(int64_t ngeom, int64_t natom, const double* centers, const apy_g
   // tables whose group starts do not fit LDS are taken function by function
   const int64_t tot = na + 1 + (sym == ERI_ALL ? 0 : nb + nc + 2 + (sym == ERI_KET ? 0 : nd + 1));
   const int grouped = tot <= ETAB;
-  // a resident grid (four workgroups a CU): the groups are found once a workgroup
+  // a resident grid (three workgroups a CU): the groups are found once a workgroup
   const double bound = (double)ngeom * na * nb * nc * nd;
-  const unsigned grid = (unsigned)std::min(bound, 4.0 * 256.0);
+  const unsigned grid = (unsigned)std::min(bound, 3.0 * 256.0);
   const size_t lds = grouped ? (size_t)tot * (sizeof(uint16_t) + 1) : 0;
   eri_kernel<<<grid, 256, lds, (hipStream_t)stream>>>(ngeom, natom, centers, T, sym, grouped, (double2*)out);
   APY_LAUNCH_CHECK();
