@@ -543,45 +543,66 @@ __device__ __forceinline__ void epi2_doubles(const Epi2Args& e) {
   int64_t i, j;
   pdec(Pij, O, i, j);
 
-  // transposed X blocks: L[lb][la] = -X[(i,b),(j,a)] + X[(j,b),(i,a)]
-  for (int q = 0; q < ET / 8; ++q) {
-    const int lb = ty + 8 * q;
-    const int64_t b = b0 + lb, a = a0 + tx;
-    double2 v = make_double2(0.0, 0.0);
-    if (b < V && a < b) {
-      const double2 x3 = e.X[(i * V + b) * OV + j * V + a], x4 = e.X[(j * V + b) * OV + i * V + a];
-      v = make_double2(x4.x - x3.x, x4.y - x3.y);
+  // The reads of each part are issued before the first is used, outside a < b at the pair (0, 1): under
+  // conditions they followed each other at a read's latency.
+  constexpr int NK = ET / 8;
+  const double2 c0 = e.c0p ? *e.c0p : make_double2(e.c0r, e.c0i);
+  {
+    // transposed X blocks: L[lb][la] = -X[(i,b),(j,a)] + X[(j,b),(i,a)]
+    double2 x3[NK], x4[NK];
+#pragma unroll
+    for (int q = 0; q < NK; ++q) {
+      int64_t b = b0 + ty + 8 * q, a = a0 + tx;
+      if (b >= V || a >= b) { a = 0; b = 1; }
+      x3[q] = e.X[(i * V + b) * OV + j * V + a];
+      x4[q] = e.X[(j * V + b) * OV + i * V + a];
     }
-    L[lb][tx] = v;
+#pragma unroll
+    for (int q = 0; q < NK; ++q) L[ty + 8 * q][tx] = make_double2(x4[q].x - x3[q].x, x4[q].y - x3[q].y);
   }
 
-  double2 s[ET / 8];
-  const double2 c0 = e.c0p ? *e.c0p : make_double2(e.c0r, e.c0i);
-  for (int q = 0; q < ET / 8; ++q) {
-    const int la = ty + 8 * q;
-    const int64_t a = a0 + la, b = b0 + tx;
-    double2 v = make_double2(0.0, 0.0);
-    if (b < V && a < b) {
-      if (e.drv) v = cm(c0, e.drv[((i * O + j) * V + a) * V + b]);
+  double2 s[NK];
+  {
+    double2 dv[NK], rp[NK], x1[NK], x2[NK], q1[NK], q2[NK];
+#pragma unroll
+    for (int q = 0; q < NK; ++q) {
+      int64_t a = a0 + ty + 8 * q, b = b0 + tx;
+      if (b >= V || a >= b) { a = 0; b = 1; }
       const int64_t Pab = pidx(a, b, V);
-      acc(v, e.Rp[Pij * Pv + Pab]);
-      acc(v, e.X[(i * V + a) * OV + j * V + b]);
-      dec(v, e.X[(j * V + a) * OV + i * V + b]);
+      if (e.drv) dv[q] = e.drv[((i * O + j) * V + a) * V + b];
+      rp[q] = e.Rp[Pij * Pv + Pab];
+      x1[q] = e.X[(i * V + a) * OV + j * V + b];
+      x2[q] = e.X[(j * V + a) * OV + i * V + b];
       if (e.QT) {
-        acc(v, e.QT[j * e.qj + i * Pv + Pab]);
-        dec(v, e.QT[i * e.qj + j * Pv + Pab]);
-      }
-      if (e.fov) {
-        const int64_t n = e.n;
-        cfma(v, e.F[(O + b) * n + j], e.t1[i * V + a]);
-        cfma(v, e.F[(O + a) * n + i], e.t1[j * V + b]);
-        const double2 m1 = cm(e.F[(O + b) * n + i], e.t1[j * V + a]);
-        const double2 m2 = cm(e.F[(O + a) * n + j], e.t1[i * V + b]);
-        v.x -= m1.x + m2.x;
-        v.y -= m1.y + m2.y;
+        q1[q] = e.QT[j * e.qj + i * Pv + Pab];
+        q2[q] = e.QT[i * e.qj + j * Pv + Pab];
       }
     }
-    s[q] = v;
+#pragma unroll
+    for (int q = 0; q < NK; ++q) {
+      const int64_t a = a0 + ty + 8 * q, b = b0 + tx;
+      double2 v = make_double2(0.0, 0.0);
+      if (b < V && a < b) {
+        if (e.drv) v = cm(c0, dv[q]);
+        acc(v, rp[q]);
+        acc(v, x1[q]);
+        dec(v, x2[q]);
+        if (e.QT) {
+          acc(v, q1[q]);
+          dec(v, q2[q]);
+        }
+        if (e.fov) {
+          const int64_t n = e.n;
+          cfma(v, e.F[(O + b) * n + j], e.t1[i * V + a]);
+          cfma(v, e.F[(O + a) * n + i], e.t1[j * V + b]);
+          const double2 m1 = cm(e.F[(O + b) * n + i], e.t1[j * V + a]);
+          const double2 m2 = cm(e.F[(O + a) * n + j], e.t1[i * V + b]);
+          v.x -= m1.x + m2.x;
+          v.y -= m1.y + m2.y;
+        }
+      }
+      s[q] = v;
+    }
   }
 
   // T1 -> T2 through <kb||ij>: -U_ab + U_ba, U_ab = sum_k t1[k,a] <kb||ij>

@@ -372,84 +372,90 @@ __device__ __forceinline__ void sp_epi_doubles(const SpEpi& e) {
     const double2* Q1 = e.Q1 ? e.Q1 + qd : nullptr;
     const double2* Q2 = e.Q2 ? e.Q2 + qd : nullptr;
     __syncthreads();  // T of the previous tile is no longer read
+    // element (b, a) = (b0 + ty + 8k, a0 + tx), read along a.  All reads of a pass are issued before the
+    // first is used, past the edge and outside the packed halves at a place inside: under conditions they
+    // followed each other at a read's latency (16 us for the 81 tiles of o=9 v=25).
+    constexpr int NK = SET / 8;
+    {
+      double2 x1t[NK], x2[NK], y2[NK], q1t[NK], q2t[NK], ps[NK], pa[NK];
 #pragma unroll
-    for (int k = 0; k < SET / 8; ++k) {  // element (b, a) = (b0 + ty + 8k, a0 + tx), read along a
-      const int64_t b = b0 + ty + 8 * k, a = a0 + tx;
-      double2 s = make_double2(0.0, 0.0);
-      if (a < v && b < v) {
-        const double2 x1t = X1[(j * v + b) * ov + i * v + a];
-        const double2 x2 = X2[(i * v + b) * ov + j * v + a];
-        s.x = x1t.x - x2.x;
-        s.y = x1t.y - x2.y;
-        if (Y) {
-          const double2 y2 = Y[((j * o + i) * v + b) * v + a];
-          s.x += y2.x;
-          s.y += y2.y;
-        }
+      for (int k = 0; k < NK; ++k) {
+        const int64_t b = min(b0 + ty + 8 * k, v - 1), a = min(a0 + tx, v - 1);
+        x1t[k] = X1[(j * v + b) * ov + i * v + a];
+        x2[k] = X2[(i * v + b) * ov + j * v + a];
+        if (Y) y2[k] = Y[((j * o + i) * v + b) * v + a];
         if (Q1) {
-          const double2 q1t = Q1[j * (o * vv) + (i * v + b) * v + a];
-          const double2 q2t = Q2[((j * o + i) * v + b) * v + a];
-          s.x += q1t.x - q2t.x;
-          s.y += q1t.y - q2t.y;
+          q1t[k] = Q1[j * (o * vv) + (i * v + b) * v + a];
+          q2t[k] = Q2[((j * o + i) * v + b) * v + a];
         }
-        if (b < a) {
-          const double2 ps = Ps[isym(b, a, v)];
-          s.x += ps.x; s.y += ps.y;
-          if (Pa) {
-            const double2 pa = Pa[ianti(b, a, v)];
-            s.x += sgn_lower * pa.x; s.y += sgn_lower * pa.y;
-          }
-        }
+        ps[k] = Ps[b < a ? isym(b, a, v) : 0];
+        if (Pa) pa[k] = Pa[b < a ? ianti(b, a, v) : 0];
       }
-      T[ty + 8 * k][tx] = s;
+#pragma unroll
+      for (int k = 0; k < NK; ++k) {
+        const int64_t b = b0 + ty + 8 * k, a = a0 + tx;
+        double2 s = make_double2(x1t[k].x - x2[k].x, x1t[k].y - x2[k].y);
+        if (Y) { s.x += y2[k].x; s.y += y2[k].y; }
+        if (Q1) { s.x += q1t[k].x - q2t[k].x; s.y += q1t[k].y - q2t[k].y; }
+        if (b < a) {
+          s.x += ps[k].x; s.y += ps[k].y;
+          if (Pa) { s.x += sgn_lower * pa[k].x; s.y += sgn_lower * pa[k].y; }
+        }
+        T[ty + 8 * k][tx] = s;
+      }
     }
     __syncthreads();
     const double2 E = e.energy[q];
     const double* ep = e.eps + q * e.s_eps;
     const double eij = ep[i] + ep[j];
     const double2 rsc = e.rb ? resp_scalar(e.re, e.rs, e.es, q) : make_double2(0.0, 0.0);
+    // output (a, b) = (a0 + ty + 8k, b0 + tx), read along b
+    double2 vo[NK], p[NK], x1[NK], x2t[NK], y1[NK], q1[NK], q2[NK], ps[NK], pa[NK], x[NK], rbv[NK], rtv[NK];
+    double ea[NK];
+    const double ebb = ep[o + min(b0 + tx, v - 1)];
 #pragma unroll
-    for (int k = 0; k < SET / 8; ++k) {  // output (a, b) = (a0 + ty + 8k, b0 + tx), read along b
+    for (int k = 0; k < NK; ++k) {
+      const int64_t a = min(a0 + ty + 8 * k, v - 1), b = min(b0 + tx, v - 1);
+      const int64_t t = ((i * o + j) * v + a) * v + b;
+      vo[k] = e.vvoo[q * e.s_vvoo + t];
+      p[k] = e.R[qd + t];
+      x1[k] = X1[(i * v + a) * ov + j * v + b];
+      x2t[k] = X2[(j * v + a) * ov + i * v + b];
+      if (Y) y1[k] = Y[t];
+      if (Q1) {
+        q1[k] = Q1[i * (o * vv) + (j * v + a) * v + b];
+        q2[k] = Q2[t];
+      }
+      ps[k] = Ps[a <= b ? isym(a, b, v) : 0];
+      if (Pa) pa[k] = Pa[a < b ? ianti(a, b, v) : 0];
+      x[k] = e.t2[qv + t];
+      if (e.rb) { rbv[k] = e.rb[qv + t]; rtv[k] = e.rt[t]; }
+      ea[k] = ep[o + a];
+    }
+#pragma unroll
+    for (int k = 0; k < NK; ++k) {
       const int64_t a = a0 + ty + 8 * k, b = b0 + tx;
       if (a >= v || b >= v) continue;
       const int64_t t = ((i * o + j) * v + a) * v + b;
-      double2 rr = e.vvoo[q * e.s_vvoo + t];
+      double2 rr = vo[k];
       const double2 tt = T[tx][ty + 8 * k];
-      const double2 p = e.R[qd + t];
-      const double2 x1 = X1[(i * v + a) * ov + j * v + b];
-      const double2 x2t = X2[(j * v + a) * ov + i * v + b];
-      rr.x += tt.x + p.x + x1.x - x2t.x;
-      rr.y += tt.y + p.y + x1.y - x2t.y;
-      if (Y) {
-        const double2 y1 = Y[t];
-        rr.x += y1.x;
-        rr.y += y1.y;
-      }
-      if (Q1) {
-        const double2 q1 = Q1[i * (o * vv) + (j * v + a) * v + b];
-        const double2 q2 = Q2[t];
-        rr.x += q1.x - q2.x;
-        rr.y += q1.y - q2.y;
-      }
+      rr.x += tt.x + p[k].x + x1[k].x - x2t[k].x;
+      rr.y += tt.y + p[k].y + x1[k].y - x2t[k].y;
+      if (Y) { rr.x += y1[k].x; rr.y += y1[k].y; }
+      if (Q1) { rr.x += q1[k].x - q2[k].x; rr.y += q1[k].y - q2[k].y; }
       if (a <= b) {
-        const double2 ps = Ps[isym(a, b, v)];
-        rr.x += ps.x; rr.y += ps.y;
-        if (Pa && a < b) {
-          const double2 pa = Pa[ianti(a, b, v)];
-          rr.x -= sgn_lower * pa.x; rr.y -= sgn_lower * pa.y;
-        }
+        rr.x += ps[k].x; rr.y += ps[k].y;
+        if (Pa && a < b) { rr.x -= sgn_lower * pa[k].x; rr.y -= sgn_lower * pa[k].y; }
       }
-      const double2 x = e.t2[qv + t];
-      rr.x -= E.x * x.x - E.y * x.y;
-      rr.y -= E.x * x.y + E.y * x.x;
+      rr.x -= E.x * x[k].x - E.y * x[k].y;
+      rr.y -= E.x * x[k].y + E.y * x[k].x;
       if (e.rb) {
-        const double2 bb = e.rb[qv + t], y = e.rt[t];
-        rr.x += bb.x - (rsc.x * y.x - rsc.y * y.y);
-        rr.y += bb.y - (rsc.x * y.y + rsc.y * y.x);
+        rr.x += rbv[k].x - (rsc.x * rtv[k].x - rsc.y * rtv[k].y);
+        rr.y += rbv[k].y - (rsc.x * rtv[k].y + rsc.y * rtv[k].x);
       }
-      const double D = eij - ep[o + a] - ep[o + b];
+      const double D = eij - ea[k] - ebb;
       e.r2[qv + t] = rr;
-      e.t2_new[qv + t] = make_double2(x.x + rr.x / D, x.y + rr.y / D);
+      e.t2_new[qv + t] = make_double2(x[k].x + rr.x / D, x[k].y + rr.y / D);
     }
   }
 }
