@@ -147,6 +147,14 @@ __device__ inline void kind_index(int kind, int64_t t, int64_t O, int64_t V, int
   }
 }
 
+// A store that leaves the caches to the integrals that are still read: for whole runs of an output that
+// does not fit them (vvvo_p of m = 60 62 -> 55 us, the others 28 -> 25 us; packed rows, which end inside cache
+// lines, lose by it, 127 -> 149 us).
+__device__ inline void nt_store(double2* p, double2 v) {
+  typedef double v2d __attribute__((ext_vector_type(2)));
+  __builtin_nontemporal_store((v2d){v.x, v.y}, (v2d*)p);
+}
+
 template <class Src>
 __global__ __launch_bounds__(256) void build_block(Src src, int kind, int64_t O, int64_t V, double2* out,
                                                    int64_t total, int accumulate, double scale) {
@@ -158,7 +166,7 @@ __global__ __launch_bounds__(256) void build_block(Src src, int kind, int64_t O,
       double2 o = out[t];
       out[t] = make_double2(o.x + scale * v.x, o.y + scale * v.y);
     } else {
-      out[t] = v;
+      nt_store(out + t, v);
     }
   }
 }
@@ -169,8 +177,8 @@ __global__ __launch_bounds__(256) void build_block(Src src, int kind, int64_t O,
 // One workgroup takes a pair (P, Q) and a 32 x 32 tile of (R, S): it reads the tile of M and the mirrored
 // one along their rows into LDS and writes the rows of the up to four spin pairs along the output's
 // contiguous index.  build_block read M[S][R] one element a cache line (stride m^2) and decoded four
-// orbitals an element: m = 60, O = 20 (57e6 elements, 0.92 GB) 560 us in all, bound by those reads; this
-// is bound by its writes.
+// orbitals an element: m = 60, O = 20 (57e6 elements, 0.92 GB) 560 us in all, bound by those reads, 335 us
+// so, bound by its writes.
 //   KIND            p       q      columns                    output index
 //   K_VVVV_P        a    <  b      r = c < s = d              [(ab)][(cd)]
 //   K_VOVV          a       j      r = c < s = b              [a][j][(cb)]
@@ -248,7 +256,8 @@ __global__ __launch_bounds__(256) void build_pair_rows(const double2* __restrict
         v.y -= u.y;
       }
       const int64_t o = TRI ? prow(r - O, V) + s - r - 1 : KIND == K_VVVO_P ? s * V + r - O : s * V * OV + r - O;
-      out[base + o] = v;
+      if (TRI) out[base + o] = v;
+      else nt_store(out + base + o, v);
     }
   }
 }
@@ -308,7 +317,7 @@ __global__ void so_fock_kernel(int64_t m, int64_t nb, const double2* fmo, double
 
 // ------------------------------------------------------------ sigma pieces
 // Every sigma works from the packed doubles T_p[(i<j)][(a<b)] (the packed
-// input itself, or pack_t2 of a dense input); the dense images the GEMMs
+// input itself, or those of a dense input); the dense images the GEMMs
 // need are expanded from it with the antisymmetry signs.
 //
 // One launch forms all of them: the grid is cut into sections (in blocks), so that the small copies of a

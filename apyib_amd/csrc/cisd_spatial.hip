@@ -637,7 +637,7 @@ int sp_gemms(int64_t o, int64_t v, int singles, int64_t nb, int64_t L, const apy
                 ov, 1.0, 0.0);
   }
   g[q - 1].gauss3m = g[q - 2].gauss3m = g3;
-  // shared integrals: the t1 of the nb vectors stacked (sp_t1_stack) into one Q1 product of nb*o rows, and
+  // shared integrals: the t1 of the nb vectors stacked (sp_prep_kernel) into one Q1 product of nb*o rows, and
   // the w4 product taken from the T half of TU, rows (q,i), with w4t [b][a][(j,c)] as a sum over b
   const bool stack = !S && nb > 1;
   const bool w4t = !S && use_w4t;
