@@ -171,7 +171,7 @@ __global__ __launch_bounds__(256) void build_block(Src src, int kind, int64_t O,
   }
 }
 
-// The four large blocks of <pq||rs> from spatial MO integrals.  For one spatial pair (P, Q) the block's
+// The four large blocks of <pq||rs> from spatial MO integrals, where they are large (launch_pair_rows).  For one spatial pair (P, Q) the block's
 // rows are the matrix M[x][y] = (Px|Qy) = E[P][x][Q][y] and its transpose:
 //   <pq||rs> = d(p,r) d(q,s) M[R][S] - d(p,s) d(q,r) M[S][R]   (spins; capitals: p/2).
 // One workgroup takes a pair (P, Q) and a 32 x 32 tile of (R, S): it reads the tile of M and the mirrored
@@ -262,16 +262,26 @@ __global__ __launch_bounds__(256) void build_pair_rows(const double2* __restrict
   }
 }
 
+// The rows form takes a block of N elements from N >= from + 1000 per workgroup on.  Below it the fill of
+// the tiles and the passes over the spin pairs (7 to 13 us whatever the size) or the padding of few occupied
+// orbitals to 32 cost more than one thread an element does, us elementwise / rows:
+//   vvvv_p  m = 16, O = 4  5.1 / 11.2   m = 24, O = 10   9.7 / 13.1   m = 32, O = 20  14.9 / 14.3   m = 48, O = 20  100 / 46
+//   ring    m = 16, O = 4  3.7 / 6.8    m = 36, O = 20   7.7 / 9.4    m = 40, O = 20   9.4 / 9.4    m = 48, O = 20  13.5 / 10.4
+//   vvvo_p  m = 16, O = 4  3.6 / 7.4    m = 48, O = 4   15.6 / 22.2   m = 32, O = 20   9.8 / 9.4    m = 48, O = 20  36.5 / 20.7
+//   vovv_p  m = 16, O = 4  3.5 / 10.3   m = 36, O = 20  15.2 / 16.0   m = 40, O = 20  21.0 / 17.6   m = 48, O = 10  29.0 / 20.4
 template <int KIND>
-int launch_pair_rows(const double2* E, int64_t m, int64_t O, int64_t V, void* out, hipStream_t st) {
-  if (!out || kind_size(KIND, O, V) <= 0) return APY_OK;
+int launch_pair_rows(const double2* E, int64_t m, int64_t O, int64_t V, void* out, hipStream_t st, unsigned& done) {
+  const int64_t N = kind_size(KIND, O, V);
+  if (!out || N <= 0) return APY_OK;
   constexpr bool TRI = KIND == K_VVVV_P || KIND == K_VOVV, PAIR = KIND == K_VVVV_P || KIND == K_VVVO_P;
+  constexpr int64_t from = KIND == K_VVVV_P ? 500000 : KIND == K_VVVO_P ? 330000 : KIND == K_VOVV ? 1500000 : 1200000;
   const int64_t nv = m - O / 2, no = (O + 1) / 2, ntv = (nv + BT - 1) / BT, nto = (no + BT - 1) / BT;
   const int64_t nq = PAIR ? nv : KIND == K_VOVV ? no : nv;
   const int64_t pairs = PAIR ? nv * (nv + 1) / 2 : nv * no, tiles = TRI ? ntv * (ntv + 1) / 2 : ntv * nto;
-  if (pairs * tiles > 0x7fffffffLL) return APY_E_ARG;
+  if (pairs * tiles > 0x7fffffffLL || N < from + 1000 * pairs * tiles) return APY_OK;
   build_pair_rows<KIND><<<(unsigned)(pairs * tiles), 256, 0, st>>>(E, m, O, V, nq, TRI ? ntv : nto, (double2*)out);
   APY_LAUNCH_CHECK();
+  done |= 1u << KIND;
   return APY_OK;
 }
 
@@ -1038,13 +1048,14 @@ int apy_so_ints_from_mo(int64_t m, const void* eri_mo, const apy_so_ints* ints, 
   const int64_t O = ints->O, V = ints->V;
   hipStream_t st = (hipStream_t)stream;
   if (O < 0 || V < 0) return APY_E_ARG;
-  int s = launch_pair_rows<K_VVVV_P>(E, m, O, V, ints->vvvv_p, st);
-  if (s == APY_OK) s = launch_pair_rows<K_VVVO_P>(E, m, O, V, ints->vvvo_p, st);
-  if (s == APY_OK) s = launch_pair_rows<K_VOVV>(E, m, O, V, ints->vovv_p, st);
-  if (s == APY_OK) s = launch_pair_rows<K_RING>(E, m, O, V, ints->ring, st);
+  unsigned done = 0;
+  int s = launch_pair_rows<K_VVVV_P>(E, m, O, V, ints->vvvv_p, st, done);
+  if (s == APY_OK) s = launch_pair_rows<K_VVVO_P>(E, m, O, V, ints->vvvo_p, st, done);
+  if (s == APY_OK) s = launch_pair_rows<K_VOVV>(E, m, O, V, ints->vovv_p, st, done);
+  if (s == APY_OK) s = launch_pair_rows<K_RING>(E, m, O, V, ints->ring, st, done);
   if (s != APY_OK) return s;
   SrcMO src{E, m};
-  return build_all(src, ints, 0, 0.0, st, 1u << K_VVVV_P | 1u << K_VVVO_P | 1u << K_VOVV | 1u << K_RING);
+  return build_all(src, ints, 0, 0.0, st, done);
 }
 
 int apy_synth_so_ints(uint64_t seed, uint64_t tag, double sd, int accumulate, double scale, int real_only,

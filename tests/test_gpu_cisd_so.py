@@ -50,12 +50,13 @@ def test_blocks_from_mo_spin_expansion(dev, m, Osp):
     assert np.array_equal(f_so, transforms.compute_F_SO_loop(f_mo))
 
 
-@pytest.mark.parametrize("m,Osp", [(2, 1), (33, 3), (40, 7), (70, 4), (36, 70)])
+@pytest.mark.parametrize("m,Osp", [(2, 1), (33, 3), (40, 7), (70, 4), (36, 70), (44, 19), (48, 22), (65, 71)])
 def test_blocks_from_mo_at_tile_edges(dev, m, Osp):
     """The spin-expanded blocks of apy_so_ints_from_mo against those of apy_so_ints_from_full (the general
     element-wise path) on the expanded tensor: virtual spaces below, at and past one and two 32-wide spatial
-    tiles, an odd number of occupied spin orbitals, more than 32 occupied spatial orbitals.  Copies and
-    single differences: equal."""
+    tiles, an odd number of occupied spin orbitals, more than 32 occupied spatial orbitals, each block on
+    either side of the size from which its rows are built by spatial pairs.  Copies and single differences:
+    equal."""
     n = 2 * m
     g = torch.Generator(device=dev).manual_seed(m)
     E = torch.randn((m,) * 4, dtype=torch.complex128, device=dev, generator=g)
