@@ -18,7 +18,8 @@
 // Two kernels per step cover every instance.  nc_z_kernel forms
 // W_ij[(ab)] = -Z_ij + Z_ji, Z_ij = sum_m Foo(m,j) x_im, for the pairs i<j: a
 // workgroup takes one (instance, slab of the (a<b) pairs) with a thread to each
-// (i, pair) and joins the two orders in LDS.  ncp_step_kernel then gives a
+// (i, pair) and joins the two orders in LDS (past O = 47 a wave takes a tile of
+// the pairs i<j instead).  ncp_step_kernel then gives a
 // workgroup one (instance, pair i<j, tile pair A <= B of the virtual plane): it
 // forms Y_ij[a,b] - Y_ij[b,a] over the tile on the FP64 matrix cores with
 // K = e staged in 8-wide chunks through LDS (the tile's rows of x_ij expanded
@@ -52,18 +53,24 @@ struct Item {
 };
 
 // The slab of W that a work item forms in LDS: SP pairs (ab) by all (i<j), at most one thread an (i, ab);
-// 0: it does not fit (O > 66), BLK pairs (ab) an item then.
+// 0: LDS holds fewer than two (O > 47), an item is four WT x WT tiles of pairs (i<j) by 64 pairs (ab) then.
+// us a step, slab / tiles:  O=33 V=40, 4 instances 155 / 197   O=46 V=12, 4  130 / 153   O=46 V=40, 2  208 / 236
+//                           O=48 V=40, 2           371 / 249   O=48 V=12, 2  119 / 109   O=66 V=40, 2  828 / 404
 constexpr int SLAB = 2192;
 __host__ __device__ inline int slab_of(int64_t O) {
   const int64_t po = O * (O - 1) / 2;
   if (O < 2 || po > SLAB) return 0;
   const int64_t a = BLK / (O < BLK ? O : BLK), b = SLAB / po;
-  return (int)(a < b ? a : b);
+  return b < 2 ? 0 : (int)(a < b ? a : b);
 }
-inline int64_t zspan(int64_t O) { return slab_of(O) ? slab_of(O) : BLK; }
+constexpr int WT = 4;
+__host__ __device__ inline int64_t wtiles(int64_t O) { const int64_t nt = (O + WT - 1) / WT; return nt * (nt + 1) / 2; }
+// pairs (ab) of an item, and items of a span of them
+inline int64_t zspan(int64_t O) { return slab_of(O) ? slab_of(O) : 64; }
+inline int64_t zrows(int64_t O) { return slab_of(O) ? 1 : (wtiles(O) + BLK / 64 - 1) / (BLK / 64); }
 
 struct ZItem {
-  int32_t inst, p0;
+  int32_t inst, p0, t0, pad;   // first pair (ab), first tile of pairs (ij)
 };
 
 struct Header {
@@ -118,7 +125,7 @@ int64_t count_zitems(int n, const apy_mp2_nc_instance* inst, int64_t* zelems) {
   for (int k = 0; k < n; ++k) {
     if (inst[k].O < 2 || inst[k].V < 2) continue;
     const int64_t Pv = npair(inst[k].V);
-    z += (Pv + zspan(inst[k].O) - 1) / zspan(inst[k].O);
+    z += (Pv + zspan(inst[k].O) - 1) / zspan(inst[k].O) * zrows(inst[k].O);
     e += npair(inst[k].O) * Pv;
   }
   if (zelems) *zelems = e;
@@ -243,6 +250,65 @@ __device__ __forceinline__ void w_slab(SF Fr, const double2* __restrict__ x, dou
   }
 }
 
+// W_(i<j)[P] of a WT x WT tile of pairs (ij) and 64 pairs P a wave: 2 WT rows of x and as many elements of Foo
+// (scalar: the tile is the wave's) a value of m for 2 WT^2 complex products, all sums in registers.  Bound by
+// the reads of x, each row from L2 once a tile.  One thread an element of W ran on the few workgroups that 256
+// pairs P an item left: O=68 V=40, two instances, 111 ms a step, 0.42 ms so.
+template <bool TF>
+__device__ __forceinline__ void w_tile(SF Fr, const double2* __restrict__ x, double2* __restrict__ W, int O, int n,
+                                       int64_t Pv, int64_t P, int t) {
+  if (t >= wtiles(O)) return;
+  const int nt = (O + WT - 1) / WT;
+  int ti = 0;
+  while (t >= nt - ti) { t -= nt - ti; ++ti; }
+  const int i0 = ti * WT, j0 = (ti + t) * WT;
+  const bool in = P < Pv;
+  const double2* xp = x + (in ? P : 0);
+  double2 acc[WT][WT];
+#pragma unroll
+  for (int a = 0; a < WT; ++a)
+#pragma unroll
+    for (int b = 0; b < WT; ++b) acc[a][b] = make_double2(0.0, 0.0);
+  // x_pm[P], p past the end: the last row, whose sums are not taken
+  auto row = [&](int p, int m) {
+    p = min(p, O - 1);
+    const int64_t r = p < m ? pidx(p, m, O) : p > m ? pidx(m, p, O) : 0;
+    double2 v = xp[r * Pv];
+    v.x = p == m ? 0.0 : p > m ? -v.x : v.x;
+    v.y = p == m ? 0.0 : p > m ? -v.y : v.y;
+    return v;
+  };
+  auto foo = [&](int m, int p) {
+    p = min(p, O - 1);
+    const SF f = Fr + 2 * (TF ? (int64_t)p * n + m : (int64_t)m * n + p);
+    return make_double2(f[0], f[1]);
+  };
+  for (int m = 0; m < O; ++m) {
+    double2 xi[WT], xj[WT], fi[WT], fj[WT];
+#pragma unroll
+    for (int a = 0; a < WT; ++a) {
+      xi[a] = row(i0 + a, m);
+      xj[a] = row(j0 + a, m);
+      fi[a] = foo(m, i0 + a);
+      fj[a] = foo(m, j0 + a);
+      fj[a] = make_double2(-fj[a].x, -fj[a].y);
+    }
+#pragma unroll
+    for (int a = 0; a < WT; ++a)
+#pragma unroll
+      for (int b = 0; b < WT; ++b) {
+        cfma(acc[a][b], fi[a], xj[b]);
+        cfma(acc[a][b], fj[b], xi[a]);
+      }
+  }
+  if (!in) return;
+#pragma unroll
+  for (int a = 0; a < WT; ++a)
+#pragma unroll
+    for (int b = 0; b < WT; ++b)
+      if (i0 + a < j0 + b && j0 + b < O) W[pidx(i0 + a, j0 + b, O) * Pv + P] = acc[a][b];
+}
+
 // W_k[(i<j)][(ab)] = sum_m (Foo(m,i) x_jm - Foo(m,j) x_im)[(ab)] for every instance and slice of pairs
 // (ab) (grid-stride over the work list, whose length is in the header).
 __device__ __forceinline__ void nc_z_phase(char* __restrict__ ws, const apy_mp2_nc_instance* __restrict__ insts,
@@ -264,27 +330,10 @@ __device__ __forceinline__ void nc_z_phase(char* __restrict__ ws, const apy_mp2_
     const SF Fr = (SF)((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)fp) |
                        (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(fp >> 32)) << 32);
     const int SP = slab_of(O);
-    if (SP == 0) {                                     // more pairs (ij) than LDS holds: an element a thread
-      const double2* F = (const double2*)I.fock;
-      auto foo = [&](int m, int j) { return I.transpose_f ? F[(int64_t)j * n + m] : F[(int64_t)m * n + j]; };
-      const int64_t P = it.p0 + threadIdx.x;
-      if (threadIdx.x >= BLK || P >= Pv) continue;
-      for (int64_t r = 0; r < npair(O); ++r) {
-        int64_t i, j;
-        pdec(r, O, i, j);
-        double2 z = make_double2(0.0, 0.0);
-        for (int m = 0; m < O; ++m) {
-          if (m != i) {
-            const double2 v = x[pidx(i < m ? i : m, i < m ? m : i, O) * Pv + P];
-            cfma(z, foo(m, (int)j), i < m ? make_double2(-v.x, -v.y) : v);
-          }
-          if (m != j) {
-            const double2 v = x[pidx(j < m ? j : m, j < m ? m : j, O) * Pv + P];
-            cfma(z, foo(m, (int)i), j < m ? v : make_double2(-v.x, -v.y));
-          }
-        }
-        W[r * Pv + P] = z;
-      }
+    if (SP == 0) {                                     // a tile of pairs (ij) a wave
+      const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+      if (I.transpose_f) w_tile<true>(Fr, x, W, O, n, Pv, it.p0 + (int64_t)(threadIdx.x & 63), it.t0 + wave);
+      else w_tile<false>(Fr, x, W, O, n, Pv, it.p0 + (int64_t)(threadIdx.x & 63), it.t0 + wave);
       continue;
     }
     __syncthreads();                                   // the slab of the previous item is written out
@@ -765,7 +814,9 @@ int apy_mp2_nc_batched_setup(int n, const apy_mp2_nc_instance* inst, void* works
     for (int32_t p = 0; p < (int32_t)npair(inst[k].O); ++p)
       for (int32_t ta = 0; ta < nt; ++ta)
         for (int32_t tb = ta; tb < nt; ++tb) it.push_back(Item{k, p, ta, tb});
-    for (int64_t p0 = 0; p0 < Pv; p0 += zspan(inst[k].O)) zit.push_back(ZItem{k, (int32_t)p0});
+    for (int64_t p0 = 0; p0 < Pv; p0 += zspan(inst[k].O))
+      for (int64_t r = 0; r < zrows(inst[k].O); ++r)
+        zit.push_back(ZItem{k, (int32_t)p0, (int32_t)(r * (BLK / 64)), 0});
     zoff[k + 1] = zoff[k] + npair(inst[k].O) * Pv;
   }
   off[n] = (int64_t)it.size();

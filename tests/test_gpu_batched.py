@@ -198,6 +198,45 @@ def test_batched_step_at_tile_edges(dev, O, V, transpose):
     assert abs(b.rnorm[0] - rr) < 1e-12 * rr
 
 
+@pytest.mark.parametrize("O,V", [(47, 5), (48, 5), (66, 5), (67, 12), (70, 24)])
+@pytest.mark.parametrize("transpose", [False, True])
+def test_batched_step_past_the_slab(dev, O, V, transpose):
+    """The largest occupied space that takes the rows of W through LDS, and those past it (tiles of 4 x 4 pairs by
+    64 pairs (ab): no remainder and one of 2 and 3 rows, one span and more)."""
+    test_batched_step_at_tile_edges(dev, O, V, transpose)
+
+
+def _us(fn, n=5):
+    """Least device time of fn in microseconds over n runs."""
+    fn()
+    best = float("inf")
+    for _ in range(n):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        fn()
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, 1e3 * a.elapsed_time(b))
+    return best
+
+
+def _random_batch(dev, O, V, seed=3):
+    g = torch.Generator(device=dev).manual_seed(seed)
+    cn = lambda *sh: torch.randn(*sh, dtype=torch.complex128, device=dev, generator=g)
+    eps = torch.cat([-2.0 + torch.rand(O, dtype=torch.float64, device=dev, generator=g),
+                     1.0 + torch.rand(V, dtype=torch.float64, device=dev, generator=g)])
+    b = MP2NCBatch([Instance(O, V, cn(O + V, O + V), eps, cn(O * O * V * V), cn(O * O * V * V))])
+    b._xbuf.copy_(cn(b._xbuf.numel()))
+    return b
+
+
+def test_step_time_past_the_slab(dev):
+    """O = 68 is 3.2 times the work of O = 46 (O (i<j) (a<b) sums): a step past the slab takes no multiple of that
+    (hundreds of times, when 256 pairs (ab) were an item whatever their number)."""
+    fits, past = _random_batch(dev, 46, 12), _random_batch(dev, 68, 12)
+    assert _us(lambda: past.step(0)) < 10 * _us(lambda: fits.step(0))
+
+
 def test_packed_storage_round_trip_and_warm_start(dev):
     """The packed amplitudes expand to the antisymmetric dense tensor and
     pack back exactly; a batch started from converged amplitudes stays at
