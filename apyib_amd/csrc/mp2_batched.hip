@@ -633,9 +633,11 @@ __device__ inline void pdec_near(int64_t P, int N, int& p, int& q) {
 
 // energy[k] = scale * sum_dense w_k x_k = 4 scale * sum_(i<j, a<b) w_k x_k (w and x
 // antisymmetric), in two fixed-order passes: EN_B partial sums per instance
-// (blockIdx.y = instance; a block takes every EN_B-th row (i<j), so a division and a double root an
-// element, 90 us for 36 instances of O 14-18 V 54-66, are one float root), then one block per instance
-// adds its partials.
+// (blockIdx.y = instance), then one block per instance adds its partials.  A pair index is one float root
+// (a division and a double root an element took 90 us for 36 instances of O 14-18 V 54-66, 53 us so).  Rows
+// of BLK pairs (ab) and more are cut where half the blocks would have none (45 rows: 13.2 us whole, 15.8 cut); of shorter ones a block takes
+// several side by side, a thread keeping its pair (one row a block at a time: O=2 V=200, two instances, 60 us,
+// 10 us so; O=68 V=12, four, 62 us, 17 us so).
 __global__ __launch_bounds__(BLK) void nc_energy_partial(const apy_mp2_nc_instance* __restrict__ insts, int use_x_new,
                                                          double2* __restrict__ epart) {
   __shared__ double2 red[BLK];
@@ -644,18 +646,30 @@ __global__ __launch_bounds__(BLK) void nc_energy_partial(const apy_mp2_nc_instan
   const double2* x = (const double2*)(use_x_new ? I.x_new : I.x);
   const int64_t O = I.O, V = I.V, Pv = npair(V), Po = npair(O);
   double2 acc = make_double2(0.0, 0.0);
-  if (w)
-    for (int64_t r = blockIdx.x; r < Po; r += EN_B) {
-      int64_t i, j;
-      pdec(r, O, i, j);
+  if (w && Po > 0 && Pv >= BLK) {
+    const int64_t cuts = 2 * Po <= EN_B ? (Pv + BLK - 1) / BLK : 1, len = cuts > 1 ? BLK : Pv;
+    for (int64_t u = blockIdx.x; u < Po * cuts; u += EN_B) {
+      const int64_t r = u / cuts, p0 = (u - r * cuts) * len;
+      int i, j;
+      pdec_near(r, (int)O, i, j);
       const double2* wr = w + (i * O + j) * V * V;
       const double2* xr = x + r * Pv;
-      for (int64_t P = threadIdx.x; P < Pv; P += BLK) {
+      for (int64_t P = p0 + threadIdx.x; P < min(p0 + len, Pv); P += BLK) {
         int a, b;
         pdec_near(P, (int)V, a, b);
         cfma(acc, wr[a * V + b], xr[P]);
       }
     }
+  } else if (w && Po > 0 && Pv > 0) {
+    const int pv = (int)Pv, rows = BLK / pv, row = threadIdx.x / pv, P = threadIdx.x % pv;
+    int a, b;
+    pdec_near(P, (int)V, a, b);
+    for (int64_t r = (int64_t)blockIdx.x * rows + row; row < rows && r < Po; r += (int64_t)EN_B * rows) {
+      int i, j;
+      pdec_near(r, (int)O, i, j);
+      cfma(acc, w[((i * O + j) * V + a) * V + b], x[r * Pv + P]);
+    }
+  }
   red[threadIdx.x] = acc;
   __syncthreads();
   for (int q = BLK / 2; q > 0; q >>= 1) {

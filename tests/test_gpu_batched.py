@@ -237,6 +237,36 @@ def test_step_time_past_the_slab(dev):
     assert _us(lambda: past.step(0)) < 10 * _us(lambda: fits.step(0))
 
 
+@pytest.mark.parametrize("O,V", [(2, 2), (2, 23), (2, 24), (2, 200), (3, 90), (12, 23), (12, 24), (23, 24),
+                                 (24, 30), (40, 7), (70, 3)])
+def test_energies_at_row_edges(dev, O, V):
+    """The energies against the dense sum: rows of pairs (ab) below, at and past the 256 threads of a block
+    (V = 23 | 24), few and many rows of either.  A sum of N products of order one in another order."""
+    g = torch.Generator(device=dev).manual_seed(O * V)
+    cn = lambda *sh: torch.randn(*sh, dtype=torch.complex128, device=dev, generator=g)
+
+    def anti(x):
+        x = x - x.transpose(0, 1)
+        return x - x.transpose(2, 3)
+
+    n = O + V
+    eps = torch.linspace(-2.0, 2.0, n, dtype=torch.float64, device=dev)
+    w, x = anti(cn(O, O, V, V)), anti(cn(O, O, V, V))
+    other = Instance(4, 6, cn(10, 10), eps[:1].expand(10), cn(16 * 36), cn(16 * 36))
+    b = MP2NCBatch([other, Instance(O, V, cn(n, n), eps, cn(O * O * V * V), w.reshape(-1))])
+    b.start_from(1, x)
+    got = b.energies(scale=1.0)[1]
+    want = (w * x).sum()
+    assert abs(got - want) <= 1e-15 * (1.0 + (w.abs() * x.abs()).sum())
+
+
+def test_energy_time_of_few_rows(dev):
+    """Two occupied orbitals are one row of pairs (ab), which the blocks share: its 19900 products take no multiple
+    of the time of a small instance's (six times, when a row was one block's)."""
+    one_row, small = _random_batch(dev, 2, 200), _random_batch(dev, 10, 4)
+    assert _us(lambda: one_row.energies(), 9) < 3 * _us(lambda: small.energies(), 9)
+
+
 def test_packed_storage_round_trip_and_warm_start(dev):
     """The packed amplitudes expand to the antisymmetric dense tensor and
     pack back exactly; a batch started from converged amplitudes stays at
