@@ -880,7 +880,11 @@ int apy_mp2_nc_batched_solve(int n, int64_t n_items, double tol, int maxit, void
   APY_HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
   APY_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, nc_persistent_kernel, SBLK, 0));
   if (per_cu < 1 || ncu < 1) return APY_E_HIP;
-  // every workgroup resident at once (a cooperative launch refuses a larger grid)
+  // every workgroup resident at once (a cooperative launch refuses a larger grid), and no more of them than the
+  // items pay for: a grid barrier takes about 0.08 us a workgroup, three an iteration.  ms a solve at 1 / 2 / 3 a
+  // CU: O=10 V=4, 1080 items 0.53 / 0.89 / 1.26; O=10 V=38, 3240 items 1.23 / 1.48 / 1.90; 36 instances of
+  // O 14-18 V 54-66, 15000 items 5.89 / 4.62 / 4.70.
+  per_cu = std::min(per_cu, n_items > 24 * (int64_t)ncu ? 2 : 1);
   const int64_t grid = std::min<int64_t>((int64_t)per_cu * ncu, n_items);
   const apy_mp2_nc_instance* insts = (const apy_mp2_nc_instance*)(w + L.inst);
   const Item* items = (const Item*)(w + L.item);

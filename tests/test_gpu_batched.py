@@ -310,6 +310,17 @@ def test_persistent_solve_equals_direct_launches(dev, tol, maxit):
     assert torch.equal(d.rnorm, p.rnorm)
 
 
+@pytest.mark.parametrize("count", [1, 11, 12])
+def test_persistent_solve_at_the_grid_rule(dev, count):
+    """Fewer items than compute units, and either side of 24 items each (528 pairs an instance), where the launch
+    takes one or two workgroups a compute unit: the direct launches' iterates bit for bit."""
+    insts = (fd_mp2_instances(33, 4, 5, 2, device=dev)[0] * 2)[:count]
+    a, b = MP2NCBatch(insts), MP2NCBatch(insts)
+    ita, itb = a.solve(tol=1e-10, maxit=60), b.solve(tol=1e-10, maxit=60, persistent=True)
+    assert ita == itb
+    assert torch.equal(a._xbuf, b._xbuf)
+
+
 def test_persistent_solve_set_b_sizes(dev):
     """The 36-instance uneven set at its own sizes (O 14-18, V 54-66): the
     persistent solve against the direct launches, bit for bit."""
