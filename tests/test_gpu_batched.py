@@ -378,6 +378,29 @@ def test_adjoint_sums_match_separate_densities_and_dots(dev):
             assert abs(out[b][q] - want) <= 1e-12 * max(1.0, abs(want)), (b, q)
 
 
+def test_adjoint_sums_of_many_directions(dev):
+    """More directions than one launch combines, the cut inside an item, an item without directions between, and
+    arrays shared within an item and across items, against torch sums of the three terms."""
+    from apyib_amd.batched import mp2_adjoint_set
+    bases = [_host_instance(O, V, 90 + k, dev)[0] for k, (O, V) in enumerate([(3, 4), (2, 5), (3, 4), (2, 3)])]
+    g = torch.Generator(device=dev).manual_seed(6)
+    rnd = lambda n: torch.randn(n, generator=g, dtype=torch.complex128, device=dev)
+    pool = {n: [rnd(n) for _ in range(5)] for n in {(B.O + B.V) ** 2 for B in bases} | {(B.O * B.V) ** 2 for B in bases}}
+    directions = []
+    for b, (B, K) in enumerate(zip(bases, (200, 0, 90, 7))):
+        n, d2 = (B.O + B.V) ** 2, (B.O * B.V) ** 2
+        directions.append(([pool[n][q * 3 % 5] for q in range(K)], [pool[d2][q % 2] for q in range(K)] if b else None,
+                           [pool[d2][0] if q % 7 else rnd(d2) for q in range(K)]))
+    out, dens = mp2_adjoint_set(bases, directions, tol=1e-13)
+    for b, (dF, dW, dV) in enumerate(directions):
+        G, t, lam = dens[b]
+        assert len(out[b]) == len(dF)
+        for q in range(len(dF)):
+            terms = [(G, dF[q], 1.0), (t, dW[q] if dW is not None else torch.zeros_like(t), 0.25), (lam, dV[q], 1.0)]
+            want = complex(sum(c * torch.sum(x.reshape(-1) * y.reshape(-1)) for x, y, c in terms).cpu())
+            assert abs(out[b][q] - want) <= 1e-12 * max(1.0, abs(want)), (b, q)
+
+
 def test_adjoint_hermitian_lambda_matches_solved_lambda(dev):
     """mp2_adjoint_set(hermitian=True) (amplitudes only, lambda = conj(t)/4
     inside apy_mp2_adjoint_sums) against the solved lambda equations on
