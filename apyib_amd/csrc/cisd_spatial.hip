@@ -348,6 +348,12 @@ constexpr int SET = 32;  // edge of the (a, b) tile of the doubles epilogue
 // a > b half of the ladder) are summed while reading them along a, into one LDS tile, and read
 // back along b; every other operand is read along b directly.  All global reads and writes are
 // along the contiguous index.
+//
+// AHEAD: all reads of a pass are issued before the first is used, past the edge and outside the packed halves
+// at a place inside: under conditions they follow each other at a read's latency (16 us for the 81 tiles of
+// o=9 v=25).  That takes 256 registers, one wave a SIMD; with more tiles than the six waves a SIMD of the
+// other form hold at once those hide the latency and read faster (SP_AHEAD_TILES).
+template <bool AHEAD>
 __device__ __forceinline__ void sp_epi_doubles(const SpEpi& e) {
   __shared__ double2 T[SET][SET + 1];  // T[b - b0][a - a0]: the transposed terms of output (a, b)
   const int64_t o = e.o, v = e.v, ov = o * v, vv = v * v, per = ov * ov;
@@ -372,11 +378,41 @@ __device__ __forceinline__ void sp_epi_doubles(const SpEpi& e) {
     const double2* Q1 = e.Q1 ? e.Q1 + qd : nullptr;
     const double2* Q2 = e.Q2 ? e.Q2 + qd : nullptr;
     __syncthreads();  // T of the previous tile is no longer read
-    // element (b, a) = (b0 + ty + 8k, a0 + tx), read along a.  All reads of a pass are issued before the
-    // first is used, past the edge and outside the packed halves at a place inside: under conditions they
-    // followed each other at a read's latency (16 us for the 81 tiles of o=9 v=25).
+    // element (b, a) = (b0 + ty + 8k, a0 + tx), read along a
     constexpr int NK = SET / 8;
-    {
+    if constexpr (!AHEAD) {
+#pragma unroll
+      for (int k = 0; k < NK; ++k) {
+        const int64_t b = b0 + ty + 8 * k, a = a0 + tx;
+        double2 s = make_double2(0.0, 0.0);
+        if (a < v && b < v) {
+          const double2 x1t = X1[(j * v + b) * ov + i * v + a];
+          const double2 x2 = X2[(i * v + b) * ov + j * v + a];
+          s.x = x1t.x - x2.x;
+          s.y = x1t.y - x2.y;
+          if (Y) {
+            const double2 y2 = Y[((j * o + i) * v + b) * v + a];
+            s.x += y2.x;
+            s.y += y2.y;
+          }
+          if (Q1) {
+            const double2 q1t = Q1[j * (o * vv) + (i * v + b) * v + a];
+            const double2 q2t = Q2[((j * o + i) * v + b) * v + a];
+            s.x += q1t.x - q2t.x;
+            s.y += q1t.y - q2t.y;
+          }
+          if (b < a) {
+            const double2 ps = Ps[isym(b, a, v)];
+            s.x += ps.x; s.y += ps.y;
+            if (Pa) {
+              const double2 pa = Pa[ianti(b, a, v)];
+              s.x += sgn_lower * pa.x; s.y += sgn_lower * pa.y;
+            }
+          }
+        }
+        T[ty + 8 * k][tx] = s;
+      }
+    } else {
       double2 x1t[NK], x2[NK], y2[NK], q1t[NK], q2t[NK], ps[NK], pa[NK];
 #pragma unroll
       for (int k = 0; k < NK; ++k) {
@@ -409,6 +445,52 @@ __device__ __forceinline__ void sp_epi_doubles(const SpEpi& e) {
     const double* ep = e.eps + q * e.s_eps;
     const double eij = ep[i] + ep[j];
     const double2 rsc = e.rb ? resp_scalar(e.re, e.rs, e.es, q) : make_double2(0.0, 0.0);
+    if constexpr (!AHEAD) {
+#pragma unroll
+      for (int k = 0; k < NK; ++k) {
+        const int64_t a = a0 + ty + 8 * k, b = b0 + tx;
+        if (a >= v || b >= v) continue;
+        const int64_t t = ((i * o + j) * v + a) * v + b;
+        double2 rr = e.vvoo[q * e.s_vvoo + t];
+        const double2 tt = T[tx][ty + 8 * k];
+        const double2 p = e.R[qd + t];
+        const double2 x1 = X1[(i * v + a) * ov + j * v + b];
+        const double2 x2t = X2[(j * v + a) * ov + i * v + b];
+        rr.x += tt.x + p.x + x1.x - x2t.x;
+        rr.y += tt.y + p.y + x1.y - x2t.y;
+        if (Y) {
+          const double2 y1 = Y[t];
+          rr.x += y1.x;
+          rr.y += y1.y;
+        }
+        if (Q1) {
+          const double2 q1 = Q1[i * (o * vv) + (j * v + a) * v + b];
+          const double2 q2 = Q2[t];
+          rr.x += q1.x - q2.x;
+          rr.y += q1.y - q2.y;
+        }
+        if (a <= b) {
+          const double2 ps = Ps[isym(a, b, v)];
+          rr.x += ps.x; rr.y += ps.y;
+          if (Pa && a < b) {
+            const double2 pa = Pa[ianti(a, b, v)];
+            rr.x -= sgn_lower * pa.x; rr.y -= sgn_lower * pa.y;
+          }
+        }
+        const double2 x = e.t2[qv + t];
+        rr.x -= E.x * x.x - E.y * x.y;
+        rr.y -= E.x * x.y + E.y * x.x;
+        if (e.rb) {
+          const double2 bb = e.rb[qv + t], y = e.rt[t];
+          rr.x += bb.x - (rsc.x * y.x - rsc.y * y.y);
+          rr.y += bb.y - (rsc.x * y.y + rsc.y * y.x);
+        }
+        const double D = eij - ep[o + a] - ep[o + b];
+        e.r2[qv + t] = rr;
+        e.t2_new[qv + t] = make_double2(x.x + rr.x / D, x.y + rr.y / D);
+      }
+      continue;
+    }
     // output (a, b) = (a0 + ty + 8k, b0 + tx), read along b
     double2 vo[NK], p[NK], x1[NK], x2t[NK], y1[NK], q1[NK], q2[NK], ps[NK], pa[NK], x[NK], rbv[NK], rtv[NK];
     double ea[NK];
@@ -485,13 +567,20 @@ __device__ __forceinline__ void sp_epi_singles(const SpEpi& e, int64_t u) {
   e.t1_new[qv + t] = make_double2(x.x + r.x / D, x.y + r.y / D);
 }
 
+// Tiles up to which the reads go ahead: one round of the other form's workgroups (256 CUs, six each).  us a step,
+// ahead / not:  162 tiles (o=9 v=25, 2 vectors) 57.5 / 66.6   375 (o=5 v=13, 15) 46.7 / 47.2   900 (o=10 v=80) 514 / 514
+//               1600 (o=20 v=60) 1123 / 1131   1800 (o=10 v=80, 2, CID) 884 / 877   3600 (4) 1707 / 1694
+//               13500 (15) 6182 / 6082
+constexpr int32_t SP_AHEAD_TILES = 6 * 256;
+
 // Both epilogues in one launch: neither reads what the other writes.
+template <bool AHEAD>
 __global__ __launch_bounds__(256) void sp_epi_kernel(SpEpi e) {
   if ((int)blockIdx.x >= e.doubles) {
     sp_epi_singles(e, (int64_t)((int)blockIdx.x - e.doubles) * 256 + threadIdx.x);
     return;
   }
-  sp_epi_doubles(e);
+  sp_epi_doubles<AHEAD>(e);
 }
 
 constexpr int EN_BLOCKS = 256;
@@ -767,7 +856,8 @@ int sp_step_impl(const apy_cisd_sp_args* A, int64_t nb, const void* resp_shift, 
           (double2*)A->t_new, (double2*)A->out, 0};
   const int64_t nt = (v + SET - 1) / SET, ns = (nb * ov + 255) / 256;
   e.doubles = (int32_t)std::min<int64_t>(nb * o * o * nt * nt, 1 << 20);
-  sp_epi_kernel<<<(unsigned)(e.doubles + ns), 256, 0, st>>>(e);
+  if (e.doubles <= SP_AHEAD_TILES) sp_epi_kernel<true><<<(unsigned)(e.doubles + ns), 256, 0, st>>>(e);
+  else sp_epi_kernel<false><<<(unsigned)(e.doubles + ns), 256, 0, st>>>(e);
   APY_LAUNCH_CHECK();
   return APY_OK;
 }

@@ -155,6 +155,46 @@ def test_batched_step_and_energy_match_single_calls(dev, singles):
         assert abs(energies[q].item() - e1) < 1e-13 * max(1.0, abs(e1))
 
 
+@pytest.mark.parametrize("nb", [24, 25])
+@pytest.mark.parametrize("singles,fold", [(True, True), (True, False), (False, True)])
+def test_batched_step_at_the_epilogue_rule(dev, nb, singles, fold):
+    """64 tiles of (a, b) a vector (two 32-wide ones a side, the second with one row): 24 vectors are the last whose
+    epilogue issues its reads ahead, 25 take the other form.  Against one step a vector, and updated in place
+    bit for bit; two orders of sums of up to o v^2 terms."""
+    import ctypes
+    from apyib_amd import _lib
+    from apyib_amd.kernels import stream_of, workspace
+    lib = _lib.load()
+    o, v = 4, 33
+    g = torch.Generator(device=dev).manual_seed(9)
+    cn = lambda *sh: torch.randn(*sh, dtype=torch.complex128, device=dev, generator=g)
+    E4 = 0.1 * cn(o + v, o + v, o + v, o + v)
+    E4 = 0.5 * (E4 + E4.permute(2, 3, 0, 1))
+    eps = np.concatenate([np.linspace(-2.0, -1.0, o), np.linspace(0.5, 3.0, v)])
+    F = torch.diag(torch.from_numpy(eps).to(dev)) + 0.01 * cn(o + v, o + v)
+    ci = SpatialCI(SPIntegrals.from_mo(E4.contiguous(), o, singles=singles), F, eps, singles=singles)
+    X, B, rt = cn(nb, ci.L), cn(nb, ci.L), cn(ci.L)
+    en, re = 0.1 * cn(nb), 0.1 * cn(nb)
+
+    def step(x, xn, r, b, e, s, n):
+        a = _args(ci, x, xn, r, e, b, rt, s)
+        a.w21_f = ci.w21_f.data_ptr() if fold else None
+        nbytes = int(lib.apy_cisd_sp_batch_workspace(o, v, int(singles), n))
+        ws = workspace(nbytes, dev)
+        assert lib.apy_cisd_sp_step_batch(ctypes.byref(a), n, None, ctypes.c_void_p(ws.data_ptr()), nbytes,
+                                          stream_of(dev)) == 0
+
+    R, Xn, R2, X2 = torch.zeros_like(X), torch.zeros_like(X), torch.zeros_like(X), X.clone()
+    step(X, Xn, R, B, en, re, nb)
+    step(X2, X2, R2, B, en, re, nb)
+    assert torch.equal(R, R2) and torch.equal(Xn, X2)
+    for q in range(0, nb, 4):
+        xn, r = torch.zeros_like(rt), torch.zeros_like(rt)
+        step(X[q].clone(), xn, r, B[q].clone(), en[q:q + 1].clone(), re[q:q + 1].clone(), 1)
+        assert (R[q] - r).abs().max() < 1e-13 * r.abs().max()
+        assert (Xn[q] - xn).abs().max() < 1e-13 * xn.abs().max()
+
+
 @pytest.mark.parametrize("singles", [True, False])
 def test_response_set_matches_single_solves(dev, singles):
     """Three perturbations iterated as one ResponseSet against three
