@@ -867,24 +867,31 @@ bool group_plan(const apy_gemm_desc* d, int n, Group& G) {
     of[i] = t;
   }
   // Tile by padding, then K slices that give every block the same work.
-  bool g3 = false;
-  for (int i = 0; i < n; ++i) g3 = g3 || (!G.alone[i] && d[i].gauss3m);
+  auto padded = [&](int i, int t) {
+    const GroupTile& g = GROUP_TILES[t];
+    return (double)((d[i].m + g.bm - 1) / g.bm * g.bm) * ((d[i].n + g.bn - 1) / g.bn * g.bn) / g.eff;
+  };
+  // Three real products instead of four on the 64 x 64 tile, unless another tile with the four pads less by more
+  // than that saves: us a step in the three-product form, 64 x 64 / so  O=4 V=150 (6 rows) 1012 / 515
+  // O=6 V=100 (15 rows) 255 / 171   O=8 V=100 (28 rows) 314 / 258
+  bool g3 = false, use3[GROUP_MAX];
+  for (int i = 0; i < n; ++i) {
+    use3[i] = !G.alone[i] && d[i].gauss3m;
+    for (int t = 1; t < NTILE; ++t) use3[i] = use3[i] && 0.75 * padded(i, 0) <= padded(i, t);
+    g3 = g3 || use3[i];
+  }
   int kind[GROUP_MAX];
   double area[GROUP_MAX], T = 0.0;
   for (int i = 0; i < n; ++i) {
     if (G.alone[i]) continue;
-    // the 64 x 64 tile of a G3 launch is for the products that ask for the three-product form
-    const int t0 = g3 && !d[i].gauss3m ? 1 : 0;
+    // the 64 x 64 tile of a G3 launch is for the products in the three-product form
+    const int t0 = g3 && !use3[i] ? 1 : 0;
     int best = t0;
-    double a = 0.0;
-    for (int t = t0; t < (d[i].gauss3m ? 1 : NTILE); ++t) {
-      const GroupTile& g = GROUP_TILES[t];
-      const double x = (double)((d[i].m + g.bm - 1) / g.bm * g.bm) * ((d[i].n + g.bn - 1) / g.bn * g.bn) / g.eff;
-      if (t == t0 || x < a) { best = t; a = x; }
-    }
+    for (int t = t0; t < (use3[i] ? 1 : NTILE); ++t)
+      if (padded(i, t) < padded(i, best)) best = t;
     kind[i] = (d[i].a_layout == APY_MK ? 1 : 0) | (d[i].b_layout == APY_NK ? 2 : 0) | best << 2;
     area[i] = (double)GROUP_TILES[best].bm * GROUP_TILES[best].bn / GROUP_TILES[best].eff;
-    T += a * d[i].k * d[i].batch;
+    T += padded(i, best) * d[i].k * d[i].batch;
   }
   const double slots = (g3 ? 2.0 : 3.0) * dev_info().cus, per = T / slots * GROUP_SHARE;
   double work[GROUP_MAX];
@@ -963,8 +970,8 @@ int apy_zgemm_group(const apy_gemm_desc* d, int n, void* workspace, size_t ws_by
     a.mtiles = (x.m + tile.bm - 1) / tile.bm; a.ntiles = (x.n + tile.bn - 1) / tile.bn;
     a.total = a.mtiles * a.ntiles * a.split * a.batch;
     a.ws = G.off[i] != SIZE_MAX ? (double2*)((char*)workspace + G.off[i]) : nullptr;
-    a.g3 = x.gauss3m ? 1 : 0;
-    g3 = g3 || x.gauss3m;
+    a.g3 = x.gauss3m && G.kind[i] < 4 ? 1 : 0;
+    g3 = g3 || a.g3;
     A.kind[q] = G.kind[i];
     A.start[q] = (int32_t)blocks;
     blocks += (a.total + 7) / 8 * 8;

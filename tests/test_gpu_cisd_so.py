@@ -134,6 +134,48 @@ def test_grouped_products_match_one_after_another(dev, O, V, singles, fov, fold,
         assert (x[live] - y[live]).abs().max() <= 1e-13 * max(1.0, y[live].abs().max().item())
 
 
+@pytest.mark.parametrize("O,V", [(2, 9), (4, 20), (6, 40), (8, 33), (11, 21), (12, 30)])
+@pytest.mark.parametrize("packed", [False, True])
+def test_three_product_form_by_rows(dev, O, V, packed):
+    """The three-product option against the four products where the ladder has few rows (it keeps four products
+    on a narrower tile there) and where it has enough; sums of up to V^2 / 2 terms of order one, and the
+    three-product form's two differences of them."""
+    F, eps = synthetic.fock(O, V, 5)
+    ints = SOIntegrals.synthetic(O, V, 5, device=dev)
+    ci = SOCI(ints, _dev(F, dev), eps, fov_coupling=True)
+    g = torch.Generator(device=dev).manual_seed(V)
+    x = torch.randn(ci.Lp if packed else ci.L, dtype=torch.complex128, device=dev, generator=g)
+    a, b = torch.zeros_like(x), torch.zeros_like(x)
+    ci.sigma(x, a, packed=packed)
+    ci.gauss3m = True
+    ci.sigma(x, b, packed=packed)
+    assert (a - b).abs().max() <= 1e-13 * a.abs().max()
+
+
+def test_three_product_form_of_few_rows_is_no_slower(dev):
+    """Six rows on a 64-row tile cost ten times their products: the three-product option took twice the time of
+    the four products it is meant to save."""
+    O, V = 4, 150
+    F, eps = synthetic.fock(O, V, 5)
+    ci = SOCI(SOIntegrals.synthetic(O, V, 5, device=dev), _dev(F, dev), eps, fov_coupling=True)
+    x, y = ci.new_vector(), ci.new_vector()
+
+    def us():
+        best = float("inf")
+        for _ in range(8):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            ci.sigma(x, y)
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best
+
+    four = us()
+    ci.gauss3m = True
+    assert us() < 1.3 * four
+
+
 def _system(O, V, seed, dev, brill=False):
     F, A, eps = synthetic.system(O, V, seed)
     if brill:
