@@ -803,8 +803,13 @@ int apy_zgemm_launch(const apy_gemm_desc* d, void* workspace, size_t ws_bytes, h
 // ------------------------------------------------------------ grouped products
 namespace {
 
-// A product of this size fills the chip for several rounds by itself and keeps its own (tuned) plan.
-constexpr double GROUP_ALONE_FLOP = 2.0e10;   // about 0.3 ms
+// A product of this size runs for milliseconds by itself and keeps its own (tuned) plan; below it the last round of
+// each product's blocks is filled by the next one's.  us a step, products from 2e10 flop on by themselves / from
+// 1.5e11 / none:  o=10 v=80, 15 vectors (5e10 to 1.2e11) 6379 / 6082 / 6106, three-product 5547 / 5477 / 5460;
+// 4 vectors 1774 / 1694; O=20 V=100 (4e10, 6e10) 1992 / 1899; O=16 V=140 (9e10) 3317 / 3180
+//                 O=20 V=160 (2.5e11) 8398 / 8395 / 8283, three-product 7012 / 7011 / 7352
+//                 O=24 V=200 29042 / 29083 / 29447, three-product 27410 / 27495 / 26367
+constexpr double GROUP_ALONE_FLOP = 1.5e11;
 constexpr int64_t GROUP_MIN_K = 64;           // shortest K slice: eight stages against the prologue
 constexpr double GROUP_PART_BYTES = 6.4e7;    // partial sums of one product at most
 // Work of a block, in shares of what one round of resident blocks would give each: a block more than a

@@ -155,17 +155,11 @@ def test_batched_step_and_energy_match_single_calls(dev, singles):
         assert abs(energies[q].item() - e1) < 1e-13 * max(1.0, abs(e1))
 
 
-@pytest.mark.parametrize("nb", [24, 25])
-@pytest.mark.parametrize("singles,fold", [(True, True), (True, False), (False, True)])
-def test_batched_step_at_the_epilogue_rule(dev, nb, singles, fold):
-    """64 tiles of (a, b) a vector (two 32-wide ones a side, the second with one row): 24 vectors are the last whose
-    epilogue issues its reads ahead, 25 take the other form.  Against one step a vector, and updated in place
-    bit for bit; two orders of sums of up to o v^2 terms."""
+def _check_batch_against_single_steps(dev, o, v, nb, singles, fold, every, in_place=False):
     import ctypes
     from apyib_amd import _lib
     from apyib_amd.kernels import stream_of, workspace
     lib = _lib.load()
-    o, v = 4, 33
     g = torch.Generator(device=dev).manual_seed(9)
     cn = lambda *sh: torch.randn(*sh, dtype=torch.complex128, device=dev, generator=g)
     E4 = 0.1 * cn(o + v, o + v, o + v, o + v)
@@ -184,15 +178,33 @@ def test_batched_step_at_the_epilogue_rule(dev, nb, singles, fold):
         assert lib.apy_cisd_sp_step_batch(ctypes.byref(a), n, None, ctypes.c_void_p(ws.data_ptr()), nbytes,
                                           stream_of(dev)) == 0
 
-    R, Xn, R2, X2 = torch.zeros_like(X), torch.zeros_like(X), torch.zeros_like(X), X.clone()
+    R, Xn = torch.zeros_like(X), torch.zeros_like(X)
     step(X, Xn, R, B, en, re, nb)
-    step(X2, X2, R2, B, en, re, nb)
-    assert torch.equal(R, R2) and torch.equal(Xn, X2)
-    for q in range(0, nb, 4):
+    if in_place:
+        R2, X2 = torch.zeros_like(X), X.clone()
+        step(X2, X2, R2, B, en, re, nb)
+        assert torch.equal(R, R2) and torch.equal(Xn, X2)
+    for q in range(0, nb, every):
         xn, r = torch.zeros_like(rt), torch.zeros_like(rt)
         step(X[q].clone(), xn, r, B[q].clone(), en[q:q + 1].clone(), re[q:q + 1].clone(), 1)
         assert (R[q] - r).abs().max() < 1e-13 * r.abs().max()
         assert (Xn[q] - xn).abs().max() < 1e-13 * xn.abs().max()
+
+
+@pytest.mark.parametrize("nb", [24, 25])
+@pytest.mark.parametrize("singles,fold", [(True, True), (True, False), (False, True)])
+def test_batched_step_at_the_epilogue_rule(dev, nb, singles, fold):
+    """64 tiles of (a, b) a vector (two 32-wide ones a side, the second with one row): 24 vectors are the last whose
+    epilogue issues its reads ahead, 25 take the other form.  Against one step a vector, and updated in place
+    bit for bit; two orders of sums of up to o v^2 terms."""
+    _check_batch_against_single_steps(dev, 4, 33, nb, singles, fold, 4, in_place=True)
+
+
+@pytest.mark.parametrize("nb", [15, 20])
+def test_batched_step_at_the_size_of_products_by_themselves(dev, nb):
+    """o = 10, v = 80: every product of 15 vectors shares one launch, the ring product of 20 (1.6e11 flop) runs
+    by itself before the others.  Against one step a vector."""
+    _check_batch_against_single_steps(dev, 10, 80, nb, True, True, 7)
 
 
 @pytest.mark.parametrize("singles", [True, False])
