@@ -175,6 +175,153 @@ __device__ inline void tri_split(int64_t x, int64_t& hi, int64_t& lo) {
 // ket tables are one table ((ab|cd) = (ab|dc): 2 images, k >= l), ERI_NONE otherwise.
 enum EriSym { ERI_NONE = 0, ERI_KET = 1, ERI_ALL = 2 };
 
+struct EriTab {
+  const apy_gto* f[4];
+  int64_t n[4];
+};
+
+// One primitive quartet of (a b | c d): terms (ta, tb, tc, td), primitives (pa, pb, pc, pd), centres ca..cd,
+// qab = A - B, qcd = C - D.  The caller has checked the table entries and that the quartet's total angular
+// momentum is at most LQ.
+__device__ double eri_prim(const apy_gto& A, const apy_gto& B, const apy_gto& C, const apy_gto& D, int ta, int tb,
+                           int tc, int td, int pa, int pb, int pc, int pd, const double* ca, const double* cb,
+                           const double* cc, const double* cd, const double* qab, const double* qcd) {
+  const int* la = A.lmn[ta];
+  const int* lb = B.lmn[tb];
+  const int* lc = C.lmn[tc];
+  const int* ld = D.lmn[td];
+  int L1[3], L2[3], Lt[3];
+  for (int x = 0; x < 3; ++x) { L1[x] = la[x] + lb[x]; L2[x] = lc[x] + ld[x]; Lt[x] = L1[x] + L2[x]; }
+  const int L = Lt[0] + Lt[1] + Lt[2];
+  const int sz = Lt[2] + 1, sy = (Lt[1] + 1) * sz;  // R index (t, u, v) -> t sy + u sz + v
+  const double a = A.exps[pa], b = B.exps[pb], p = a + b;
+  const double c = C.exps[pc], d = D.exps[pd], q = c + d;
+  double Eab[3][NE], Ecd[3][NE], PQ[3];
+  for (int x = 0; x < 3; ++x) {
+    herm_E(la[x], lb[x], qab[x], a, b, Eab[x]);
+    herm_E(lc[x], ld[x], qcd[x], c, d, Ecd[x]);
+    PQ[x] = (a * ca[x] + b * cb[x]) / p - (c * cc[x] + d * cd[x]) / q;
+  }
+  const double alpha = p * q / (p + q);
+  double F[LQ + 1];
+  boys_fn(L, alpha * (PQ[0] * PQ[0] + PQ[1] * PQ[1] + PQ[2] * PQ[2]), F);
+  double Rb[2][NRB];
+  const double* R = Rb[herm_R(L, Lt, alpha, PQ, F, Rb)];
+  double val = 0.0;
+  for (int t = 0; t <= L1[0]; ++t)
+    for (int u = 0; u <= L1[1]; ++u)
+      for (int v = 0; v <= L1[2]; ++v) {
+        const double e1 = Eab[0][t] * Eab[1][u] * Eab[2][v];
+        double s2 = 0.0;
+        for (int tt = 0; tt <= L2[0]; ++tt)
+          for (int uu = 0; uu <= L2[1]; ++uu)
+            for (int vv = 0; vv <= L2[2]; ++vv) {
+              const double e2 = Ecd[0][tt] * Ecd[1][uu] * Ecd[2][vv];
+              const double sg = ((tt + uu + vv) & 1) ? -1.0 : 1.0;
+              s2 += sg * e2 * R[(t + tt) * sy + (u + uu) * sz + (v + vv)];
+            }
+        val += e1 * s2;
+      }
+  const double pref0 = 2.0 * M_PI * M_PI * sqrt(M_PI);
+  return A.coefs[ta][pa] * B.coefs[tb][pb] * C.coefs[tc][pc] * D.coefs[td][pd] * pref0 / (p * q * sqrt(p + q)) * val;
+}
+
+// Whether every term combination of the quartet stays within the total angular momentum LQ.
+__device__ bool quartet_ok(const apy_gto& A, const apy_gto& B, const apy_gto& C, const apy_gto& D) {
+  for (int ta = 0; ta < A.nterm; ++ta)
+    for (int tb = 0; tb < B.nterm; ++tb)
+      for (int tc = 0; tc < C.nterm; ++tc)
+        for (int td = 0; td < D.nterm; ++td)
+          if (lsum(A.lmn[ta]) + lsum(B.lmn[tb]) + lsum(C.lmn[tc]) + lsum(D.lmn[td]) > LQ) return false;
+  return true;
+}
+
+// The elements one by one, a wavefront each (wave-uniform control flow): the lanes split the element's
+// (term, primitive) quartets and a fixed-order butterfly sums them; lane 0 writes the value to every
+// image of the element under the launch's symmetry.  A table entry outside the limits (angular
+// momentum, primitive count, term count, atom index) gives NaN before any indexing.
+__device__ __forceinline__ void eri_elements(int64_t ngeom, int64_t natom, const double* __restrict__ centers,
+                                             const EriTab& T, int sym, double2* __restrict__ out) {
+  const int lane = threadIdx.x & 63;
+  const int64_t na = T.n[0], nb = T.n[1], nc = T.n[2], nd = T.n[3], full = na * nb * nc * nd;
+  const int64_t pc = nc * (nc + 1) / 2;
+  const int64_t per = sym == ERI_ALL ? pc * (pc + 1) / 2 : sym == ERI_KET ? na * nb * pc : full;
+  const int64_t total = ngeom * per;
+  const int64_t nwave = (int64_t)gridDim.x * (blockDim.x >> 6);
+  for (int64_t e = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6; e < total; e += nwave) {
+    const int64_t g = e / per, r = e % per;
+    int64_t i, j, k, l;
+    if (sym == ERI_ALL) {
+      int64_t bra, ket;
+      tri_split(r, bra, ket);
+      tri_split(bra, i, j);
+      tri_split(ket, k, l);
+    } else if (sym == ERI_KET) {
+      tri_split(r % pc, k, l);
+      j = (r / pc) % nb;
+      i = r / (pc * nb);
+    } else {
+      l = r % nd; k = (r / nd) % nc; j = (r / (nd * nc)) % nb; i = r / (nd * nc * nb);
+    }
+    double2* o = out + g * full;
+    // element (p, q, s, t) of the [na][nb][nc][nd] output
+    auto at = [&](int64_t p, int64_t q, int64_t s2, int64_t t) { return ((p * nb + q) * nc + s2) * nd + t; };
+    auto put = [&](double v) {
+      const double2 w = make_double2(v, 0.0);
+      o[at(i, j, k, l)] = w;
+      if (sym == ERI_NONE) return;
+      o[at(i, j, l, k)] = w;
+      if (sym == ERI_KET) return;
+      o[at(j, i, k, l)] = w;
+      o[at(j, i, l, k)] = w;
+      o[at(k, l, i, j)] = w;
+      o[at(l, k, i, j)] = w;
+      o[at(k, l, j, i)] = w;
+      o[at(l, k, j, i)] = w;
+    };
+    const apy_gto& A = T.f[0][i];
+    const apy_gto& B = T.f[1][j];
+    const apy_gto& C = T.f[2][k];
+    const apy_gto& D = T.f[3][l];
+    if (!gto_ok(A, natom) || !gto_ok(B, natom) || !gto_ok(C, natom) || !gto_ok(D, natom) ||
+        !quartet_ok(A, B, C, D)) {
+      if (lane == 0) put(kNaN);
+      continue;
+    }
+    const double* cen = centers + 3 * natom * g;
+    const double* ca = cen + 3 * A.atom;
+    const double* cb = cen + 3 * B.atom;
+    const double* cc = cen + 3 * C.atom;
+    const double* cd = cen + 3 * D.atom;
+    const double qab[3] = {ca[0] - cb[0], ca[1] - cb[1], ca[2] - cb[2]};
+    const double qcd[3] = {cc[0] - cd[0], cc[1] - cd[1], cc[2] - cd[2]};
+    // quartet w = ((((((ta nbt + tb) nct + tc) ndt + td) npa + pa) npb + pb) npc + pc) npd + pd
+    const int nt = A.nterm * B.nterm * C.nterm * D.nterm;
+    const int np = A.nprim * B.nprim * C.nprim * D.nprim;
+    double acc = 0.0;
+    for (int w = lane; w < nt * np; w += 64) {
+      int x = w;
+      const int pd = x % D.nprim; x /= D.nprim;
+      const int pc = x % C.nprim; x /= C.nprim;
+      const int pb = x % B.nprim; x /= B.nprim;
+      const int pa = x % A.nprim; x /= A.nprim;
+      const int td = x % D.nterm; x /= D.nterm;
+      const int tc = x % C.nterm; x /= C.nterm;
+      const int tb = x % B.nterm; x /= B.nterm;
+      const int ta = x;
+      acc += eri_prim(A, B, C, D, ta, tb, tc, td, pa, pb, pc, pd, ca, cb, cc, cd, qab, qcd);
+    }
+    for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+    if (lane == 0) put(acc);
+  }
+}
+
+__global__ __launch_bounds__(256) void eri_element_kernel(int64_t ngeom, int64_t natom,
+                                                          const double* __restrict__ centers, EriTab T, int sym,
+                                                          double2* __restrict__ out) {
+  eri_elements(ngeom, natom, centers, T, sym, out);
+}
+
 // Functions that sit next to each other in a table on one centre with the same exponents (an sp or a d
 // shell) form a group of up to EG.  A group quartet shares every primitive quartet's Boys functions and
 // Hermite Coulomb integrals, which is why the work is split by group quartets and not by elements: at
@@ -195,7 +342,7 @@ enum EriSym { ERI_NONE = 0, ERI_KET = 1, ERI_ALL = 2 };
 // loops of two slots by EU primitive pairs side by side (as loops over t, u and v with the products of E in
 // them, one sp quartet of three primitives took 165 us, now 50), and 168 registers and 52 KB of LDS keep three
 // workgroups on a CU.  H2O2/6-31G*: 5040 us with a wave an element and every expansion redone for each
-// quartet of functions, 158 us so.
+// quartet of functions, 140 us so.
 constexpr int EG = 6;                 // functions of a group
 constexpr int EPP = APY_GTO_MAXPRIM * APY_GTO_MAXPRIM;
 constexpr int EW = 1536;              // doubles: G, powers and R of a batch
@@ -229,11 +376,6 @@ struct SmallDiv {
 // an LDS value that every thread reads alike, in a scalar register
 __device__ inline int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
-struct EriTab {
-  const apy_gto* f[4];
-  int64_t n[4];
-};
-
 // A slot of an element: the places of E^x_t, E^y_u and E^z_v in a primitive pair's E block and the two
 // functions' coefficient rows (2 member + term); ca = 255 pads an element to an even count.
 struct EriSlot {
@@ -254,17 +396,38 @@ struct EriShared {
   uint8_t stuv[2][ES];                // tuv index of each slot of the slice
   uint8_t sum[ESUM];                  // tuv index of the sum of a bra and a ket (t, u, v)
   EriSlot rec[2][ES];
-  int size[4], nprim[4], L[4], first[4], ngrp[4];
+  int size[4], nprim[4], L[4], first[4], ngrp[4], nshort[4][2];
 };
 
-// Starts of the groups of a table into `start` (start[ngrp] = n); by one thread.
-__device__ int find_groups(int64_t n, const uint8_t* joins, uint16_t* start) {
-  int g = 0, len = 0;
-  for (int i = 0; i < (int)n; ++i) {
-    if (i == 0 || !joins[i] || len == EG) { start[g++] = (uint16_t)i; len = 0; }
-    ++len;
+// Starts of the groups of a table into `start` (start[ngrp] = n) and over the flags of its functions (bit 0: joins
+// the one before, bits 1-2: one term of L = 0 or 1) each group's class: L of such a function by itself, else ECLS;
+// how many of each class into nshort.  By one wave, 64 functions at a time (by one thread 2 us at 34 functions).
+constexpr int ECLS = 2;
+__device__ int find_groups(int n, uint8_t* flags, uint16_t* start, int* nshort, int lane) {
+  int g = 0, run = 0, ns = 0, np = 0;                  // run: where the functions that join each other began
+  for (int base = 0; base < n; base += 64) {
+    const int i = base + lane;
+    const int f = i < n ? flags[i] : 1, next = i + 1 < n ? flags[i + 1] : 0;
+    const unsigned long long cut = __ballot(i == 0 || !(f & 1)), upto = cut & ((2ull << lane) - 1ull);
+    const int r = upto ? base + 63 - __clzll((long long)upto) : run;
+    const bool first = i < n && (i - r) % EG == 0;
+    const unsigned long long firsts = __ballot(first);
+    const int cls = next & 1 ? ECLS : f & 2 ? 0 : f & 4 ? 1 : ECLS;
+    if (first) {
+      const int at = g + __popcll(firsts & ((1ull << lane) - 1ull));
+      start[at] = (uint16_t)i;
+      flags[at] = (uint8_t)cls;                        // at <= i: read by all lanes above
+    }
+    ns += __popcll(__ballot(first && cls == 0));
+    np += __popcll(__ballot(first && cls == 1));
+    g += __popcll(firsts);
+    run = __shfl(r, 63, 64);
   }
-  start[g] = (uint16_t)n;
+  if (lane == 0) {
+    start[g] = (uint16_t)n;
+    nshort[0] = ns;
+    nshort[1] = np;
+  }
   return g;
 }
 
@@ -320,10 +483,65 @@ __device__ double boys_one(int n, double T) {
   return F;
 }
 
+// (ab|cd) of four functions of one term, all s but at most one p (about its own centre, axis x):
+//   (ss|ss) = sum K_ab K_cd F_0,  bra p: K_ab K_cd ((P - A)_x F_0 - alpha / p (P - Q)_x F_1), ket p alike with the
+// other sign of P - Q; the lanes split the primitive quartets.  A chain of 12 hydrogens in a split-valence basis
+// (24 s functions, each a group by itself): 852 us as groups, 379 as elements of the general form, 235 so.
+__device__ double eri_short(const apy_gto& A, const apy_gto& B, const apy_gto& C, const apy_gto& D, const double* cen,
+                            int lane) {
+  int pf = -1, px = 0;                                 // the p function and its axis
+  double r[4][3];
+  auto centre = [&](const apy_gto& f, int y) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      r[y][k] = cen[3 * f.atom + k];
+      if (f.lmn[0][k]) { pf = y; px = k; }
+    }
+  };
+  centre(A, 0);
+  centre(B, 1);
+  centre(C, 2);
+  centre(D, 3);
+  double ab = 0.0, cd = 0.0, rx[4];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    ab += (r[0][k] - r[1][k]) * (r[0][k] - r[1][k]);
+    cd += (r[2][k] - r[3][k]) * (r[2][k] - r[3][k]);
+  }
+#pragma unroll
+  for (int y = 0; y < 4; ++y) rx[y] = px == 0 ? r[y][0] : px == 1 ? r[y][1] : r[y][2];
+  const double at = pf == 0 ? rx[0] : pf == 1 ? rx[1] : pf == 2 ? rx[2] : rx[3];
+  const SmallDiv dD(D.nprim), dC(C.nprim), dB(B.nprim);
+  const int np = A.nprim * B.nprim * C.nprim * D.nprim;
+  double acc = 0.0;
+  for (int w = lane; w < np; w += 64) {
+    const int w1 = dD.div(w), w2 = dC.div(w1), w3 = dB.div(w2);
+    const int pd = dD.mod(w), pc = dC.mod(w1), pb = dB.mod(w2), pa = w3;
+    const double a = A.exps[pa], b = B.exps[pb], c = C.exps[pc], d = D.exps[pd];
+    const double p = a + b, q = c + d, ip = 1.0 / p, iq = 1.0 / q, alpha = p * q / (p + q);
+    double r2 = 0.0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const double x = (a * r[0][k] + b * r[1][k]) * ip - (c * r[2][k] + d * r[3][k]) * iq;
+      r2 += x * x;
+    }
+    const double F0 = boys_one(0, alpha * r2);
+    double v = F0;
+    if (pf >= 0) {
+      const double P = (a * rx[0] + b * rx[1]) * ip, Q = (c * rx[2] + d * rx[3]) * iq, F1 = boys_one(1, alpha * r2);
+      v = pf < 2 ? (P - at) * F0 - alpha * ip * (P - Q) * F1 : (Q - at) * F0 + alpha * iq * (P - Q) * F1;
+    }
+    acc += A.coefs[0][pa] * B.coefs[0][pb] * C.coefs[0][pc] * D.coefs[0][pd] *
+           (2.0 * M_PI * M_PI * sqrt(M_PI) / (p * q * sqrt(p + q))) * exp(-a * b * ip * ab - c * d * iq * cd) * v;
+  }
+  for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+  return acc;
+}
+
 __global__ __launch_bounds__(256, 3) void eri_kernel(int64_t ngeom, int64_t natom, const double* __restrict__ centers,
-                                                  EriTab T, int sym, int grouped, double2* __restrict__ out) {
+                                                  EriTab T, int sym, double2* __restrict__ out) {
   __shared__ EriShared S;
-  extern __shared__ uint16_t starts[];               // group starts, then the join flags (grouped only)
+  extern __shared__ uint16_t starts[];               // group starts, then the functions' flags, the groups' classes
   const int tid = threadIdx.x;
   const int64_t n0 = T.n[0], n1 = T.n[1], n2 = T.n[2], n3 = T.n[3], full = n0 * n1 * n2 * n3;
 
@@ -331,23 +549,27 @@ __global__ __launch_bounds__(256, 3) void eri_kernel(int64_t ngeom, int64_t nato
   const int ntab = sym == ERI_ALL ? 1 : sym == ERI_KET ? 3 : 4;
   int64_t tot = 0, off[5];
   for (int x = 0; x < 4; ++x) { off[x] = tot; if (x < ntab) tot += T.n[x] + 1; }
-  if (grouped) {
-    uint8_t* joins = (uint8_t*)(starts + tot);
-    for (int x = 0; x < ntab; ++x)
-      for (int64_t i = tid; i < T.n[x]; i += 256) {
-        const apy_gto& f = T.f[x][i];
-        bool same = false;
-        if (i > 0 && gto_ok(f, natom)) {
+  uint8_t* flags = (uint8_t*)(starts + tot);
+  for (int x = 0; x < ntab; ++x)
+    for (int64_t i = tid; i < T.n[x]; i += 256) {
+      const apy_gto& f = T.f[x][i];
+      int v = 0;
+      if (gto_ok(f, natom)) {
+        bool same = i > 0;
+        if (same) {
           const apy_gto& e = T.f[x][i - 1];
           same = gto_ok(e, natom) && e.atom == f.atom && e.nprim == f.nprim;
           for (int k = 0; same && k < f.nprim; ++k) same = e.exps[k] == f.exps[k];
         }
-        joins[off[x] + i] = same;
+        const int L = lsum(f.lmn[0]);
+        v = (same ? 1 : 0) | (f.nterm == 1 && L < ECLS && f.nprim <= 4 ? 2 << L : 0);
       }
-    __syncthreads();
-    if (tid < ntab) S.ngrp[tid] = find_groups(T.n[tid], joins + off[tid], starts + off[tid]);
-  } else if (tid < 4) {
-    S.ngrp[tid] = (int)T.n[tid];
+      flags[off[x] + i] = (uint8_t)v;
+    }
+  __syncthreads();
+  if (const int x = tid >> 6; x < ntab) {
+    const int g = find_groups((int)T.n[x], flags + off[x], starts + off[x], S.nshort[x], tid & 63);
+    if ((tid & 63) == 0) S.ngrp[x] = g;
   }
   for (int r = tid; r < ENR; r += 256) {
     int s = 0, w = 0;
@@ -369,12 +591,21 @@ __global__ __launch_bounds__(256, 3) void eri_kernel(int64_t ngeom, int64_t nato
   const int tx[4] = {0, sym == ERI_ALL ? 0 : 1, sym == ERI_ALL ? 0 : 2, sym == ERI_ALL ? 0 : sym == ERI_KET ? 2 : 3};
   int64_t ng[4];
   for (int x = 0; x < 4; ++x) ng[x] = uniform(S.ngrp[tx[x]]);
+  // the short form (below) where it takes most quartets: the passes over all of them that it needs beside the
+  // workgroups' cost a molecule of mixed shells more than it saves there (13 geometries of H2O2/6-31G* 1.31 -> 1.36 ms)
+  double all = 1.0, ss = 1.0, sp = 0.0;
+  for (int x = 0; x < 4; ++x) {
+    const int* c = S.nshort[tx[x]];
+    all *= (double)ng[x];
+    sp = sp * (double)c[0] + ss * (double)c[1];
+    ss *= (double)c[0];
+  }
+  const bool shorts = uniform(ss + sp >= 0.5 * all);
   const int64_t pk = sym == ERI_NONE ? ng[2] * ng[3] : ng[2] * (ng[2] + 1) / 2;
   const int64_t per = sym == ERI_ALL ? pk * (pk + 1) / 2 : ng[0] * ng[1] * pk;
 
-  for (int64_t item = blockIdx.x; item < ngeom * per; item += gridDim.x) {
-    const int64_t g = item / per, r0 = item % per;
-    int64_t G[4];
+  // the groups of an item, and whether the short form takes it
+  auto decode = [&](int64_t r0, int64_t (&G)[4]) {
     if (sym == ERI_ALL) {
       int64_t bra, ket;
       tri_split(r0, bra, ket);
@@ -389,12 +620,38 @@ __global__ __launch_bounds__(256, 3) void eri_kernel(int64_t ngeom, int64_t nato
       G[1] = (r0 / pk) % ng[1];
       G[0] = r0 / (pk * ng[1]);
     }
+    int c = shorts ? 0 : 2;
+    for (int x = 0; shorts && x < 4; ++x) {
+      const int y = flags[off[tx[x]] + G[x]];
+      c += y < ECLS ? y : 2;
+    }
+    return c < 2;
+  };
+  // the value of a canonical element to every image under the launch's symmetry
+  auto put = [&](int64_t g, int64_t i, int64_t j, int64_t k, int64_t l, double v) {
+    const double2 y = make_double2(v, 0.0);
+    double2* o = out + g * full;
+    auto at = [&](int64_t p, int64_t q, int64_t s, int64_t t) { return ((p * n1 + q) * n2 + s) * n3 + t; };
+    o[at(i, j, k, l)] = y;
+    if (sym == ERI_NONE) return;
+    o[at(i, j, l, k)] = y;
+    if (sym == ERI_KET) return;
+    o[at(j, i, k, l)] = y;
+    o[at(j, i, l, k)] = y;
+    o[at(k, l, i, j)] = y;
+    o[at(l, k, i, j)] = y;
+    o[at(k, l, j, i)] = y;
+    o[at(l, k, j, i)] = y;
+  };
+  for (int64_t item = blockIdx.x; item < ngeom * per; item += gridDim.x) {
+    const int64_t g = item / per, r0 = item % per;
+    int64_t G[4];
+    if (uniform(decode(r0, G))) continue;
     // ---- the four groups into LDS
     __syncthreads();                                  // the previous item's elements are done with LDS
     if (tid < 4) {
       const int x = tid;
-      const int64_t b = grouped ? starts[off[tx[x]] + G[x]] : G[x];
-      const int64_t e = grouped ? starts[off[tx[x]] + G[x] + 1] : b + 1;
+      const int64_t b = starts[off[tx[x]] + G[x]], e = starts[off[tx[x]] + G[x] + 1];
       const apy_gto& f = T.f[x][b];
       const bool ok = gto_ok(f, natom);
       S.first[x] = (int)b;
@@ -706,7 +963,7 @@ __global__ __launch_bounds__(256, 3) void eri_kernel(int64_t ngeom, int64_t nato
         else bra(std::integral_constant<int, EU>{});
         __syncthreads();                              // H, E and the slots of this batch are read
       }
-      // ---- out: the value of a canonical element to every image under the launch's symmetry
+      // ---- out
 #pragma unroll
       for (int m = 0; m < EACC; ++m) {
         const int w = tid + 256 * m;
@@ -733,22 +990,22 @@ __global__ __launch_bounds__(256, 3) void eri_kernel(int64_t ngeom, int64_t nato
           }
           if (Lm[0] + Lm[1] + Lm[2] + Lm[3] > LQ) v = kNaN;
         }
-        const double2 y = make_double2(v, 0.0);
-        double2* o = out + g * full;
-        auto at = [&](int64_t p, int64_t q, int64_t s, int64_t t) { return ((p * n1 + q) * n2 + s) * n3 + t; };
-        o[at(i, j, k, l)] = y;
-        if (sym == ERI_NONE) continue;
-        o[at(i, j, l, k)] = y;
-        if (sym == ERI_KET) continue;
-        o[at(j, i, k, l)] = y;
-        o[at(j, i, l, k)] = y;
-        o[at(k, l, i, j)] = y;
-        o[at(l, k, i, j)] = y;
-        o[at(k, l, j, i)] = y;
-        o[at(l, k, j, i)] = y;
+        put(g, i, j, k, l, v);
       }
       }
     }
+  }
+  // ---- the short form, a wave an element: one s function each, or one of them p (the derivative of an s)
+  const int lane = tid & 63;
+  for (int64_t item = (int64_t)blockIdx.x * 4 + (tid >> 6); shorts && item < ngeom * per;
+       item += (int64_t)gridDim.x * 4) {
+    const int64_t g = item / per, r0 = item % per;
+    int64_t G[4];
+    if (!uniform(decode(r0, G))) continue;
+    int64_t f[4];
+    for (int x = 0; x < 4; ++x) f[x] = starts[off[tx[x]] + G[x]];
+    const double v = eri_short(T.f[0][f[0]], T.f[1][f[1]], T.f[2][f[2]], T.f[3][f[3]], centers + 3 * natom * g, lane);
+    if (lane == 0) put(g, f[0], f[1], f[2], f[3], v);
   }
 }
 
@@ -928,14 +1185,25 @@ int apy_eri_gto(int64_t ngeom, int64_t natom, const double* centers, const apy_g
   if (na > INT32_MAX || nb > INT32_MAX || nc > INT32_MAX || nd > INT32_MAX) return APY_E_ARG;
   if (const int rc = ensure_boys_table((hipStream_t)stream); rc != APY_OK) return rc;
   const EriTab T = {{fa, fb, fc, fd}, {na, nb, nc, nd}};
-  // tables whose group starts do not fit LDS are taken function by function
+  // Tables whose group starts do not fit LDS are taken element by element, and so are launches of fewer elements
+  // than the waves of two a SIMD: the longest one then sets the time, and a wave has its sums sooner
+  // than a workgroup its group.  us a call, elements / groups: 406 elements of H2O/STO-3G 102 / 108, their 1372
+  // derivatives 178 / 186; 3081 of H2O2/STO-3G 145 / 107.
   const int64_t tot = na + 1 + (sym == ERI_ALL ? 0 : nb + nc + 2 + (sym == ERI_KET ? 0 : nd + 1));
-  const int grouped = tot <= ETAB;
+  const double nk = (double)nc * (nc + 1) / 2;
+  const double elements = (double)ngeom * (sym == ERI_ALL   ? nk * (nk + 1) / 2
+                                           : sym == ERI_KET ? (double)na * nb * nk
+                                                            : (double)na * nb * nc * nd);
+  if (tot > ETAB || elements <= 2048.0) {
+    const unsigned grid = (unsigned)std::min((elements + 3.0) / 4.0, 65536.0);
+    eri_element_kernel<<<grid, 256, 0, (hipStream_t)stream>>>(ngeom, natom, centers, T, sym, (double2*)out);
+    APY_LAUNCH_CHECK();
+    return APY_OK;
+  }
   // a resident grid (three workgroups a CU): the groups are found once a workgroup
-  const double bound = (double)ngeom * na * nb * nc * nd;
-  const unsigned grid = (unsigned)std::min(bound, 3.0 * 256.0);
-  const size_t lds = grouped ? (size_t)tot * (sizeof(uint16_t) + 1) : 0;
-  eri_kernel<<<grid, 256, lds, (hipStream_t)stream>>>(ngeom, natom, centers, T, sym, grouped, (double2*)out);
+  const unsigned grid = (unsigned)std::min(elements, 3.0 * 256.0);
+  const size_t lds = (size_t)tot * (sizeof(uint16_t) + 1);
+  eri_kernel<<<grid, 256, lds, (hipStream_t)stream>>>(ngeom, natom, centers, T, sym, (double2*)out);
   APY_LAUNCH_CHECK();
   return APY_OK;
 }

@@ -284,3 +284,64 @@ def test_eri_function_groups(dev, case):
         for p in good[rng.integers(0, len(good), 120)]:
             want = gaussian.eri(*[fns[q] for q in p])
             assert abs(G[tuple(p)] - want) < 1e-12 * max(1.0, abs(want)), (case, p)
+
+
+def test_eri_short_form(dev):
+    """Tables of mostly single s functions take a wave an element in closed form, with one of the four a p function
+    (the derivative of an s) in any place too; an s of six primitives and a p shell in the same table take the
+    groups' way.  Against the host's integrals: sums of up to 81 terms of one sign, or their differences along one
+    axis, of magnitude at most 1e2 times the result."""
+    rng = np.random.default_rng(7)
+    cen = np.array([[0.1, -0.2, 0.3], [0.9, 0.4, -0.5], [-0.7, 1.1, 0.2]])
+    e3 = np.array([3.4, 0.62, 0.17])
+    spec = [(k % 3, (0, 0, 0), e3[:1 + k % 3] * (1.0 + 0.05 * k)) for k in range(13)]
+    spec += [(1, (0, 0, 0), np.array([23.0, 8.0, 3.1, 1.3, 0.6, 0.25]))]
+    spec += [(2, l, np.array([0.9, 0.35])) for l in ((1, 0, 0), (0, 1, 0), (0, 0, 1))]
+    fns = [gaussian.RawGaussian(cen[a], l, e, rng.uniform(0.5, 1.5, len(e))) for a, l, e in spec]
+    atoms, n = [a for a, _, _ in spec], len(spec)
+    tab = basis_table(fns, atoms, dev)
+    copy = tab.clone()
+    D = [derivative_table(fns, atoms, x, dev) for x in range(3)]
+    plain = lambda f: [f]
+    cases = [((tab, tab, tab, tab), None), ((copy, copy, tab, tab), None), ((copy, copy, copy, tab), None)]
+    for place in range(4):
+        tabs = [tab] * 4
+        tabs[place] = D[place % 3]
+        cases.append((tuple(tabs), (place, place % 3)))
+    for tabs, der in cases:
+        G = eri(*tabs, (n,) * 4, cen[None], dev).cpu().numpy()[0].real
+        terms = [plain] * 4
+        if der:
+            terms[der[0]] = lambda f: gaussian.center_derivative(f, der[1])
+        for p in np.concatenate([rng.integers(0, 13, (80, 4)), rng.integers(0, n, (80, 4))]):
+            want = sum(gaussian.eri(a, b, c, d) for a in terms[0](fns[p[0]]) for b in terms[1](fns[p[1]])
+                       for c in terms[2](fns[p[2]]) for d in terms[3](fns[p[3]]))
+            assert abs(G[tuple(p)] - want) < 1e-12 * max(1.0, abs(want)), (der, p)
+
+
+def test_eri_groups_of_a_long_table(dev):
+    """72 functions: groups that begin before and end after the 64th, one of them longer than a group may be, against
+    tables of six of them (few enough elements that each is a wave's own)."""
+    rng = np.random.default_rng(8)
+    cen = np.array([[0.1, -0.2, 0.3], [0.9, 0.4, -0.5], [-0.7, 1.1, 0.2]])
+    lmns = lambda L: [(x, y, L - x - y) for x in range(L, -1, -1) for y in range(L - x, -1, -1)]
+    spec = [(k % 3, (0, 0, 0), [0.2 + 0.04 * k, 2.0]) for k in range(57)]
+    spec += [(1, l, [1.1, 0.4]) for l in lmns(0) + lmns(1) + lmns(2)]          # 57..66: six and four
+    spec += [(0, (0, 0, 0), [0.3, 0.7]), (0, (0, 0, 0), [0.3, 0.7]), (2, (1, 0, 0), [0.5]), (2, (0, 0, 0), [0.5]),
+             (1, (0, 0, 0), [0.9])]
+    fns = [gaussian.RawGaussian(cen[a], l, np.asarray(e, dtype=float), rng.uniform(0.5, 1.5, len(e)))
+           for a, l, e in spec]
+    atoms, n = [a for a, _, _ in spec], len(spec)
+    assert n == 72
+    tab = basis_table(fns, atoms, dev)
+    copy = tab.clone()
+    picks = [(0, 56, 57, 62, 63, 64), (58, 63, 64, 65, 66, 67), (67, 68, 69, 70, 71, 3)]
+    picks += [tuple(rng.choice(n, 6, replace=False)) for _ in range(6)]
+    for tabs in ((tab, tab, tab, tab), (copy, copy, tab, tab)):
+        G = eri(*tabs, (n,) * 4, cen[None], dev)[0].real
+        for pick in picks:
+            sub = basis_table([fns[k] for k in pick], [atoms[k] for k in pick], dev)
+            want = eri(sub, sub, sub, sub, (6,) * 4, cen[None], dev)[0].real
+            ix = torch.tensor(pick, device=dev)
+            got = G[ix][:, ix][:, :, ix][:, :, :, ix]
+            assert (got - want).abs().max() < 1e-12 * max(1.0, want.abs().max().item()), pick
