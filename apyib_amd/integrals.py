@@ -210,8 +210,9 @@ def mixed_overlaps(pairs, device):
     function at its own centre (utils.py:371-376 for every pair): pairs with
     the same function shapes share one apy_oei_gto launch.  Returns a list of
     float64 device tensors [na, nb] in the order of `pairs`."""
-    # a finite-difference set pairs a few dozen function lists in hundreds of ways: each list (alive in `pairs`
-    # throughout) is read once
+    # a finite-difference set pairs a few dozen function lists in hundreds of ways: each list (held here, so that
+    # no other can take its identity) is read once
+    pairs = [(bra, ket) for bra, ket in pairs]
     seen = {}
     for pair in pairs:
         for fns in pair:

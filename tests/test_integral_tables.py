@@ -59,3 +59,23 @@ def test_two_terms_share_their_exponents():
     other = gaussian.RawGaussian(t[1].center, t[1].lmn, np.array(t[1].exps) * 2.0, t[1].coefs)
     with pytest.raises(ValueError):
         integrals._table([0], [(t[0], other)], "cpu")
+
+
+def test_mixed_overlaps_of_lists_made_on_access(monkeypatch):
+    """A sequence that makes its function lists anew each time it is read: every pair keeps its own centres."""
+    class Pairs:
+        def __len__(self):
+            return 40
+
+        def __getitem__(self, q):
+            if q >= len(self):
+                raise IndexError
+            return [_f(center=(float(q), 0.0, 0.0))], [_f(center=(0.0, float(q), 0.0)), _f(center=(0.0, 0.0, float(q)))]
+
+    def centres_only(fa, ca, fb, cb, which, device):
+        return torch.from_numpy(np.concatenate([ca.reshape(len(ca), -1), cb.reshape(len(cb), -1)], axis=1))[:, None]
+
+    monkeypatch.setattr(integrals, "one_electron", centres_only)
+    out = integrals.mixed_overlaps(Pairs(), "cpu")
+    for q, S in enumerate(out):
+        assert S.tolist() == [q, 0, 0, 0, q, 0, 0, 0, q]
