@@ -114,6 +114,8 @@ def eri_so(eri_mo_t):
 
 def so_fock(f_mo):
     """utils.py:283-313 for one matrix [m, m] or a batch [nb, m, m]."""
+    if f_mo.dim() not in (2, 3) or f_mo.shape[-1] != f_mo.shape[-2]:
+        raise ValueError(f"expected [m, m] or [nb, m, m], got {tuple(f_mo.shape)}")
     lib = _lib.load()
     m = f_mo.shape[-1]
     f_mo = f_mo.contiguous()
