@@ -147,17 +147,21 @@ __device__ inline void kind_index(int kind, int64_t t, int64_t O, int64_t V, int
   }
 }
 
-// A store that leaves the caches to the integrals that are still read: for whole runs of an output that
-// does not fit them (vvvo_p of m = 60 62 -> 55 us, the others 28 -> 25 us; packed rows, which end inside cache
-// lines, lose by it, 127 -> 149 us).
-__device__ inline void nt_store(double2* p, double2 v) {
+// A store that leaves the caches to the integrals that are still read (past): for whole runs where the blocks of a
+// call hold NT_ELEMENTS (64 MB) or more together (vvvo_p of m = 60, 158 MB, 62 -> 55 us; packed rows, which end
+// inside cache lines, lose by it, 127 -> 149 us).  Fewer are still in the caches when the next kernel reads them: us
+// to build the blocks and read each once, kept / past: m = 16, O = 10 178 / 247; m = 24, O = 12 144 / 166;
+// m = 30, O = 20 (70 MB) 156 / 165, the build alone 62 / 57; m = 50, O = 20 (370 MB) 403 / 379, 215 / 196.
+constexpr int64_t NT_ELEMENTS = 4 << 20;
+__device__ inline void put_block(double2* p, double2 v, int past) {
   typedef double v2d __attribute__((ext_vector_type(2)));
-  __builtin_nontemporal_store((v2d){v.x, v.y}, (v2d*)p);
+  if (past) __builtin_nontemporal_store((v2d){v.x, v.y}, (v2d*)p);
+  else *p = v;
 }
 
 template <class Src>
 __global__ __launch_bounds__(256) void build_block(Src src, int kind, int64_t O, int64_t V, double2* out,
-                                                   int64_t total, int accumulate, double scale) {
+                                                   int64_t total, int accumulate, double scale, int past) {
   for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total; t += (int64_t)gridDim.x * blockDim.x) {
     int64_t p, q, r, s;
     kind_index(kind, t, O, V, p, q, r, s);
@@ -166,7 +170,7 @@ __global__ __launch_bounds__(256) void build_block(Src src, int kind, int64_t O,
       double2 o = out[t];
       out[t] = make_double2(o.x + scale * v.x, o.y + scale * v.y);
     } else {
-      nt_store(out + t, v);
+      put_block(out + t, v, past);
     }
   }
 }
@@ -188,7 +192,7 @@ constexpr int BT = 32;   // spatial tile edge
 
 template <int KIND>
 __global__ __launch_bounds__(256) void build_pair_rows(const double2* __restrict__ E, int64_t m, int64_t O, int64_t V,
-                                                       int64_t nq, int64_t nts, double2* __restrict__ out) {
+                                                       int64_t nq, int64_t nts, int past, double2* __restrict__ out) {
   constexpr bool TRI = KIND == K_VVVV_P || KIND == K_VOVV;      // columns r < s, both virtual
   constexpr bool PAIR = KIND == K_VVVV_P || KIND == K_VVVO_P;   // rows a < b
   __shared__ double2 A[BT][BT + 1], B[BT][BT + 1];              // M[R][S] and M[S][R] of the tile
@@ -257,7 +261,7 @@ __global__ __launch_bounds__(256) void build_pair_rows(const double2* __restrict
       }
       const int64_t o = TRI ? prow(r - O, V) + s - r - 1 : KIND == K_VVVO_P ? s * V + r - O : s * V * OV + r - O;
       if (TRI) out[base + o] = v;
-      else nt_store(out + base + o, v);
+      else put_block(out + base + o, v, past);
     }
   }
 }
@@ -270,7 +274,8 @@ __global__ __launch_bounds__(256) void build_pair_rows(const double2* __restrict
 //   vvvo_p  m = 16, O = 4  3.6 / 7.4    m = 48, O = 4   15.6 / 22.2   m = 32, O = 20   9.8 / 9.4    m = 48, O = 20  36.5 / 20.7
 //   vovv_p  m = 16, O = 4  3.5 / 10.3   m = 36, O = 20  15.2 / 16.0   m = 40, O = 20  21.0 / 17.6   m = 48, O = 10  29.0 / 20.4
 template <int KIND>
-int launch_pair_rows(const double2* E, int64_t m, int64_t O, int64_t V, void* out, hipStream_t st, unsigned& done) {
+int launch_pair_rows(const double2* E, int64_t m, int64_t O, int64_t V, int past, void* out, hipStream_t st,
+                     unsigned& done) {
   const int64_t N = kind_size(KIND, O, V);
   if (!out || N <= 0) return APY_OK;
   constexpr bool TRI = KIND == K_VVVV_P || KIND == K_VOVV, PAIR = KIND == K_VVVV_P || KIND == K_VVVO_P;
@@ -279,7 +284,7 @@ int launch_pair_rows(const double2* E, int64_t m, int64_t O, int64_t V, void* ou
   const int64_t nq = PAIR ? nv : KIND == K_VOVV ? no : nv;
   const int64_t pairs = PAIR ? nv * (nv + 1) / 2 : nv * no, tiles = TRI ? ntv * (ntv + 1) / 2 : ntv * nto;
   if (pairs * tiles > 0x7fffffffLL || N < from + 1000 * pairs * tiles) return APY_OK;
-  build_pair_rows<KIND><<<(unsigned)(pairs * tiles), 256, 0, st>>>(E, m, O, V, nq, TRI ? ntv : nto, (double2*)out);
+  build_pair_rows<KIND><<<(unsigned)(pairs * tiles), 256, 0, st>>>(E, m, O, V, nq, TRI ? ntv : nto, past, (double2*)out);
   APY_LAUNCH_CHECK();
   done |= 1u << KIND;
   return APY_OK;
@@ -300,10 +305,18 @@ void* block_ptr(const apy_so_ints* I, int kind) {
   return nullptr;
 }
 
+int stored_past(const apy_so_ints* I) {
+  int64_t n = 0;
+  for (int kind = 0; kind < K_COUNT; ++kind)
+    if (block_ptr(I, kind)) n += std::max<int64_t>(kind_size(kind, I->O, I->V), 0);
+  return n >= NT_ELEMENTS;
+}
+
 template <class Src>
 int build_all(const Src& src, const apy_so_ints* I, int accumulate, double scale, hipStream_t st,
               unsigned skip = 0) {
   if (!I || I->O < 0 || I->V < 0) return APY_E_ARG;
+  const int past = stored_past(I);
   for (int kind = 0; kind < K_COUNT; ++kind) {
     if (skip >> kind & 1) continue;
     double2* out = (double2*)block_ptr(I, kind);
@@ -311,7 +324,7 @@ int build_all(const Src& src, const apy_so_ints* I, int accumulate, double scale
     int64_t total = kind_size(kind, I->O, I->V);
     if (total <= 0) continue;
     build_block<Src><<<apy_grid1d(total, 1 << 20), 256, 0, st>>>(src, kind, I->O, I->V, out, total, accumulate,
-                                                                 scale);
+                                                                 scale, past);
     APY_LAUNCH_CHECK();
   }
   return APY_OK;
@@ -1049,10 +1062,11 @@ int apy_so_ints_from_mo(int64_t m, const void* eri_mo, const apy_so_ints* ints, 
   hipStream_t st = (hipStream_t)stream;
   if (O < 0 || V < 0) return APY_E_ARG;
   unsigned done = 0;
-  int s = launch_pair_rows<K_VVVV_P>(E, m, O, V, ints->vvvv_p, st, done);
-  if (s == APY_OK) s = launch_pair_rows<K_VVVO_P>(E, m, O, V, ints->vvvo_p, st, done);
-  if (s == APY_OK) s = launch_pair_rows<K_VOVV>(E, m, O, V, ints->vovv_p, st, done);
-  if (s == APY_OK) s = launch_pair_rows<K_RING>(E, m, O, V, ints->ring, st, done);
+  const int past = stored_past(ints);
+  int s = launch_pair_rows<K_VVVV_P>(E, m, O, V, past, ints->vvvv_p, st, done);
+  if (s == APY_OK) s = launch_pair_rows<K_VVVO_P>(E, m, O, V, past, ints->vvvo_p, st, done);
+  if (s == APY_OK) s = launch_pair_rows<K_VOVV>(E, m, O, V, past, ints->vovv_p, st, done);
+  if (s == APY_OK) s = launch_pair_rows<K_RING>(E, m, O, V, past, ints->ring, st, done);
   if (s != APY_OK) return s;
   SrcMO src{E, m};
   return build_all(src, ints, 0, 0.0, st, done);
