@@ -176,9 +176,13 @@ constexpr size_t QLDS = 150 * 1024;   // of a CU's 160 KB
 
 size_t quarter_lds(int64_t K, int64_t M) { return (size_t)((K + 3) / 4 * 4) * ((M + 15) / 16 * 16) * sizeof(double2); }
 
-// The resident form: C within LDS and at most six 16-wide blocks of accumulators (96: 96 registers each
-// of re and im with the next k steps in flight).  Larger ones take the general GEMM, whose K is long enough.
-bool quarter_fits(int64_t nbf, int64_t nact) { return nact <= 96 && quarter_lds(nbf, nact) <= QLDS; }
+// The resident form: C within LDS and at most six 16-wide blocks of accumulators (96 orbitals: 96 registers of re and
+// im together, with the next k steps in flight).  Larger ones take the general GEMM, whose K is long enough, and so do 17
+// to 25 orbitals, whose second block is mostly padding: us, GEMMs / resident  16 of 16 21.0 / 19.1   18 of 18 23.2 /
+// 24.8   24 of 24 30.6 / 32.2   26 of 26 36.8 / 37.0   30 of 30 47.8 / 44.2   32 of 16 32.3 / 28.0.
+bool quarter_fits(int64_t nbf, int64_t nact) {
+  return nact <= 96 && quarter_lds(nbf, nact) <= QLDS && (nact <= 16 || nbf > 25);
+}
 
 template <int NB, bool ROWS>
 int quarter_nb(int K, int M, const double2* C, int64_t ldc, int conj, const double2* X, int64_t total, int64_t N,

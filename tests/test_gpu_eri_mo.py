@@ -1,6 +1,6 @@
-"""apy_eri_mo at the edges of its forms: the two fused quarter transforms up to 48 orbitals (16-wide blocks in
-rows and columns), the coefficients resident in LDS up to 96 active orbitals, and the general products beyond
-or where the coefficients outgrow LDS."""
+"""apy_eri_mo at the edges of its forms: quarter transforms with the coefficients resident in LDS (16-wide blocks of
+up to 96 active orbitals, 150 KB of LDS), and the general products where a second block would be mostly padding
+(17 to 25 orbitals), beyond 96 active orbitals and where the coefficients outgrow LDS."""
 import pytest
 import torch
 
@@ -10,7 +10,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("nbf,nact", [(1, 1), (2, 1), (7, 7), (16, 16), (17, 15), (32, 17), (33, 32), (34, 9), (48, 48),
-                                      (48, 33), (49, 48), (52, 17), (65, 64), (81, 80), (96, 96), (98, 97), (80, 3)])
+                                      (48, 33), (49, 48), (52, 17), (65, 64), (81, 80), (96, 96), (98, 97), (80, 3),
+                                      (25, 16), (25, 17), (25, 25), (26, 26), (100, 96), (101, 81)])
 def test_eri_mo_matches_torch(dev, nbf, nact):
     """Against the four quarter transforms in torch: sums of nbf terms of order one a quarter, 1e-13 of the
     largest element covers four roundings of each."""
