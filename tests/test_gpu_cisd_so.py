@@ -131,9 +131,10 @@ def test_small_blocks_stay_in_the_caches(dev):
 @pytest.mark.parametrize("singles,fov,fold,packed", [(True, False, True, False), (True, True, True, True),
                                                      (True, True, False, False), (False, False, True, False)])
 def test_grouped_products_match_one_after_another(dev, O, V, singles, fov, fold, packed):
-    """A step's products in one launch (the workspace the library asks for) against the same products one
-    launch after another (the smaller workspace the step still takes, found by bisection): two orders of
-    sums of up to O V^2 terms of order one."""
+    """A step's products in one launch against the same products one launch after another (the form that timing
+    events ask for; they time the first product, so both must have been recorded): two orders of sums of up to
+    O V^2 terms of order one.  The products share targets (R and the singles) and, at the larger sizes, have several
+    K slices each."""
     import ctypes
     from apyib_amd import _lib
     lib = _lib.load()
@@ -144,29 +145,30 @@ def test_grouped_products_match_one_after_another(dev, O, V, singles, fov, fold,
     t = torch.randn(ci.Lp if packed else ci.L, dtype=torch.complex128, device=dev, generator=g) * 0.1
     mode = _lib.APY_MODE_SIGMA if packed or fov else _lib.APY_MODE_RESIDUAL
 
-    def run(nbytes):
+    def run(events):
         out, tn = torch.full_like(t, 7.0), torch.full_like(t, 7.0)
+        ev = [e.cuda_event for e in events] if events else [None, None]
         a = _lib.CisdSoArgs(O, V, ci.fock.data_ptr(), ci.eps.data_ptr(), ctypes.pointer(ints.struct), ci.hoo.data_ptr(),
                             int(singles), int(mode), int(fov), ci.energy_dev.data_ptr(), 1.0, 0.0, t.data_ptr(),
-                            tn.data_ptr(), out.data_ptr(), None, None, None,
+                            tn.data_ptr(), out.data_ptr(), *ev, None,
                             ci.ring_f.data_ptr() if fold else None, int(packed), 0)
-        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-        rc = lib.apy_cisd_so_step(ctypes.byref(a), ctypes.c_void_p(ws.data_ptr()), nbytes,
-                                  ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        ws = torch.empty(ci.ws_bytes, dtype=torch.uint8, device=dev)
+        assert lib.apy_cisd_so_step(ctypes.byref(a), ctypes.c_void_p(ws.data_ptr()), ci.ws_bytes,
+                                    ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
         torch.cuda.synchronize()
-        return rc, out, tn
+        return out, tn
 
-    full = ci.ws_bytes
-    rc, out, tn = run(full)
-    assert rc == 0
-    lo, hi = 0, full                 # run(lo) refused, run(hi) accepted
-    while hi - lo > 256:
-        mid = (lo + hi) // 2
-        lo, hi = (lo, mid) if run(mid)[0] == 0 else (mid, hi)
-    rc, out1, tn1 = run(hi)
-    assert rc == 0
+    grouped = run(None)
+    events = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+    for e in events:
+        e.record()                                      # creates the handles
+    torch.cuda.synchronize()
+    alone = run(events)
+    assert 0.0 < events[0].elapsed_time(events[1]) < 1e3
+    if O * V > 500:                                     # other tiles and slices: not the same sums bit for bit
+        assert not torch.equal(grouped[0], alone[0])
     live = slice(None) if singles else slice(ci.OV, None)
-    for x, y in ((out, out1), (tn, tn1)):
+    for x, y in zip(grouped, alone):
         assert (x[live] - y[live]).abs().max() <= 1e-13 * max(1.0, y[live].abs().max().item())
 
 
