@@ -944,9 +944,10 @@ void sigma_gemms(int64_t O, int64_t V, int nb, int singles, const apy_so_ints* I
 }
 
 // exact = 1 sizes the GEMM region for the plans that would run now instead of
-// every plan the tuner may pick (the no-allocation entry point); grouped = 1 for
-// the products in one launch (a query's size: a step takes less, one product after
-// another then).
+// every plan the tuner may pick (the no-allocation entry point); grouped = 1: at
+// least the partial sums of the products in one launch (a query's size; they are
+// far below the largest single product's, and where a step's workspace does not
+// hold them the products run one after another).
 SigmaWS carve(int64_t O, int64_t V, int nb, int singles, int dense_in, const void* ring_f, void* base,
               int exact = 0, int grouped = 0) {
   const int64_t Po = npair(O), Pv = npair(V), OV = O * V;

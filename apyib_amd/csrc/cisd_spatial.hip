@@ -586,7 +586,7 @@ __global__ __launch_bounds__(256) void sp_epi_kernel(SpEpi e) {
 constexpr int EN_BLOCKS = 256;
 
 // E = sum g[0:ov] t1 + sum L t2 (no conjugation; g[0:ov] = 2 F_ov); instance blockIdx.y of vectors
-// `stride` apart, partial sums [instance][EN_BLOCKS]
+// `stride` apart, partial sums [instance][blocks of the launch, at most EN_BLOCKS]
 __global__ __launch_bounds__(256) void sp_energy_partial(int64_t ov, int singles, const double2* __restrict__ gv,
                                                          const double2* __restrict__ Lv, const double2* __restrict__ tv,
                                                          int64_t stride, int64_t s_g, int64_t s_l,

@@ -4,7 +4,8 @@
 // real/imaginary planes (re += ar*br - ai*bi, im += ar*bi + ai*br), i.e.
 // 8 real flops per complex MAC, executed with v_mfma_f64_16x16x4f64.
 //
-// Tiling: 256 threads = 4 waves arranged 2x2; each wave owns a WM x WN
+// Tiling: 256 threads = 4 waves (2x2; 1x4 in the 16 x 64 and 48 x 64 tiles of
+// grouped launches); each wave owns a WM x WN
 // complex output tile built from 16x16 MFMA blocks.  K is staged through a
 // double-buffered LDS tile, BK complex elements at a time, with two register
 // stages in front of it: while the MFMAs consume LDS buffer s, stage s+1
@@ -810,7 +811,7 @@ namespace {
 //                 O=20 V=160 (2.5e11) 8398 / 8395 / 8283, three-product 7012 / 7011 / 7352
 //                 O=24 V=200 29042 / 29083 / 29447, three-product 27410 / 27495 / 26367
 constexpr double GROUP_ALONE_FLOP = 1.5e11;
-constexpr int64_t GROUP_MIN_K = 64;           // shortest K slice: eight stages against the prologue
+constexpr int64_t GROUP_MIN_K = 64;           // shortest K slice: eight stages of 8 or four of 16 against the prologue
 constexpr double GROUP_PART_BYTES = 6.4e7;    // partial sums of one product at most
 // Work of a block, in shares of what one round of resident blocks would give each: a block more than a
 // round costs another whole one (o=18 v=50 by share 1: 271 us a step, 0.7: 263, 0.6: 241, 0.5: 250, 0.25:

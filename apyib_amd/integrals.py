@@ -14,6 +14,7 @@ mixed-geometry overlaps of utils.py:371-376 come from apy_oei_gto, again
 for many geometries (or bra/ket geometry pairs) per launch.
 """
 import ctypes
+import math
 
 import numpy as np
 import torch
@@ -33,21 +34,27 @@ def _table(atoms, functions, device):
     atoms[i] with the terms functions[i], one or two objects with lmn, exps and coefs that share exps.  Filled a
     field at a time: an entry at a time through ctypes took 12 us a function, 0.4 ms of host time for 34 functions
     whose integrals take 0.2 ms."""
-    n, mp = min(len(atoms), len(functions)), _lib.APY_GTO_MAXPRIM
-    functions = functions[:n]
+    n, mp = len(functions), _lib.APY_GTO_MAXPRIM
+    if len(atoms) != n:
+        n = min(len(atoms), n)
+        atoms, functions = atoms[:n], functions[:n]
     tab = np.zeros(n, dtype=_GTO)
     nterm = [len(t) for t in functions]
     first = [t[0] for t in functions]
     nprim = [len(f.exps) for f in first]
     if n and (max(nprim) > mp or min(nterm) < 1 or max(nterm) > 2):
         raise ValueError("function outside the integral kernel's limits")
-    tab["atom"] = np.array([int(a) for a in atoms[:n]], dtype=np.int64).astype(np.int32)
+    try:
+        tab["atom"] = atoms
+    except OverflowError:                              # an index outside the table's 32 bits: its low ones
+        tab["atom"] = np.array(atoms, dtype=np.int64).astype(np.int32)
     tab["nprim"], tab["nterm"] = nprim, nterm
     used = np.arange(mp) < np.asarray(nprim, dtype=np.int64).reshape(n, 1)
     if n:
-        tab["exps"][used] = np.concatenate([f.exps for f in first])
-        if np.isnan(tab["exps"]).any():
+        exps = np.concatenate([f.exps for f in first])
+        if math.isnan(np.dot(exps, exps)):
             raise ValueError("function outside the integral kernel's limits")
+        tab["exps"][used] = exps
     for k in range(2):
         rows = [i for i in range(n) if nterm[i] > k]
         if not rows:
@@ -58,12 +65,12 @@ def _table(atoms, functions, device):
                 k and f.exps is not first[i].exps and not np.array_equal(f.exps, first[i].exps)
                 for i, f in zip(rows, terms)):
             raise ValueError("function outside the integral kernel's limits")
-        if any(len(f.coefs) < len(f.exps) for f in terms):
-            raise IndexError("fewer coefficients than exponents")
         tab["lmn"][rows, k] = lmn
         at = np.nonzero(used[rows])
-        tab["coefs"][np.asarray(rows)[at[0]], k, at[1]] = np.concatenate(
-            [f.coefs[:len(f.exps)] for f in terms])
+        coefs = np.concatenate([f.coefs[:len(f.exps)] for f in terms])   # none longer than its exponents,
+        if len(coefs) != len(at[0]):                                     # so equal in all if equal in sum
+            raise IndexError("fewer coefficients than exponents")
+        tab["coefs"][np.asarray(rows)[at[0]], k, at[1]] = coefs
     return torch.from_numpy(tab.view(np.uint8)).to(device)
 
 

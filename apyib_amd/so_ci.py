@@ -195,7 +195,11 @@ class SOCI:
 
     def tune(self, t=None, reps=2):
         """Time the candidate GEMM plans of one step on this problem's
-        operands and cache the fastest per shape (process-wide)."""
+        operands and cache the fastest per shape (process-wide).  A step runs
+        its products of 1.5e11 flop and more (8 m n k) with the plan found;
+        the smaller ones share one launch whose tiles and K slices follow
+        from their sizes, and take the plan only where the products run one
+        after another (with timing events) or as products of their own."""
         t = self.new_vector() if t is None else t
         args = _lib.CisdSoArgs(
             self.O, self.V, self.fock.data_ptr(), self.eps.data_ptr(), ctypes.pointer(self.ints.struct),

@@ -121,7 +121,10 @@ class SpatialCI(SOCI):
     def tune(self, nb=1, reps=3):
         """Time the candidate GEMM plans of one step over nb vectors
         (apy_cisd_sp_tune; nb > 1 is the shared-integral batch of
-        ResponseSet) and cache the fastest per shape, process-wide."""
+        ResponseSet) and cache the fastest per shape, process-wide.  A step
+        runs its products of 1.5e11 flop and more (8 m n k) with the plan
+        found; the smaller ones share one launch whose tiles and K slices
+        follow from their sizes."""
         t = torch.zeros((nb, self.L), dtype=CDT, device=self.device)
         e = torch.zeros(nb, dtype=CDT, device=self.device)
         args = _lib.CisdSpArgs(self.O, self.V, self.fock.data_ptr(), self.eps.data_ptr(),

@@ -281,7 +281,9 @@ int apy_cisd_sp_energy_multi(int64_t o, int64_t v, int singles, int64_t nb, cons
 /* apy_cisd_sp_tune: time the candidate tile/split plans of every GEMM of one
  * spin-adapted step (nb instances; multi = 0 for apy_cisd_sp_step_batch's
  * shared-integral form, 1 for apy_cisd_sp_step_multi) and keep the fastest
- * in the process-wide plan cache that later steps of the same shapes use.
+ * in the process-wide plan cache, from which later steps take the plans of
+ * their products of 1.5e11 flop (8 m n k batch) and more; the others share one
+ * launch with tiles and K slices of its own.
  * The arguments are those of the step; workspace as for that step.  Writes
  * only the workspace.  No counterpart in the reference (its einsums have no
  * launch plans). */
@@ -360,7 +362,10 @@ int apy_cisd_so_ring_fock(int64_t O, int64_t V, const void* fock, const void* ri
 size_t apy_cisd_so_workspace(int64_t O, int64_t V, int singles);
 int apy_cisd_so_step(const apy_cisd_so_args* a, void* workspace, size_t ws_bytes, void* stream);
 /* Autotune every GEMM of a step for this (O, V) on the operands in `a`
- * (apy_zgemm_tune; only workspace is written).  Synchronises the stream. */
+ * (apy_zgemm_tune; only workspace is written).  Synchronises the stream.  A step
+ * takes the plans of its products of 1.5e11 flop (8 m n k batch) and more, and of
+ * all of them where they run one after another (timing events); the others share
+ * one launch with tiles and K slices of its own. */
 int apy_cisd_so_tune(const apy_cisd_so_args* a, void* workspace, size_t ws_bytes, int reps, void* stream);
 
 /* Sigma products (SIGMA mode) of nb instances sharing `ints` and (O, V),
